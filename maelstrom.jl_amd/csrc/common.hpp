@@ -260,13 +260,12 @@ constexpr double FIX_INV = 1.0 / 4294967296.0;
 __device__ inline unsigned long long tofix(float c) {
     return (unsigned long long)(long long)__double2ll_rn((double)c * FIX_SCALE);
 }
-// tofix for |c| < 2^19, in fewer instructions: c 2^32 is exact in FP64, and adding
-// 1.5 * 2^52 rounds it to an integer (to nearest even, as tofix does) whose two's
-// complement is the sum's low bits.
+// tofix for |c| < 2^19, in three instructions: adding 1.5 * 2^20 in FP64 rounds c to a
+// multiple of 2^-32 (to nearest even, as tofix does), whose two's complement is the sum's
+// low bits; the constant's bits come off the high word alone.
 __device__ inline unsigned long long tofix_near(float c) {
-    constexpr double MAGIC = 6755399441055744.0;   // 1.5 * 2^52
-    const double x = (double)c * FIX_SCALE + MAGIC;
-    return (unsigned long long)(__double_as_longlong(x) - __double_as_longlong(MAGIC));
+    const double x = (double)c + 1572864.0;
+    return (unsigned long long)(unsigned)__double2loint(x) | (unsigned long long)(unsigned)(__double2hiint(x) - 0x41380000) << 32;
 }
 __device__ inline float fromfix(unsigned long long v) { return (float)((double)(long long)v * FIX_INV); }
 

@@ -78,11 +78,51 @@ template <int N> __device__ inline int32_t faceat(const STopo& t, int a, int I, 
     return (s - 1) * per + ffn(N, a, a == 0 ? N : (Im & m), a == 1 ? N : (Jm & m), a == 2 ? N : (Km & m));
 }
 __device__ inline int32_t finefaceat(const STopo& t, int a, int I, int J, int K) { return faceat<16>(t, a, I, J, K); }
+// The slots of the blocks under a box of cells or face nodes, and of those one layer below
+// (whose top faces a node may be), for a table in LDS: fineat and finefaceat without reads
+// of the slot table.
+struct BlockTab {
+    static constexpr int CAP = 64;
+    int x, y, z, nx, ny, nz;
+    bool use;
+    __device__ BlockTab(bool any, const int lo[3], const int hi[3]) {
+        x = (lo[0] - 1) >> 4; y = (lo[1] - 1) >> 4; z = (lo[2] - 1) >> 4;
+        nx = (hi[0] >> 4) - x + 1; ny = (hi[1] >> 4) - y + 1; nz = (hi[2] >> 4) - z + 1;
+        use = any && nx <= CAP && ny <= CAP && nz <= CAP && nx * ny * nz <= CAP;
+    }
+    __device__ void stage(const STopo& t, int32_t* tab) const {
+        const int k = (int)threadIdx.x;
+        if (use && k < nx * ny * nz) {
+            const int bi = x + k % nx, bj = y + (k / nx) % ny, bk = z + k / (nx * ny);
+            tab[k] = inblocks(t.g, bi, bj, bk) ? t.slot[blockid(t.g, bi, bj, bk)] : 0;
+        }
+    }
+    __device__ int32_t cell(const int32_t* tab, int I, int J, int K) const {
+        const int32_t s = tab[(I >> 4) - x + nx * ((J >> 4) - y + ny * ((K >> 4) - z))];
+        return s == 0 ? -1 : (s - 1) * SBCELLS + (I & 15) + 16 * ((J & 15) + 16 * (K & 15));
+    }
+    __device__ int32_t face(const int32_t* tab, int a, int I, int J, int K) const {
+        const int e = (I >> 4) - x + nx * ((J >> 4) - y + ny * ((K >> 4) - z));
+        const int32_t s1 = tab[e];
+        if (s1 != 0) return (s1 - 1) * SBFACES + ffn(16, a, I & 15, J & 15, K & 15);
+        if (((a == 0 ? I : (a == 1 ? J : K)) & 15) != 0) return -1;
+        const int32_t s2 = tab[e - (a == 0 ? 1 : (a == 1 ? nx : nx * ny))];
+        return s2 == 0 ? -1 : (s2 - 1) * SBFACES + ffn(16, a, a == 0 ? 16 : (I & 15), a == 1 ? 16 : (J & 15), a == 2 ? 16 : (K & 15));
+    }
+};
 // flip.jl:513-537 over the topology: the deposit's nodes are fine faces (the upper block's
 // copy on a plane between blocks), as the tiled fixed-point reduction indexes them.
 struct SparseNodes {
     STopo t;
+    static constexpr bool HOLES = true;
     __device__ int32_t index(int a, int I, int J, int K) const { return finefaceat(t, a, I, J, K); }
+    static constexpr int TAB = BlockTab::CAP;
+    using Near = BlockTab;
+    __device__ Near near(bool any, const int lo[3], const int hi[3]) const { return BlockTab(any, lo, hi); }
+    __device__ void stage(const Near& b, int32_t* tab) const { b.stage(t, tab); }
+    __device__ int32_t at(const Near& b, const int32_t* tab, int a, int I, int J, int K) const {
+        return b.use ? b.face(tab, a, I, J, K) : index(a, I, J, K);
+    }
 };
 // Whether coarse cell (I, J, K) lies in a fine block (sflip.jl:127-128).
 __device__ inline bool covered(const STopo& t, int I, int J, int K) {

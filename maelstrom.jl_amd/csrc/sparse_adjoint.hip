@@ -219,7 +219,7 @@ void SparseBasin::g2p_adjoint(float dt) {
                      reached.p, 4.0f / (g.dx * g.dx)};
     P2GArgs A{{g.lo[0], g.lo[1], g.lo[2]}, g.dx, {adjacc[0].p, adjacc[1].p, adjacc[2].p}, {nullptr, nullptr, nullptr},
               (float)scale};
-    hipLaunchKernelGGL((k_p2g_tiled<SparseNodes, G2PAdjSource>), dim3(cdiv(n, P2G_THREADS)), dim3(P2G_THREADS), 0, s, view(cur),
+    hipLaunchKernelGGL((k_p2g_tiled<SparseNodes, G2PAdjSource>), p2g_grid(n), dim3(P2G_THREADS), 0, s, view(cur),
                        n, SparseNodes{t}, src, A);
     for (int a = 0; a < 3; ++a)
         if (F) hipLaunchKernelGGL(k_adj_fromfix, dim3(cdiv(F, 256)), dim3(256), 0, s, ub[a].fine.p, adjacc[a].p, F, 1.0 / scale);

@@ -192,6 +192,13 @@ int64_t SparseBasin::resample(bool seeding, uint32_t seed) {
 struct FineCellMap {
     STopo t;
     __device__ int32_t index(int I, int J, int K) const { return fineat(t, I, J, K); }
+    static constexpr int TAB = BlockTab::CAP;
+    using Near = BlockTab;
+    __device__ Near near(bool any, const int lo[3], const int hi[3]) const { return BlockTab(any, lo, hi); }
+    __device__ void stage(const Near& b, int32_t* tab) const { b.stage(t, tab); }
+    __device__ int32_t at(const Near& b, const int32_t* tab, int I, int J, int K) const {
+        return b.use ? b.cell(tab, I, J, K) : index(I, J, K);
+    }
 };
 
 // sflip.jl:620-640 syncplanes_kernel!, on the fixed-point accumulators.
@@ -258,7 +265,7 @@ void SparseBasin::p2g(float dt) {
         PView ps = view(cur);
         kt.begin(K_P2G, s);
         P2GArgs A{{g.lo[0], g.lo[1], g.lo[2]}, g.dx, {mom[0].p, mom[1].p, mom[2].p}, {wt[0].p, wt[1].p, wt[2].p}, 1.0f};
-        hipLaunchKernelGGL((k_p2g_tiled<SparseNodes, P2GSource>), dim3(cdiv(n, P2G_THREADS)), dim3(P2G_THREADS), 0, s, ps, n,
+        hipLaunchKernelGGL((k_p2g_tiled<SparseNodes, P2GSource>), p2g_grid(n), dim3(P2G_THREADS), 0, s, ps, n,
                            SparseNodes{t}, P2GSource{ps, dt}, A);
         kt.end(K_P2G, s);
         for (int a = 0; a < 3; ++a) {
@@ -290,189 +297,13 @@ void SparseBasin::p2g(float dt) {
 
 // ─── grid to particles (sflip.jl:2141-2144; flip.jl:1226-1244 over the topology) ──
 
-// One component's gather at a particle: the flag sum (finegather_value) and the APIC
-// value and affine row (finegather, sflip.jl:193-215) in one pass over the 27 nodes, in
-// the reference's order; `fetch(I, J, K, present, u, flag)` reads a node.
-// With ZERO the fetch returns 0 for the value and a negative flag where no face is, and a
-// missing node adds zero products instead of being skipped: the sums start at +0 and are
-// never -0, so adding a zero leaves them bit for bit as skipping does, without a branch.
-template <bool ZERO = false, class Fetch>
-__device__ inline void gather_component(const SGrid& g, int a, float px, float py, float pz, Fetch fetch, float& flag,
-                                        float& vel, float& a0, float& a1, float& a2) {
-    float q0 = ispace(px, g.lo[0], g.dx, a == 0 ? 0.0f : 0.5f);
-    float q1 = ispace(py, g.lo[1], g.dx, a == 1 ? 0.0f : 0.5f);
-    float q2 = ispace(pz, g.lo[2], g.dx, a == 2 ? 0.0f : 0.5f);
-    BSpline bx = bspline(q0), by = bspline(q1), bz = bspline(q2);
-    flag = 0.0f; vel = 0.0f; a0 = 0.0f; a1 = 0.0f; a2 = 0.0f;
-#pragma unroll
-    for (int mz = 0; mz < 3; ++mz) {
-        float wz = pick(bz, mz), dz = (float)(bz.b + mz) - q2;
-#pragma unroll
-        for (int my = 0; my < 3; ++my) {
-            float wy = pick(by, my), dy = (float)(by.b + my) - q1;
-#pragma unroll
-            for (int mx = 0; mx < 3; ++mx) {
-                bool pres;
-                float uv, fv;
-                fetch(bx.b + mx, by.b + my, bz.b + mz, pres, uv, fv);
-                if (ZERO || pres) {
-                    float wgt = pick(bx, mx) * wy * wz;
-                    if (ZERO) wgt = pres ? wgt : 0.0f;
-                    flag += wgt * fv;
-                    float tt = wgt * uv;
-                    vel += tt;
-                    a0 += (tt * ((float)(bx.b + mx) - q0)) * g.dx;
-                    a1 += (tt * dy) * g.dx;
-                    a2 += (tt * dz) * g.dx;
-                }
-            }
-        }
-    }
-    float c = __fdiv_rn(4.0f, g.dx * g.dx);
-    a0 *= c; a1 *= c; a2 *= c;
-}
-
-// flip.jl:1226-1244 g2p_kernel! over the topology, tiled: a workgroup's 256 particles
-// (cell-sorted, so close together) gather each component from a box of faces staged in
-// LDS (the value, and the flag or -1 where no fine face is there), loaded once per box
-// node instead of once per particle and node; a workgroup spread over more nodes than the
-// box holds reads the faces directly. Both paths sum the same terms in the same order. The
-// box's faces are found through a table of the slots of the blocks under it (and one
-// layer below along the component's axis, for a lower block's top faces).
-constexpr int G2P_BOX = 2048, G2P_TAB = 64;   // 16 KB: a band sheet through a block spans up to ~2000 nodes
-__global__ __launch_bounds__(256) void k_sparse_g2p(PView ps, int64_t n, STopo t, const float* __restrict__ u,
-                                                    const float* __restrict__ v, const float* __restrict__ w,
-                                                    const uint8_t* __restrict__ fu, const uint8_t* __restrict__ fv,
-                                                    const uint8_t* __restrict__ fw, float dt, float gravity) {
-    __shared__ float2 sbox[G2P_BOX];      // value, flag (-1: no face)
-    __shared__ int32_t stab[G2P_TAB];
-    __shared__ int red[6 * 4];
-    const SGrid& g = t.g;
-    int64_t p = (int64_t)xcd_tile(blockIdx.x, gridDim.x) * 256 + threadIdx.x;   // neighbouring tiles on one XCD
-    bool live = p < n;
-    float xp = 0, yp = 0, zp = 0;
-    if (live) { xp = ps.f[0][p]; yp = ps.f[1][p]; zp = ps.f[2][p]; }
-    const float* U[3] = {u, v, w};
-    const uint8_t* F[3] = {fu, fv, fw};
-    float fl[3], val[3], c0[3], c1[3], c2[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        float q0 = ispace(xp, g.lo[0], g.dx, a == 0 ? 0.0f : 0.5f);
-        float q1 = ispace(yp, g.lo[1], g.dx, a == 1 ? 0.0f : 0.5f);
-        float q2 = ispace(zp, g.lo[2], g.dx, a == 2 ? 0.0f : 0.5f);
-        BSpline bx = bspline(q0), by = bspline(q1), bz = bspline(q2);
-        bool ok = live && bx.b > -(1 << 24) && bx.b < (1 << 24) && by.b > -(1 << 24) && by.b < (1 << 24) &&
-                  bz.b > -(1 << 24) && bz.b < (1 << 24) && isfinite(q0) && isfinite(q1) && isfinite(q2);
-        const int BIG = 1 << 30;
-        int x0, y0, z0, x1, y1, z1;
-        wg_bounds(ok, bx.b, by.b, bz.b, red, x0, y0, z0, x1, y1, z1);
-        int ex = x1 - x0 + 3, ey = y1 - y0 + 3, ez = z1 - z0 + 3;
-        bool boxed = x0 != BIG && ex <= G2P_BOX && ey <= G2P_BOX && ez <= G2P_BOX && ex * ey * ez <= G2P_BOX;
-        const float* Ua = U[a];
-        const uint8_t* Fa = F[a];
-        if (boxed) {
-            const int tx = (x0 >> 4) - (a == 0), ty = (y0 >> 4) - (a == 1), tz = (z0 >> 4) - (a == 2);
-            const int nx = ((x0 + ex - 1) >> 4) - tx + 1, ny = ((y0 + ey - 1) >> 4) - ty + 1, nz = ((z0 + ez - 1) >> 4) - tz + 1;
-            const bool tab = nx * ny * nz <= G2P_TAB;
-            if (tab && (int)threadIdx.x < nx * ny * nz) {
-                int bi = tx + (int)threadIdx.x % nx, bj = ty + ((int)threadIdx.x / nx) % ny, bk = tz + (int)threadIdx.x / (nx * ny);
-                stab[threadIdx.x] = inblocks(g, bi, bj, bk) ? t.slot[blockid(g, bi, bj, bk)] : 0;
-            }
-            __syncthreads();
-            int V = ex * ey * ez;
-            for (int k = threadIdx.x; k < V; k += 256) {
-                const int I = x0 + k % ex, J = y0 + (k / ex) % ey, K = z0 + k / (ex * ey);
-                int32_t idx;
-                if (tab) {   // finefaceat through the table
-                    const int di = (I >> 4) - tx, dj = (J >> 4) - ty, dk = (K >> 4) - tz;
-                    const int32_t s1 = stab[di + nx * (dj + ny * dk)];
-                    if (s1 != 0) {
-                        idx = (s1 - 1) * SBFACES + ffn(16, a, I & 15, J & 15, K & 15);
-                    } else {
-                        const int GA = a == 0 ? I : (a == 1 ? J : K);
-                        const int32_t s2 =
-                            (GA & 15) == 0 ? stab[(di - (a == 0)) + nx * ((dj - (a == 1)) + ny * (dk - (a == 2)))] : 0;
-                        idx = s2 != 0 ? (s2 - 1) * SBFACES + ffn(16, a, a == 0 ? 16 : (I & 15), a == 1 ? 16 : (J & 15),
-                                                                 a == 2 ? 16 : (K & 15))
-                                      : -1;
-                    }
-                } else {
-                    idx = finefaceat(t, a, I, J, K);
-                }
-                sbox[k] = idx >= 0 ? make_float2(Ua[idx], (float)Fa[idx]) : make_float2(0.0f, -1.0f);
-            }
-            __syncthreads();
-        }
-        if (live) {
-            if (boxed && ok) {
-                // gather_component<true> over the box, the factors shared along rows hoisted:
-                // the same operations on the same values in the same order, so the same bits
-                const float wx[3] = {bx.w0, bx.w1, bx.w2}, wy[3] = {by.w0, by.w1, by.w2}, wz[3] = {bz.w0, bz.w1, bz.w2};
-                float d0[3], d1[3], d2[3];
-#pragma unroll
-                for (int m = 0; m < 3; ++m) {
-                    d0[m] = (float)(bx.b + m) - q0;
-                    d1[m] = (float)(by.b + m) - q1;
-                    d2[m] = (float)(bz.b + m) - q2;
-                }
-                const float2* bp = sbox + ((bx.b - x0) + ex * ((by.b - y0) + ey * (bz.b - z0)));
-                float f_ = 0.0f, v_ = 0.0f, s0 = 0.0f, s1 = 0.0f, s2 = 0.0f;
-#pragma unroll
-                for (int mz = 0; mz < 3; ++mz)
-#pragma unroll
-                    for (int my = 0; my < 3; ++my) {
-                        const float2* row = bp + ex * (my + ey * mz);
-#pragma unroll
-                        for (int mx = 0; mx < 3; ++mx) {
-                            const float2 e = row[mx];
-                            float wgt = (wx[mx] * wy[my]) * wz[mz];
-                            wgt = e.y >= 0.0f ? wgt : 0.0f;
-                            f_ += wgt * e.y;
-                            const float tt = wgt * e.x;
-                            v_ += tt;
-                            s0 += (tt * d0[mx]) * g.dx;
-                            s1 += (tt * d1[my]) * g.dx;
-                            s2 += (tt * d2[mz]) * g.dx;
-                        }
-                    }
-                const float c = __fdiv_rn(4.0f, g.dx * g.dx);
-                fl[a] = f_; val[a] = v_; c0[a] = s0 * c; c1[a] = s1 * c; c2[a] = s2 * c;
-            } else {
-                auto fetch = [&](int I, int J, int K, bool& pres, float& uv, float& fv_) {
-                    int32_t idx = finefaceat(t, a, I, J, K);
-                    pres = idx >= 0;
-                    uv = pres ? Ua[idx] : 0.0f;
-                    fv_ = pres ? (float)Fa[idx] : 0.0f;
-                };
-                gather_component(g, a, xp, yp, zp, fetch, fl[a], val[a], c0[a], c1[a], c2[a]);
-            }
-        }
-        if (boxed) __syncthreads();   // the box is reused by the next component
-    }
-    if (!live) return;
-    bool k1 = fl[0] > 0.999f, k2 = fl[1] > 0.999f, k3 = fl[2] > 0.999f;
-    float rec[12];   // stored unconditionally (see k_dense_spawn)
-    if (k1 && k2 && k3) {
-        rec[0] = val[0]; rec[3] = c0[0]; rec[4] = c1[0]; rec[5] = c2[0];
-        rec[1] = val[1]; rec[6] = c0[1]; rec[7] = c1[1]; rec[8] = c2[1];
-        rec[2] = val[2]; rec[9] = c0[2]; rec[10] = c1[2]; rec[11] = c2[2];
-    } else {
-        rec[0] = ps.f[3][p];
-        rec[1] = ps.f[4][p];
-        rec[2] = ps.f[5][p] - gravity * dt;
-#pragma unroll
-        for (int f = 3; f < 12; ++f) rec[f] = 0.0f;
-    }
-#pragma unroll
-    for (int f = 0; f < 12; ++f) ps.f[3 + f][p] = rec[f];
-}
-
 void SparseBasin::g2p(float dt, float grav) {
     if (n == 0) return;
     kt.begin(K_G2P, st.s);
     const SField<float>* fv = reflect_flow ? ur : u;   // sflip.jl:2312: the reflected velocity in a first half-step
-    hipLaunchKernelGGL(k_sparse_g2p, dim3(cdiv(n, 256)), dim3(256), 0, st.s, view(cur), n, topo(), fv[0].fine.p, fv[1].fine.p,
-                       fv[2].fine.p, fl[0].fine.p, fl[1].fine.p, fl[2].fine.p, dt, grav);
+    const G2PFaces F{{fv[0].fine.p, fv[1].fine.p, fv[2].fine.p}, {fl[0].fine.p, fl[1].fine.p, fl[2].fine.p}};
+    hipLaunchKernelGGL(k_g2p_tiled<SparseNodes>, dim3(cdiv(n, P2G_THREADS)), dim3(P2G_THREADS), 0, st.s, view(cur), n,
+                       SparseNodes{topo()}, g.lo[0], g.lo[1], g.lo[2], g.dx, F, dt, grav);
     kt.end(K_G2P, st.s);
     MAEL_LAUNCH_CHECK();
 }

@@ -22,6 +22,11 @@ struct DenseNodes {
         if (I < 0 || I >= n1 || J < 0 || J >= n2 || K < 0 || K >= n3) return -1;
         return (int64_t)I + (int64_t)n1 * ((int64_t)J + (int64_t)n2 * K);
     }
+    static constexpr int TAB = 1;   // no table
+    struct Near {};
+    __device__ Near near(bool, const int*, const int*) const { return {}; }
+    __device__ void stage(const Near&, int32_t*) const {}
+    __device__ int64_t at(const Near&, const int32_t*, int a, int I, int J, int K) const { return index(a, I, J, K); }
 };
 
 struct DenseCells {
@@ -30,6 +35,11 @@ struct DenseCells {
         if (I < 0 || I >= n[0] || J < 0 || J >= n[1] || K < 0 || K >= n[2]) return -1;
         return (int64_t)I + (int64_t)n[0] * ((int64_t)J + (int64_t)n[1] * K);
     }
+    static constexpr int TAB = 1;   // no table
+    struct Near {};
+    __device__ Near near(bool, const int*, const int*) const { return {}; }
+    __device__ void stage(const Near&, int32_t*) const {}
+    __device__ int64_t at(const Near&, const int32_t*, int I, int J, int K) const { return index(I, J, K); }
 };
 
 // flip.jl:562-565 union_kernel!.
@@ -82,12 +92,11 @@ void DenseBasin::p2g(float dt) {
         kt.begin(K_P2G, s);
         DenseNodes map{{g.n[0], g.n[1], g.n[2]}};
         P2GArgs A{{g.lo[0], g.lo[1], g.lo[2]}, g.dx, {mom[0].p, mom[1].p, mom[2].p}, {wt[0].p, wt[1].p, wt[2].p}, 1.0f};
-        hipLaunchKernelGGL((k_p2g_tiled<DenseNodes, P2GSource, P2G_BOX_DENSE>), dim3(cdiv(n, P2G_THREADS)), dim3(P2G_THREADS), 0,
-                           s, ps, n,
+        hipLaunchKernelGGL((k_p2g_tiled<DenseNodes, P2GSource>), p2g_grid(n), dim3(P2G_THREADS), 0, s, ps, n,
                            map, P2GSource{ps, dt}, A);
         kt.end(K_P2G, s);
         kt.begin(K_SPLAT, s);
-        hipLaunchKernelGGL((k_splat_tiled<DenseCells, SPLAT_BOX_DENSE>), dim3(cdiv(n, P2G_THREADS)), dim3(P2G_THREADS), 0, s, ps, n,
+        hipLaunchKernelGGL((k_splat_tiled<DenseCells>), dim3(cdiv(n, P2G_THREADS)), dim3(P2G_THREADS), 0, s, ps, n,
                            DenseCells{{g.n[0], g.n[1], g.n[2]}}, g.lo[0], g.lo[1], g.lo[2], g.dx, dt, phip.p);
         kt.end(K_SPLAT, s);
         MAEL_LAUNCH_CHECK();
@@ -135,114 +144,28 @@ __device__ inline float gather_value(const V* __restrict__ u, int n1, int n2, in
     return vel;
 }
 
-// flip.jl:1226-1244 g2p_kernel!, tiled: per component, a workgroup's 256 particles
-// (cell-sorted, so close together) gather the flags and the velocity from a box of
-// (value, flag) staged in LDS, one read of each face per workgroup instead of two per
-// particle and node; a workgroup spread over more nodes than the box holds, or a particle
-// outside it, reads the faces directly. Both paths take the flags' sum (gather_value) and
-// the APIC sums (gather) in their order of operations, with the indices clamped to the
-// array as there, so the result is theirs bit for bit.
-constexpr int DG2P_BOX = 4096;   // 32 KB: the cell order runs along whole rows, two runs of a row far apart
-__global__ __launch_bounds__(256) void k_dense_g2p(PView ps, int64_t n, DGrid g, const float* __restrict__ u,
-                                                   const float* __restrict__ v, const float* __restrict__ w,
-                                                   const uint8_t* __restrict__ fu, const uint8_t* __restrict__ fv,
-                                                   const uint8_t* __restrict__ fw, float dt, float gravity) {
-    __shared__ float2 sbox[DG2P_BOX];   // value, flag
-    __shared__ int red[6 * 4];
-    const int64_t p = (int64_t)xcd_tile(blockIdx.x, gridDim.x) * 256 + threadIdx.x;   // neighbouring tiles on one XCD
-    const bool live = p < n;
-    float xp = 0, yp = 0, zp = 0;
-    if (live) { xp = ps.f[0][p]; yp = ps.f[1][p]; zp = ps.f[2][p]; }
-    const float* U[3] = {u, v, w};
-    const uint8_t* F[3] = {fu, fv, fw};
-    float fl[3], val[3], c0[3], c1[3], c2[3];
-    for (int a = 0; a < 3; ++a) {
-        const int n1 = g.n[0] + (a == 0), n2 = g.n[1] + (a == 1), n3 = g.n[2] + (a == 2);
-        const float q0 = ispace(xp, g.lo[0], g.dx, a == 0 ? 0.0f : 0.5f);
-        const float q1 = ispace(yp, g.lo[1], g.dx, a == 1 ? 0.0f : 0.5f);
-        const float q2 = ispace(zp, g.lo[2], g.dx, a == 2 ? 0.0f : 0.5f);
-        const BSpline bx = bspline(q0), by = bspline(q1), bz = bspline(q2);
-        const bool ok = live && bx.b > -(1 << 24) && bx.b < (1 << 24) && by.b > -(1 << 24) && by.b < (1 << 24) &&
-                        bz.b > -(1 << 24) && bz.b < (1 << 24) && isfinite(q0) && isfinite(q1) && isfinite(q2);
-        const int BIG = 1 << 30;
-        int x0, y0, z0, x1, y1, z1;
-        wg_bounds(ok, bx.b, by.b, bz.b, red, x0, y0, z0, x1, y1, z1);
-        const int ex = x1 - x0 + 3, ey = y1 - y0 + 3, ez = z1 - z0 + 3;
-        const bool boxed = x0 != BIG && ex <= DG2P_BOX && ey <= DG2P_BOX && ez <= DG2P_BOX && ex * ey * ez <= DG2P_BOX;
-        const float* Ua = U[a];
-        const uint8_t* Fa = F[a];
-        if (boxed) {
-            const int V = ex * ey * ez;
-            for (int k = threadIdx.x; k < V; k += 256) {
-                const int i = min(max(x0 + k % ex, 0), n1 - 1), j = min(max(y0 + (k / ex) % ey, 0), n2 - 1),
-                          kk = min(max(z0 + k / (ex * ey), 0), n3 - 1);
-                const size_t idx = (size_t)i + (size_t)n1 * ((size_t)j + (size_t)n2 * kk);
-                sbox[k] = make_float2(Ua[idx], (float)Fa[idx]);
-            }
-            __syncthreads();
-        }
-        if (live) {
-            if (boxed && ok) {
-                const float wx[3] = {bx.w0, bx.w1, bx.w2}, wy[3] = {by.w0, by.w1, by.w2}, wz[3] = {bz.w0, bz.w1, bz.w2};
-                float d0[3], d1[3], d2[3];
-#pragma unroll
-                for (int m = 0; m < 3; ++m) {
-                    d0[m] = (float)(bx.b + m) - q0;
-                    d1[m] = (float)(by.b + m) - q1;
-                    d2[m] = (float)(bz.b + m) - q2;
-                }
-                const float2* bp = sbox + ((bx.b - x0) + ex * ((by.b - y0) + ey * (bz.b - z0)));
-                float f_ = 0.0f, v_ = 0.0f, s0 = 0.0f, s1 = 0.0f, s2 = 0.0f;
-#pragma unroll
-                for (int mz = 0; mz < 3; ++mz)
-#pragma unroll
-                    for (int my = 0; my < 3; ++my) {
-                        const float2* row = bp + ex * (my + ey * mz);
-#pragma unroll
-                        for (int mx = 0; mx < 3; ++mx) {
-                            const float2 e = row[mx];
-                            const float wgt = (wx[mx] * wy[my]) * wz[mz];
-                            f_ += wgt * e.y;
-                            const float t = wgt * e.x;
-                            v_ += t;
-                            s0 += (t * d0[mx]) * g.dx;
-                            s1 += (t * d1[my]) * g.dx;
-                            s2 += (t * d2[mz]) * g.dx;
-                        }
-                    }
-                const float c = __fdiv_rn(4.0f, g.dx * g.dx);
-                fl[a] = f_; val[a] = v_; c0[a] = s0 * c; c1[a] = s1 * c; c2[a] = s2 * c;
-            } else {
-                fl[a] = gather_value(Fa, n1, n2, n3, g, a, xp, yp, zp);
-                gather(Ua, n1, n2, n3, g, a, xp, yp, zp, val[a], c0[a], c1[a], c2[a]);
-            }
-        }
-        if (boxed) __syncthreads();   // the box is reused by the next component
+// The gather's face nodes: indices clamped to the array (flip.jl:1210-1224).
+struct DenseClampNodes {
+    static constexpr bool HOLES = false;
+    int n[3];
+    __device__ int64_t index(int a, int I, int J, int K) const {
+        int n1 = n[0] + (a == 0), n2 = n[1] + (a == 1), n3 = n[2] + (a == 2);
+        I = min(max(I, 0), n1 - 1); J = min(max(J, 0), n2 - 1); K = min(max(K, 0), n3 - 1);
+        return (int64_t)I + (int64_t)n1 * ((int64_t)J + (int64_t)n2 * K);
     }
-    if (!live) return;
-    // v and c (fields 3..14) built in registers and stored unconditionally, so no store's
-    // target depends on the divergent branch (see k_dense_spawn).
-    float rec[12];
-    if (fl[0] > 0.999f && fl[1] > 0.999f && fl[2] > 0.999f) {
-        rec[0] = val[0]; rec[3] = c0[0]; rec[4] = c1[0]; rec[5] = c2[0];
-        rec[1] = val[1]; rec[6] = c0[1]; rec[7] = c1[1]; rec[8] = c2[1];
-        rec[2] = val[2]; rec[9] = c0[2]; rec[10] = c1[2]; rec[11] = c2[2];
-    } else {
-        rec[0] = ps.f[3][p];
-        rec[1] = ps.f[4][p];
-        rec[2] = ps.f[5][p] - gravity * dt;
-#pragma unroll
-        for (int f = 3; f < 12; ++f) rec[f] = 0.0f;
-    }
-#pragma unroll
-    for (int f = 0; f < 12; ++f) ps.f[3 + f][p] = rec[f];
-}
+    static constexpr int TAB = 1;   // no table
+    struct Near {};
+    __device__ Near near(bool, const int*, const int*) const { return {}; }
+    __device__ void stage(const Near&, int32_t*) const {}
+    __device__ int64_t at(const Near&, const int32_t*, int a, int I, int J, int K) const { return index(a, I, J, K); }
+};
 
 void DenseBasin::g2p(float dt, float grav) {
     if (n == 0) return;
     kt.begin(K_G2P, st.s);
-    hipLaunchKernelGGL(k_dense_g2p, dim3(cdiv(n, 256)), dim3(256), 0, st.s, view(cur), n, g, u[0].p, u[1].p, u[2].p,
-                       flag[0].p, flag[1].p, flag[2].p, dt, grav);
+    const G2PFaces F{{u[0].p, u[1].p, u[2].p}, {flag[0].p, flag[1].p, flag[2].p}};
+    hipLaunchKernelGGL(k_g2p_tiled<DenseClampNodes>, dim3(cdiv(n, P2G_THREADS)), dim3(P2G_THREADS), 0, st.s, view(cur), n,
+                       DenseClampNodes{{g.n[0], g.n[1], g.n[2]}}, g.lo[0], g.lo[1], g.lo[2], g.dx, F, dt, grav);
     kt.end(K_G2P, st.s);
     MAEL_LAUNCH_CHECK();
 }
@@ -257,17 +180,6 @@ namespace mael {
 // velocities; these are their transposes, for reverse-mode gradients. The G2P adjoint is
 // a deposit (the tiled fixed-point scatter, so it is deterministic), the P2G adjoint a
 // gather.
-
-// The gather's face nodes: indices clamped to the array (flip.jl:1210-1224).
-struct DenseClampNodes {
-    int n[3];
-    __device__ int64_t index(int a, int I, int J, int K) const {
-        int n1 = n[0] + (a == 0), n2 = n[1] + (a == 1), n3 = n[2] + (a == 2);
-        I = min(max(I, 0), n1 - 1); J = min(max(J, 0), n2 - 1); K = min(max(K, 0), n3 - 1);
-        return (int64_t)I + (int64_t)n1 * ((int64_t)J + (int64_t)n2 * K);
-    }
-};
-
 
 // Which particles took the grid's velocity in G2P (the flags' gathers, as k_dense_g2p),
 // and the largest contribution one of them makes to a node, as float bits (for the scale).
@@ -360,8 +272,7 @@ void DenseBasin::g2p_adjoint(float dt) {
                      reached.p, 4.0f / (g.dx * g.dx)};
     P2GArgs A{{g.lo[0], g.lo[1], g.lo[2]}, g.dx, {adjacc[0].p, adjacc[1].p, adjacc[2].p}, {nullptr, nullptr, nullptr},
               (float)scale};
-    hipLaunchKernelGGL((k_p2g_tiled<DenseClampNodes, G2PAdjSource, P2G_BOX_DENSE>), dim3(cdiv(n, P2G_THREADS)), dim3(P2G_THREADS),
-                       0, s,
+    hipLaunchKernelGGL((k_p2g_tiled<DenseClampNodes, G2PAdjSource>), p2g_grid(n), dim3(P2G_THREADS), 0, s,
                        view(cur), n, DenseClampNodes{{g.n[0], g.n[1], g.n[2]}}, src, A);
     for (int a = 0; a < 3; ++a)
         hipLaunchKernelGGL(k_adj_fromfix, dim3(cdiv(faces(a), 256)), dim3(256), 0, s, ub[a].p, adjacc[a].p, faces(a),
