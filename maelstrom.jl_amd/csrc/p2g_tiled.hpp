@@ -93,6 +93,12 @@ struct P2GSource {   // flip.jl:513-537: v_a and the APIC row c_a, weighted by t
     }
 };
 
+// b + m where b may be the saturated coordinate of a particle far off the grid or not finite:
+// a defined wrap, so that the bounds test of the sum and its use see one value. (In signed
+// arithmetic the compiler tested b < -m on one side and b + m + 1 > n on the other, which
+// together pass INT_MAX, and the add went out of bounds.)
+__device__ inline int node_at(int b, int m) { return (int)((unsigned)b + (unsigned)m); }
+
 // The contributions of a particle to the 27 nodes from (bx.b, by.b, bz.b), in the order of
 // operations of flip.jl:524-533 with the factors shared along rows hoisted:
 // wgt = ((wT w_x) w_y) w_z and v = vp + ((c0 d0 + c1 d1) + c2 d2) are the same operations on
@@ -121,13 +127,25 @@ __device__ inline void p2g_nodes(const BSpline& bx, const BSpline& by, const BSp
             }
         }
 }
-__device__ inline bool p2g_base_ok(const BSpline& b) { return b.b > -(1 << 24) && b.b < (1 << 24); }
-
-// b + m where b may be the saturated coordinate of a particle far off the grid or not finite:
-// a defined wrap, so that the bounds test of the sum and its use see one value. (In signed
-// arithmetic the compiler tested b < -m on one side and b + m + 1 > n on the other, which
-// together pass INT_MAX, and the add went out of bounds.)
-__device__ inline int node_at(int b, int m) { return (int)((unsigned)b + (unsigned)m); }
+// The same contributions one by one (the rare paths, kept rolled), rounded by tofix.
+template <bool SCALED, class Add>
+__device__ __forceinline__ void p2g_one_by_one(int a, float qx, float qy, float qz, float vp, float c0, float c1, float c2,
+                                               float wT, float dx, float scale, Add add) {
+    const float q0 = a == 0 ? qx : qx - 0.5f, q1 = a == 1 ? qy : qy - 0.5f, q2 = a == 2 ? qz : qz - 0.5f;
+    const BSpline bx = bspline(q0), by = bspline(q1), bz = bspline(q2);
+    const float x0 = bx.w0, x1 = bx.w1, x2 = bx.w2, y0 = by.w0, y1 = by.w1, y2 = by.w2, z0 = bz.w0, z1 = bz.w1, z2 = bz.w2;
+#pragma unroll 1
+    for (int m = 0; m < 27; ++m) {
+        const int mx = m % 3, my = (m / 3) % 3, mz = m / 9;
+        const int I = node_at(bx.b, mx), J = node_at(by.b, my), K = node_at(bz.b, mz);
+        const float wx = mx == 0 ? x0 : (mx == 1 ? x1 : x2), wy = my == 0 ? y0 : (my == 1 ? y1 : y2),
+                    wz = mz == 0 ? z0 : (mz == 1 ? z1 : z2);
+        const float wgt = wT * wx * wy * wz;
+        const float d0 = ((float)I - q0) * dx, d1 = ((float)J - q1) * dx, d2 = ((float)K - q2) * dx;
+        const float mo = wgt * (vp + (c0 * d0 + c1 * d1 + c2 * d2));
+        add(I, J, K, tofix(SCALED ? mo * scale : mo), tofix(wgt));
+    }
+}
 
 // The boxes a workgroup's particles take: over its `act` lanes, the bounds of the first
 // nodes of the three components. A component sits at offset 0 along its own axis and 1/2
@@ -143,12 +161,13 @@ struct NodeBoxes {
     __device__ static bool fits(float qo) {
         return fabsf(qo) < 8388608.0f && (unsigned)first_o(qo) - (unsigned)first_h(qo) <= 1u;
     }
+    __device__ static int sum(bool act, float qo) { return act ? first_o(qo) + first_h(qo) : 0; }
     __device__ NodeBoxes(bool act, const float (&qo)[3], int* red) {
         const int BIG = 1 << 30;
         int v[6];
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-            const int s = act ? first_o(qo[k]) + first_h(qo[k]) : 0;
+            const int s = sum(act, qo[k]);
             v[k] = act ? s : BIG; v[3 + k] = act ? -s : BIG;
         }
         wg_mins(v, red);
@@ -181,12 +200,12 @@ struct NodeBoxes {
 // sides hold particles, so this ends). act becomes the lanes of the box.
 __device__ inline NodeBoxes fitting_boxes(bool& act, const float (&qo)[3], int cap, int* red) {
     NodeBoxes B(act, qo, red);
+    const int s0 = NodeBoxes::sum(act, qo[0]), s1 = NodeBoxes::sum(act, qo[1]), s2 = NodeBoxes::sum(act, qo[2]);
     while (B.any && B.largest() > cap) {
         const int e0 = B.hi[0] - B.lo[0], e1 = B.hi[1] - B.lo[1], e2 = B.hi[2] - B.lo[2];
         const int k = e0 >= e1 && e0 >= e2 ? 0 : (e1 >= e2 ? 1 : 2);
         const int lo = k == 0 ? B.lo[0] : (k == 1 ? B.lo[1] : B.lo[2]), hi = k == 0 ? B.hi[0] : (k == 1 ? B.hi[1] : B.hi[2]);
-        const float q = k == 0 ? qo[0] : (k == 1 ? qo[1] : qo[2]);
-        act = act && NodeBoxes::first_o(q) + NodeBoxes::first_h(q) < (lo + hi + 1) >> 1;
+        act = act && (k == 0 ? s0 : (k == 1 ? s1 : s2)) < (lo + hi + 1) >> 1;
         B = NodeBoxes(act, qo, red);
     }
     return B;
@@ -233,27 +252,9 @@ __global__ __launch_bounds__(P2G_THREADS, 4) void k_p2g_tiled(PView ps, int64_t 
 #pragma unroll
     for (int k = 0; k < 3; ++k) ok = ok && NodeBoxes::fits(qo[k]);
 
-    // component a's contributions added to the accumulators one by one (the rare path, kept
-    // rolled), the same operations in the same order
-    auto direct = [&](int a, float vp, float c0, float c1, float c2) {
-        const float q0 = a == 0 ? qo[0] : qo[0] - 0.5f, q1 = a == 1 ? qo[1] : qo[1] - 0.5f, q2 = a == 2 ? qo[2] : qo[2] - 0.5f;
-        const BSpline bx = bspline(q0), by = bspline(q1), bz = bspline(q2);
-#pragma unroll 1
-        for (int m = 0; m < 27; ++m) {
-            const int mx = m % 3, my = (m / 3) % 3, mz = m / 9;
-            const int I = node_at(bx.b, mx), J = node_at(by.b, my), K = node_at(bz.b, mz);
-            auto idx = map.index(a, I, J, K);
-            if (idx < 0) continue;
-            const float wgt = wT * pick(bx, mx) * pick(by, my) * pick(bz, mz);
-            const float d0 = ((float)I - q0) * A.dx, d1 = ((float)J - q1) * A.dx, d2 = ((float)K - q2) * A.dx;
-            const float mo = wgt * (vp + (c0 * d0 + c1 * d1 + c2 * d2));
-            atomicAdd(&A.mom[a][idx], tofix(Source::SCALED ? mo * A.scale : mo));
-            if (Source::WEIGHTS) atomicAdd(&A.wt[a][idx], tofix(wgt));
-        }
-    };
-
     // the workgroup's components: all three, or the launch's y-th (p2g_grid)
     auto takes = [&](int a) { return gridDim.y == 1 || (int)blockIdx.y == a; };
+    int large = 0;   // the components left to the direct path
     bool todo = ok;
 #pragma unroll 1
     for (int round = 0; round < BOX_ROUNDS; ++round) {
@@ -268,9 +269,9 @@ __global__ __launch_bounds__(P2G_THREADS, 4) void k_p2g_tiled(PView ps, int64_t 
         B.nodes(lo, hi);
         const typename NodeMap::Near near = map.near(true, lo, hi);
         map.stage(near, stab);
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            if (!takes(a)) continue;
+        auto component = [&](auto axis) __attribute__((always_inline)) {
+            constexpr int a = decltype(axis)::value;
+            if (!takes(a)) return;   // the whole workgroup
             const int x0 = B.first(a, 0), y0 = B.first(a, 1), z0 = B.first(a, 2);
             const int ex = B.extent(a, 0), ey = B.extent(a, 1), size = B.size(a);
             float vp = 0, c0 = 0, c1 = 0, c2 = 0;
@@ -282,21 +283,24 @@ __global__ __launch_bounds__(P2G_THREADS, 4) void k_p2g_tiled(PView ps, int64_t 
             }
             __syncthreads();
             // A particle whose contributions all lie within 2^18 in magnitude takes the short
-            // fixed-point rounding (tofix_near); others go direct, through tofix.
+            // fixed-point rounding (tofix_near), and others go direct at the end; the
+            // adjoint's deposit, whose scale brings most of them past that, takes tofix.
             const float bound = wT * (fabsf(vp) + (fabsf(c0) + fabsf(c1) + fabsf(c2)) * (2.0f * A.dx)) * fabsf(A.scale);
-            if (act && bound < 262144.0f) {
+            if (act) {
                 const float q0 = a == 0 ? qo[0] : qo[0] - 0.5f, q1 = a == 1 ? qo[1] : qo[1] - 0.5f,
                             q2 = a == 2 ? qo[2] : qo[2] - 0.5f;
                 const BSpline bx = bspline(q0), by = bspline(q1), bz = bspline(q2);
                 const int sz = ex * ey, l0 = (bx.b - x0) + ex * (by.b - y0) + sz * (bz.b - z0);
-                p2g_nodes<Source::SCALED>(bx, by, bz, q0, q1, q2, vp, c0, c1, c2, wT, A.dx, A.scale,
-                                          [&](int mx, int my, int mz, float m, float w) {
-                                              const int l = l0 + mx + ex * my + sz * mz;
-                                              atomicAdd(&smom[l], tofix_near(m));
-                                              if (Source::WEIGHTS) atomicAdd(&swt[l], tofix_near(w));
-                                          });
-            } else if (act) {
-                direct(a, vp, c0, c1, c2);
+                if (Source::SCALED || bound < 262144.0f) {
+                    p2g_nodes<Source::SCALED>(bx, by, bz, q0, q1, q2, vp, c0, c1, c2, wT, A.dx, A.scale,
+                                              [&](int mx, int my, int mz, float m, float w) {
+                                                  const int l = l0 + mx + ex * my + sz * mz;
+                                                  atomicAdd(&smom[l], Source::SCALED ? tofix(m) : tofix_near(m));
+                                                  if (Source::WEIGHTS) atomicAdd(&swt[l], tofix_near(w));
+                                              });
+                } else {
+                    large |= 1 << a;
+                }
             }
             __syncthreads();
             const BoxIndex at(ex, ey);
@@ -311,15 +315,26 @@ __global__ __launch_bounds__(P2G_THREADS, 4) void k_p2g_tiled(PView ps, int64_t 
                     if (w) atomicAdd(&A.wt[a][idx], w);
                 }
             }
-        }
+        };
+        component(std::integral_constant<int, 0>{});
+        component(std::integral_constant<int, 1>{});
+        component(std::integral_constant<int, 2>{});
     }
-    if (todo || (live && !ok)) {   // left over: far apart, not finite or far off the grid
-#pragma unroll
+    if (todo || (live && !ok)) large = 7;   // far apart, not finite or far off the grid
+    if (large) {
+#pragma unroll 1
         for (int a = 0; a < 3; ++a) {
-            if (!takes(a)) continue;
+            if (!takes(a) || !(large >> a & 1)) continue;
             float vp, c0, c1, c2;
             src.comp(p, a, vp, c0, c1, c2);
-            direct(a, vp, c0, c1, c2);
+            p2g_one_by_one<Source::SCALED>(a, qo[0], qo[1], qo[2], vp, c0, c1, c2, wT, A.dx, A.scale,
+                                           [&](int I, int J, int K, unsigned long long m, unsigned long long w) {
+                                               auto idx = map.index(a, I, J, K);
+                                               if (idx >= 0) {
+                                                   atomicAdd(&A.mom[a][idx], m);
+                                                   if (Source::WEIGHTS) atomicAdd(&A.wt[a][idx], w);
+                                               }
+                                           });
         }
     }
 }
