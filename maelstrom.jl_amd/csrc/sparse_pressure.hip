@@ -10,6 +10,7 @@
 #include "sparse.hpp"
 #include "scan.hpp"
 #include "precision.hpp"
+#include "mg_levels.hpp"
 #include <chrono>
 #include <cmath>
 
@@ -1081,12 +1082,6 @@ __global__ __launch_bounds__(256) void k_head0(T* __restrict__ outf, T* __restri
 
 // ─── dense levels (sflip.jl:1574-1657) ───────────────────────────────────────
 
-template <class C> struct DViewT {
-    int3 n;
-    const C* c[3];
-    const C* dD;
-    const uint8_t* act;
-};
 // A dense level's cell: diag and the neighbours' sum; all loads issued before any use
 // (an index off the grid reads the cell itself, and its coupling adds nothing).
 template <class T, class C, bool Z = false>
@@ -1167,55 +1162,6 @@ __global__ void k_prolongdense(T* __restrict__ xf, const T* __restrict__ xc, con
     unlin(l, nf.x, nf.y, i, j, k);
     if (actf[l] != 0) xf[l] = sf<T>(lf(xf[l]) + boost * lf(xc[cl(i >> 1, j >> 1, k >> 1, nc.x, nc.y)]));
 }
-// sflip.jl:1623-1657 coarsest_kernel!: red-black Gauss-Seidel from zero in one workgroup,
-// in arithmetic A (FP64 in the mixed-precision solve).
-template <class T, class C, class A>
-__global__ __launch_bounds__(1024) void k_scoarsest(T* __restrict__ x, const T* __restrict__ b, DViewT<C> L, int sweeps) {
-    __shared__ A xs[1024];
-    int t = threadIdx.x;
-    int n0 = L.n.x, n1 = L.n.y, n2 = L.n.z, N = n0 * n1 * n2;
-    bool inside = t < N;
-    int i = t % n0, j = (t / n0) % n1, k = t / (n0 * n1);
-    bool act = inside && L.act[t] != 0;
-    A bi = inside ? (A)lf(b[t]) : A(0);
-    A dg = A(0), cw[6] = {0, 0, 0, 0, 0, 0};
-    int nb[6] = {0, 0, 0, 0, 0, 0};
-    if (act) {
-        dg = (A)lf(L.dD[t]);
-        float c;
-        c = lf(L.c[0][cl(i, j, k, n0 + 1, n1)]);     if (c > 0.0f && i > 0) { cw[0] = c; nb[0] = t - 1; }
-        c = lf(L.c[0][cl(i + 1, j, k, n0 + 1, n1)]); if (c > 0.0f && i < n0 - 1) { cw[1] = c; nb[1] = t + 1; }
-        c = lf(L.c[1][cl(i, j, k, n0, n1 + 1)]);     if (c > 0.0f && j > 0) { cw[2] = c; nb[2] = t - n0; }
-        c = lf(L.c[1][cl(i, j + 1, k, n0, n1 + 1)]); if (c > 0.0f && j < n1 - 1) { cw[3] = c; nb[3] = t + n0; }
-        c = lf(L.c[2][cl(i, j, k, n0, n1)]);         if (c > 0.0f && k > 0) { cw[4] = c; nb[4] = t - n0 * n1; }
-        c = lf(L.c[2][cl(i, j, k + 1, n0, n1)]);     if (c > 0.0f && k < n2 - 1) { cw[5] = c; nb[5] = t + n0 * n1; }
-    }
-    // the diagonal is the same every pass; a pass reads the six neighbours together and
-    // adds the coupled ones (an absent neighbour reads cell 0 and adds nothing)
-    A diag = dg;
-#pragma unroll
-    for (int m = 0; m < 6; ++m)
-        if (cw[m] > A(0)) diag += cw[m];
-    xs[t] = A(0);
-    __syncthreads();
-    int par = (i + j + k + 1) & 1;
-    for (int s = 1; s <= 2 * sweeps; ++s)
-        for (int half = 0; half < 2; ++half) {
-            int colour = s <= sweeps ? half : 1 - half;
-            if (act && par == colour) {
-                A v[6];
-#pragma unroll
-                for (int m = 0; m < 6; ++m) v[m] = xs[nb[m]];
-                A acc = bi;
-#pragma unroll
-                for (int m = 0; m < 6; ++m) acc = cw[m] > A(0) ? acc + cw[m] * v[m] : acc;
-                xs[t] = diag > A(0) ? acc / diag : A(0);
-            }
-            __syncthreads();
-        }
-    if (inside) x[t] = sf<T>((float)xs[t]);
-}
-
 // ─── between the composite levels (sflip.jl:1661-1705) ───────────────────────
 
 template <class T>
@@ -1906,6 +1852,13 @@ struct SVec {   // a pressure-sized vector: fine pool part and coarse part
     float* c;
 };
 
+// Dense levels of at most MG_TILED cells take the tiled launches, with 8^3 tiles up to
+// MG_SMALL cells. At 2.9 M cells (FP16) the halo's repeated rows cost what the saved passes
+// gain (a 5 cm solve 18.1 ms tiled, 18.0 ms with a launch a sweep there); at 368,640 the tiles
+// are ahead (18.1 ms without them). 8^3 tiles put a level of up to 80,000 cells on more
+// CUs: 144 workgroups for 73,728 cells, where 16x8x8 would make 72.
+constexpr size_t MG_TILED = 500000, MG_SMALL = 80000;
+
 struct SparseSolver {
     SparseBasin& s;
     hipStream_t st;
@@ -2116,6 +2069,80 @@ struct SparseSolver {
         smooth<N>(x, b, tmp, L, sweeps - 1);
     }
 
+    // The dense levels of the V-cycle (from the right-hand side in Db[0]); returns the first
+    // level's result. With one pair of sweeps a side, the reference's, the levels of at most
+    // MG_TILED cells take a launch down and one up, and the last ones a launch together.
+    template <class T, class C, class A> T* dense_levels(Hier<T, C>& H, int sweeps, int coarse, float boost) {
+        const int nl = (int)s.D.size();
+        auto cells = [&](int l) { return s.D[l].cells(); };
+        int tail = nl - 1, tiled = nl - 1;   // the first level of the tail, the first tiled one
+        if (sweeps == 1) {
+            while (tail > 0 && nl - tail < MG_TAIL_LEVELS && cells(tail - 1) <= 2048) --tail;
+            tiled = tail;
+            while (tiled > 0 && cells(tiled - 1) <= MG_TILED) --tiled;
+        }
+        std::vector<T*> x(nl);   // each level's result
+        for (int l = 0; l < nl; ++l) x[l] = H.Dx[l];
+        for (int l = 0; l < tiled; ++l) dense_down<T, C>(H, l, sweeps);
+        for (int l = tiled; l < tail; ++l) {
+            const int* n = s.D[l].n;
+            // 8^3 tiles while the larger ones would leave CUs idle
+            if (cells(l) <= MG_SMALL)
+                hipLaunchKernelGGL((k_mgdown<T, C, 8, 8, 8>), dim3(cdiv(n[0], 8) * cdiv(n[1], 8) * cdiv(n[2], 8)), dim3(MG_THREADS), 0,
+                                   st, H.Dx[l], H.Db[l + 1], H.Db[l], H.D[l], i3(s.D[l + 1].n), H.rscale);
+            else
+                hipLaunchKernelGGL((k_mgdown<T, C, 16, 8, 8>), dim3(cdiv(n[0], 16) * cdiv(n[1], 8) * cdiv(n[2], 8)), dim3(MG_THREADS),
+                                   0, st, H.Dx[l], H.Db[l + 1], H.Db[l], H.D[l], i3(s.D[l + 1].n), H.rscale);
+        }
+        MGTailArgs<T, C> G;
+        G.nl = nl - tail;
+        for (int l = tail; l < nl; ++l) G.L[l - tail] = H.D[l];
+        G.b = H.Db[tail];
+        G.x = H.Dx[tail];
+        const int* nc = s.D[nl - 1].n;   // the coarsest solve takes a thread per two cells of a row
+        if (cells(tail) <= 512 && (nc[0] + 1) / 2 * nc[1] * nc[2] <= 256)
+            hipLaunchKernelGGL((k_mgtail<T, C, A, 256>), dim3(1), dim3(256), 0, st, G, coarse, H.rscale, boost);
+        else
+            hipLaunchKernelGGL((k_mgtail<T, C, A, 1024>), dim3(1), dim3(1024), 0, st, G, coarse, H.rscale, boost);
+        for (int l = tail - 1; l >= tiled; --l) {
+            const int* n = s.D[l].n;
+            if (cells(l) <= MG_SMALL)
+                hipLaunchKernelGGL((k_mgup<T, C, 8, 8, 8>), dim3(cdiv(n[0], 8) * cdiv(n[1], 8) * cdiv(n[2], 8)), dim3(MG_THREADS), 0, st,
+                                   H.Dt[l], H.Dx[l], x[l + 1], H.Db[l], H.D[l], i3(s.D[l + 1].n), boost);
+            else
+                hipLaunchKernelGGL((k_mgup<T, C, 16, 8, 8>), dim3(cdiv(n[0], 16) * cdiv(n[1], 8) * cdiv(n[2], 8)), dim3(MG_THREADS), 0,
+                                   st, H.Dt[l], H.Dx[l], x[l + 1], H.Db[l], H.D[l], i3(s.D[l + 1].n), boost);
+            x[l] = H.Dt[l];
+        }
+        for (int l = tiled - 1; l >= 0; --l) dense_up<T, C>(H, l, x[l + 1], sweeps, boost);
+        return x[0];
+    }
+    // a level's way down and up with any number of sweep pairs, a launch a sweep
+    template <class T, class C> void dense_down(Hier<T, C>& H, int l, int sweeps) {
+        SLevel &Dl = s.D[l], &Cn = s.D[l + 1];
+        size_t c = Dl.cells();
+        if (sweeps < 1) zero_t(H.Dx[l], c);
+        for (int k = 0; k < sweeps; ++k) {   // from x = 0: the first sweep reads no x
+            if (k == 0)
+                hipLaunchKernelGGL((k_rowdense<3, T, C>), dim3(cdiv(c, 256)), dim3(256), 0, st, H.Dt[l], H.Dx[l], H.Db[l], H.D[l]);
+            else
+                hipLaunchKernelGGL((k_rowdense<0, T, C>), dim3(cdiv(c, 256)), dim3(256), 0, st, H.Dt[l], H.Dx[l], H.Db[l], H.D[l]);
+            hipLaunchKernelGGL((k_rowdense<0, T, C>), dim3(cdiv(c, 256)), dim3(256), 0, st, H.Dx[l], H.Dt[l], H.Db[l], H.D[l]);
+        }
+        hipLaunchKernelGGL((k_residrestrict<T, C>), dim3(cdiv(Cn.cells(), 256)), dim3(256), 0, st, H.Db[l + 1], H.Dx[l], H.Db[l],
+                           H.D[l], i3(Cn.n), H.rscale);
+    }
+    template <class T, class C> void dense_up(Hier<T, C>& H, int l, const T* coarser, int sweeps, float boost) {
+        SLevel &Dl = s.D[l], &Cn = s.D[l + 1];
+        size_t c = Dl.cells();
+        hipLaunchKernelGGL(k_prolongdense<T>, dim3(cdiv(c, 256)), dim3(256), 0, st, H.Dx[l], coarser, Dl.act.p, i3(Dl.n), i3(Cn.n),
+                           boost);
+        for (int k = 0; k < sweeps; ++k) {
+            hipLaunchKernelGGL((k_rowdense<0, T, C>), dim3(cdiv(c, 256)), dim3(256), 0, st, H.Dt[l], H.Dx[l], H.Db[l], H.D[l]);
+            hipLaunchKernelGGL((k_rowdense<0, T, C>), dim3(cdiv(c, 256)), dim3(256), 0, st, H.Dx[l], H.Dt[l], H.Db[l], H.D[l]);
+        }
+    }
+
     // sflip.jl:1722-1762 vcycle!: z = M^-1 r in the hierarchy H (coarsest in arithmetic A).
     template <class T, class C, class A>
     void vcycle_t(Hier<T, C>& H, SVecT<T> z, SVecT<T> r, int sweeps, int coarse, float boost, bool queued = false) {
@@ -2128,39 +2155,11 @@ struct SparseSolver {
         smooth0<8>(H.X1x, H.X1b, H.X1t, H.L1, sweeps, (size_t)ns * SBCELLS1);
         rows<8, 1>(H.X1r, H.X1x, H.X1b, H.L1);
         hipLaunchKernelGGL(k_restrict12<T>, dim3(cdiv(Cc, 256)), dim3(256), 0, st, H.Db[0], H.X1r.f, H.X1r.c, t);
-        int nl = (int)s.D.size();
-        for (int l = 0; l + 1 < nl; ++l) {
-            SLevel& Dl = s.D[l];
-            size_t c = Dl.cells();
-            if (sweeps < 1) zero_t(H.Dx[l], c);
-            for (int k = 0; k < sweeps; ++k) {   // from x = 0: the first sweep reads no x
-                if (k == 0)
-                    hipLaunchKernelGGL((k_rowdense<3, T, C>), dim3(cdiv(c, 256)), dim3(256), 0, st, H.Dt[l], H.Dx[l], H.Db[l],
-                                       H.D[l]);
-                else
-                    hipLaunchKernelGGL((k_rowdense<0, T, C>), dim3(cdiv(c, 256)), dim3(256), 0, st, H.Dt[l], H.Dx[l], H.Db[l],
-                                       H.D[l]);
-                hipLaunchKernelGGL((k_rowdense<0, T, C>), dim3(cdiv(c, 256)), dim3(256), 0, st, H.Dx[l], H.Dt[l], H.Db[l], H.D[l]);
-            }
-            SLevel& Cn = s.D[l + 1];
-            hipLaunchKernelGGL((k_residrestrict<T, C>), dim3(cdiv(Cn.cells(), 256)), dim3(256), 0, st, H.Db[l + 1], H.Dx[l],
-                               H.Db[l], H.D[l], i3(Cn.n), H.rscale);
-        }
-        hipLaunchKernelGGL((k_scoarsest<T, C, A>), dim3(1), dim3(1024), 0, st, H.Dx[nl - 1], H.Db[nl - 1], H.D[nl - 1], coarse);
-        for (int l = nl - 2; l >= 0; --l) {
-            SLevel &Dl = s.D[l], &Cn = s.D[l + 1];
-            size_t c = Dl.cells();
-            hipLaunchKernelGGL(k_prolongdense<T>, dim3(cdiv(c, 256)), dim3(256), 0, st, H.Dx[l], H.Dx[l + 1], Dl.act.p, i3(Dl.n),
-                               i3(Cn.n), boost);
-            for (int k = 0; k < sweeps; ++k) {
-                hipLaunchKernelGGL((k_rowdense<0, T, C>), dim3(cdiv(c, 256)), dim3(256), 0, st, H.Dt[l], H.Dx[l], H.Db[l], H.D[l]);
-                hipLaunchKernelGGL((k_rowdense<0, T, C>), dim3(cdiv(c, 256)), dim3(256), 0, st, H.Dx[l], H.Dt[l], H.Db[l], H.D[l]);
-            }
-        }
+        T* x2 = dense_levels<T, C, A>(H, sweeps, coarse, boost);
         SLevel& D2 = s.D[0];
         const uint32_t ncb = (uint32_t)cdiv(Cc, 256), nfb1 = (uint32_t)cdiv((size_t)ns * SBCELLS1, 256);
-        hipLaunchKernelGGL((k_prolongcomp<T, 1>), dim3(nfb1 + ncb), dim3(256), 0, st, H.X1x.f, H.Dx[0], s.act1.p, H.X1x.c,
-                           H.Dx[0], D2.act.p, t, boost, ns, nfb1);
+        hipLaunchKernelGGL((k_prolongcomp<T, 1>), dim3(nfb1 + ncb), dim3(256), 0, st, H.X1x.f, x2, s.act1.p, H.X1x.c, x2,
+                           D2.act.p, t, boost, ns, nfb1);
         smooth<8>(H.X1x, H.X1b, H.X1t, H.L1, sweeps);
         const uint32_t nfb0 = (uint32_t)cdiv((size_t)nf, 1024);
         hipLaunchKernelGGL((k_prolongcomp<T, 0>), dim3(nfb0 + ncb), dim3(256), 0, st, z.f, H.X1x.f, s.types.fine.p, z.c, H.X1x.c,

@@ -1,0 +1,46 @@
+"""The dense levels of the sparse basin's V-cycle on grids whose levels take each of their
+launches: tiles of 8^3 and 16x8x8 cells with remainders, a launch a sweep (the largest
+level, and more than one pair of sweeps), the one-workgroup tail of one, two and three
+levels, and an odd coarsest level. No fine blocks: the composite levels are the coarse grid."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+# radius, depth -> the coarse grid; V-cycle levels follow by halves to at most 1024 cells
+CASES = {
+    "one level, 16^3 halved once": (18.0, 12.0, (16, 16, 16)),
+    "8^3 tiles and an odd coarsest level, 112x112x48 .. 14x14x6, 7x7x3": (125.0, 85.0, (112, 112, 48)),
+    "16x8x8 tiles, 80x80x32 .. 10x10x4": (90.0, 60.0, (80, 80, 32)),
+}
+
+
+@pytest.mark.parametrize("precision,sweeps", [(0, 1), (0, 2), (1, 1), (2, 1)])
+@pytest.mark.parametrize("case", sorted(CASES))
+def test_levels_match_oracle(mael, case, precision, sweeps):
+    radius, depth, dims = CASES[case]
+    print("case: %s precision %d sweeps %d" % (case, precision, sweeps), flush=True)
+    o = O.SparseOracle(radius, depth, 3.0, 0.6, 2, 1, 16, 4, 8)
+    g = o.grid
+    rmax = np.float32(np.hypot(np.float32(g.lo[0]), np.float32(g.lo[1])))
+    o.init_coarse(O.surface_table(225.0, 2.5, 9.81, rmax), rmax, 225.0, 2.5)
+    o.classify()
+    s = mael.SparseBasin(mael.Basin(radius=radius, depth=depth, Γ=225.0, core=2.5), dx=0.6, blocks=1, capacity=16)
+    assert s.nc == dims
+    s.set("PHI_C", o.array("phi_c"))
+    s.set("TYPES_C", o.array("types_c"))
+    rng = np.random.default_rng(5)
+    rc = np.where(o.array("types_c") == 1, rng.normal(0, 1, o.array("types_c").size), 0).astype(np.float32)
+    s.set("RHS_C", rc)
+    opts = mael.sparse.solve_options(precision=precision, boost=1.0, sweeps=sweeps)
+    s.ctx.check(mael.lib().mael_sparse_vcycle(s.h, C.byref(opts), 0))
+    z = s.get("P_C").ravel().astype(np.float64)
+    _, ze = o.vcycle(np.zeros(o.array("P_f").size, np.float32), rc, sweeps=sweeps, coarse=opts.coarse, boost=1.0)
+    err = np.linalg.norm(z - ze) / np.linalg.norm(ze)
+    print("rel L2 vs FP64 oracle %.3e" % err, flush=True)
+    # the storage's rounding (2^-24, 2^-11, 2^-8) through a few tens of passes
+    assert err < {0: 1e-5, 1: 3e-3, 2: 2e-2}[precision], err
