@@ -14,6 +14,7 @@
 // FP32 stagnation floor (fgmres.jl:56-58 notes one above 5e-4).
 #include "dense.hpp"
 #include "scan.hpp"
+#include "mg_rbgs.hpp"
 #include <chrono>
 #include <cmath>
 
@@ -114,6 +115,32 @@ __global__ void k_diag(float* __restrict__ diag, const uint8_t* __restrict__ typ
         }
     }
     diag[c] = d;
+}
+
+// flip.jl:838-848 celldiag of the coarse levels, up to CDIAG_LEVELS of them in one launch
+// (a level a row of workgroups): the neighbours that are not SOLID, 0 off the LIQUID cells.
+constexpr int CDIAG_LEVELS = 8;
+struct CoarseDiags {
+    float* d[CDIAG_LEVELS];
+    const uint8_t* t[CDIAG_LEVELS];
+    int3 n[CDIAG_LEVELS];
+};
+__global__ void k_coarsediag(CoarseDiags A) {
+    const int3 n = A.n[blockIdx.y];
+    const uint8_t* __restrict__ t = A.t[blockIdx.y];
+    const size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= (size_t)n.x * n.y * n.z) return;
+    int i, j, k;
+    unlin(c, n.x, n.y, i, j, k);
+    const Nb6 nb = nb6(i, j, k, n);
+    uint8_t tv[6];
+#pragma unroll
+    for (int m = 0; m < 6; ++m) tv[m] = t[nb.e[m]];
+    float d = 0.0f;
+#pragma unroll
+    for (int m = 0; m < 6; ++m)
+        if (nb.in[m] && tv[m] != SOLID) d += 1.0f;
+    A.d[blockIdx.y][c] = t[c] == LIQUID ? d : 0.0f;
 }
 
 // flip.jl:838-857 celldiag / liquidsum; `diag` null on the coarse levels.
@@ -270,50 +297,6 @@ __global__ void k_prolong(float* __restrict__ xf, const float* __restrict__ xc, 
     for (int m = 0; m < 8; ++m)
         if (in[m] && tv[m] == LIQUID) s += WA[m & 1] * WB[(m >> 1) & 1] * WC[(m >> 2) & 1] * xv[m];
     xf[c] = x0 + s;
-}
-
-// flip.jl:931-962 coarse_kernel!: the coarsest level (<= 1024 cells) in one workgroup,
-// `sweeps` RBGS sweeps from zero then as many in reverse colour order. Accumulates in T
-// (FP32 as the reference, or FP64).
-template <class T>
-__global__ __launch_bounds__(1024) void k_coarsest(float* __restrict__ x, const float* __restrict__ b,
-                                                   const uint8_t* __restrict__ types, int3 n, int sweeps) {
-    __shared__ T xs[1024];
-    int t = threadIdx.x;
-    int N = n.x * n.y * n.z;
-    bool active = t < N;
-    int i = t % n.x, j = (t / n.x) % n.y, k = t / (n.x * n.y);
-    uint8_t ti = active ? types[t] : SOLID;
-    T bi = active ? (T)b[t] : T(0);
-    T d = 0;
-    int nbr[6];
-    bool liq[6];
-#pragma unroll
-    for (int m = 0; m < 6; ++m) {
-        int a = i + NB6[m][0], bb = j + NB6[m][1], c = k + NB6[m][2];
-        uint8_t tn = active ? typeat(types, a, bb, c, n.x, n.y, n.z) : SOLID;
-        if (tn != SOLID) d += T(1);
-        liq[m] = tn == LIQUID;
-        nbr[m] = liq[m] ? a + n.x * (bb + n.y * c) : 0;
-    }
-    xs[t] = T(0);
-    __syncthreads();
-    int par = (i + j + k + 1) & 1;
-    for (int s = 1; s <= 2 * sweeps; ++s)
-        for (int half = 0; half < 2; ++half) {
-            int colour = s <= sweeps ? half : 1 - half;
-            if (active && ti == LIQUID && par == colour) {
-                T v[6];   // the six neighbours read together (a non-liquid one reads cell 0)
-#pragma unroll
-                for (int m = 0; m < 6; ++m) v[m] = xs[nbr[m]];
-                T acc = bi;
-#pragma unroll
-                for (int m = 0; m < 6; ++m) acc = liq[m] ? acc + v[m] : acc;
-                xs[t] = d > T(0) ? acc / d : T(0);
-            }
-            __syncthreads();
-        }
-    if (active) x[t] = (float)xs[t];
 }
 
 // ─── CG passes ───────────────────────────────────────────────────────────────
@@ -482,6 +465,14 @@ static inline dim3 grid3(int n1, int n2, int n3) { return dim3(cdiv(n1, BX), cdi
 static inline int3 i3(const int n[3]) { return make_int3(n[0], n[1], n[2]); }
 constexpr int RED_BLOCKS = 1024;   // workgroups of the 1-D reductions
 
+// Levels of at most RB_TILED cells take a launch down and one up: a level of 131,072 cells
+// is 256 tiles, one a CU (a backward pass on 128x128x64 1,700 us, 1,845 us with that level a
+// launch a pass), and one of 1 M cells is 2,048 of them (1,890 us tiled there too). The
+// one-workgroup tail holds a level of RB_TAIL_SMALL or RB_TAIL_CELLS cells with the layer
+// round it.
+constexpr size_t RB_TILED = 300000;
+constexpr int RB_TAIL_SMALL = 4096, RB_TAIL_CELLS = 12288;
+
 struct DenseSolver {
     DenseBasin& s;
     hipStream_t st;
@@ -504,45 +495,90 @@ struct DenseSolver {
         hipLaunchKernelGGL(k_rbgs, grid3(n.x / 2, n.y, n.z), dim3(BX, BY), 0, st, x, b, types(l), diag(l), n, colour);
         if (l == 0) s.kt.end(K_RBGS, st);
     }
-    // The V-cycle's first launches (level 0's start and first sweep) queued ahead of a
-    // host read that decides whether the V-cycle runs, so the device works through the
-    // read's round trip; the next vcycle() skips them. Whoever leaves the solve or changes
-    // r first clears `head`.
+    // A level's way down and up in one launch each (mg_rbgs.hpp), for levels of at most
+    // RB_TILED cells and the reference's two sweeps. Down leaves its x in the level's
+    // residual array, for up to read.
+    bool tiled(int l, int sweeps) const { return sweeps == 2 && s.lv[l].cells() <= RB_TILED; }
+    unsigned tiles(int l) const { return cdiv(s.lv[l].n[0], RB) * cdiv(s.lv[l].n[1], RB) * cdiv(s.lv[l].n[2], RB); }
+    float* scratch(int l) { return l == 0 ? s.rv.p : s.lv[l].r.p; }
+    const float* cdiag(int l) const { return l == 0 ? s.diag.p : s.lv[l].diag.p; }
+    void down(int l, const float* b) {
+        hipLaunchKernelGGL(k_rbdown, dim3(tiles(l)), dim3(RB_THREADS), 0, st, scratch(l), s.lv[l + 1].b.p, b, cdiag(l), types(l),
+                           types(l + 1), dims(l), dims(l + 1));
+    }
+    void up(int l, float* x, const float* b) {
+        hipLaunchKernelGGL(k_rbup, dim3(tiles(l)), dim3(RB_THREADS), 0, st, x, scratch(l), s.lv[l + 1].x.p, b, cdiag(l), types(l),
+                           dims(l), dims(l + 1));
+    }
+    // The last levels, from `first`, in one workgroup: the coarsest, and the one before it
+    // where it fits (at most 8,192 cells, as the coarsest has at most 1,024; a long thin one
+    // may not, with the layer round it).
+    int tail_first() const {
+        if (L < 2) return L - 1;
+        const int* n = s.lv[L - 2].n;
+        return (int64_t)(n[0] + 2) * (n[1] + 2) * (n[2] + 2) <= RB_TAIL_CELLS ? L - 2 : L - 1;
+    }
+    void tail(int first, float* x, const float* b, int sweeps, int coarse) {
+        auto level = [&](int l) { return RBLevel{l == first ? x : s.lv[l].x.p, l == first ? b : s.lv[l].b.p, cdiag(l), types(l), dims(l)}; };
+        const RBLevel K = level(L - 1);
+        s.kt.begin(K_COARSEST, st);
+        if (first == L - 1)
+            hipLaunchKernelGGL((k_rbtail<0, 0>), dim3(1), dim3(RB_THREADS), 0, st, K, K, sweeps, coarse);
+        else if (s.lv[first].cells() <= 2048 && rb_padded(dims(first)) <= RB_TAIL_SMALL)
+            hipLaunchKernelGGL((k_rbtail<1, RB_TAIL_SMALL>), dim3(1), dim3(RB_THREADS), 0, st, level(first), K, sweeps, coarse);
+        else
+            hipLaunchKernelGGL((k_rbtail<4, RB_TAIL_CELLS>), dim3(1), dim3(RB_THREADS), 0, st, level(first), K, sweeps, coarse);
+        s.kt.end(K_COARSEST, st);
+    }
+    // The V-cycle's first launches (level 0's start and first sweep, or its way down)
+    // queued ahead of a host read that decides whether the V-cycle runs, so the device
+    // works through the read's round trip; the next vcycle() skips them. Whoever leaves the
+    // solve or changes r first clears `head`.
     bool head = false;
     void queue_head(float* z, const float* r, int sweeps) {
         int3 n = dims(0);
-        hipLaunchKernelGGL(k_start, grid3(n.x, n.y, n.z), dim3(BX, BY), 0, st, z, r, types(0), diag(0), n);
-        if (2 * sweeps - 1 >= 1) smooth(0, z, r, 1);
+        if (tail_first() == 0) return;
+        if (tiled(0, sweeps)) {
+            down(0, r);
+        } else {
+            hipLaunchKernelGGL(k_start, grid3(n.x, n.y, n.z), dim3(BX, BY), 0, st, z, r, types(0), diag(0), n);
+            if (2 * sweeps - 1 >= 1) smooth(0, z, r, 1);
+        }
         head = true;
     }
     // flip.jl:986-1014 vcycle!.
     void vcycle(float* z, const float* r, int sweeps, int coarse) {
         const bool queued = head;
         head = false;
-        std::vector<float*> xs(L), bs(L), rs(L);
+        std::vector<float*> xs(L), bs(L);
         for (int l = 0; l < L; ++l) {
             xs[l] = l == 0 ? z : s.lv[l].x.p;
             bs[l] = l == 0 ? const_cast<float*>(r) : s.lv[l].b.p;
-            rs[l] = l == 0 ? s.rv.p : s.lv[l].r.p;
         }
-        for (int l = 0; l < L - 1; ++l) {
+        const int last = tail_first();
+        for (int l = 0; l < last; ++l) {
             int3 n = dims(l), nc = dims(l + 1);
-            const bool skip = queued && l == 0;   // start and first sweep already queued
+            const bool skip = queued && l == 0;   // start and first sweep, or the way down, already queued
+            if (tiled(l, sweeps)) {
+                if (!skip) down(l, bs[l]);
+                continue;
+            }
             if (!skip)
                 hipLaunchKernelGGL(k_start, grid3(n.x, n.y, n.z), dim3(BX, BY), 0, st, xs[l], bs[l], types(l), diag(l), n);
             for (int c = skip ? 1 : 0; c < 2 * sweeps - 1; ++c) smooth(l, xs[l], bs[l], (c & 1) ? 0 : 1);   // 1,0,1,...
-            residual(l, rs[l], xs[l], bs[l]);
+            residual(l, scratch(l), xs[l], bs[l]);
             if (l == 0) s.kt.begin(K_RESTRICT, st);
-            hipLaunchKernelGGL(k_restrict, grid3(nc.x, nc.y, nc.z), dim3(BX, BY), 0, st, bs[l + 1], rs[l], types(l),
+            hipLaunchKernelGGL(k_restrict, grid3(nc.x, nc.y, nc.z), dim3(BX, BY), 0, st, bs[l + 1], scratch(l), types(l),
                                types(l + 1), n, nc);
             if (l == 0) s.kt.end(K_RESTRICT, st);
         }
-        int3 nL = dims(L - 1);
-        s.kt.begin(K_COARSEST, st);
-        hipLaunchKernelGGL(k_coarsest<float>, dim3(1), dim3(1024), 0, st, xs[L - 1], bs[L - 1], types(L - 1), nL, coarse);
-        s.kt.end(K_COARSEST, st);
-        for (int l = L - 2; l >= 0; --l) {
+        tail(last, xs[last], bs[last], sweeps, coarse);
+        for (int l = last - 1; l >= 0; --l) {
             int3 n = dims(l), nc = dims(l + 1);
+            if (tiled(l, sweeps)) {
+                up(l, xs[l], bs[l]);
+                continue;
+            }
             if (l == 0) s.kt.begin(K_PROLONG, st);
             hipLaunchKernelGGL(k_prolong, grid3(n.x, n.y, n.z), dim3(BX, BY), 0, st, xs[l], xs[l + 1], types(l), types(l + 1),
                                n, nc);
@@ -653,6 +689,12 @@ void DenseBasin::operator_setup() {
         hipLaunchKernelGGL(k_coarsen, grid3(nc.x, nc.y, nc.z), dim3(BX, BY), 0, s, lv[l].types.p, S.types(l - 1), nc, nf);
     }
     hipLaunchKernelGGL(k_diag, grid3(n.x, n.y, n.z), dim3(BX, BY), 0, s, diag.p, types.p, phi.p, n);
+    for (int l = 1; l < levels; l += CDIAG_LEVELS) {
+        CoarseDiags A;
+        const int m = std::min(CDIAG_LEVELS, levels - l);
+        for (int q = 0; q < m; ++q) { A.d[q] = lv[l + q].diag.p; A.t[q] = lv[l + q].types.p; A.n[q] = i3(lv[l + q].n); }
+        hipLaunchKernelGGL(k_coarsediag, dim3(cdiv(lv[l].cells(), 256), m), dim3(256), 0, s, A);
+    }
     MAEL_LAUNCH_CHECK();
 }
 

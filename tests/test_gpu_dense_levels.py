@@ -1,4 +1,6 @@
-"""The dense levels of the sparse basin's V-cycle on grids whose levels take each of their
+"""The V-cycles' small levels, which share launches.
+
+The dense levels of the sparse basin's V-cycle on grids whose levels take each of their
 launches: tiles of 8^3 and 16x8x8 cells with remainders, a launch a sweep (the largest
 level, and more than one pair of sweeps), the one-workgroup tail of one, two and three
 levels, and an odd coarsest level. No fine blocks: the composite levels are the coarse grid."""
@@ -44,3 +46,37 @@ def test_levels_match_oracle(mael, case, precision, sweeps):
     print("rel L2 vs FP64 oracle %.3e" % err, flush=True)
     # the storage's rounding (2^-24, 2^-11, 2^-8) through a few tens of passes
     assert err < {0: 1e-5, 1: 3e-3, 2: 2e-2}[precision], err
+
+
+# radius, depth, top, dx -> cells; the dense V-cycle's levels halve them to at most 1024
+DENSE = {
+    "tiles and a 2,048-cell tail, 64x64x32 .. 8x8x4": (18.0, 12.0, 3.0, 0.6, (64, 64, 32)),
+    "tile remainders and a 4,840-cell tail, 44x44x20 .. 11x11x5": (4.0, 2.0, 1.5, 0.2, (44, 44, 20)),
+    "a level too wide for the tail, 128x128x4 .. 32x32x1": (36.9, 0.6, 0.9, 0.6, (128, 128, 4)),
+    "tiles off by half, 40x40x24 .. 10x10x6": (10.2, 8.0, 5.0, 0.6, (40, 40, 24)),
+}
+
+
+@pytest.mark.parametrize("sweeps,queued", [(1, 0), (2, 0), (2, 1), (3, 1)])
+@pytest.mark.parametrize("case", sorted(DENSE))
+def test_dense_levels_bits(mael, orc, case, sweeps, queued):
+    """The dense basin's V-cycle on random cell types (empty rows and single-cell pools among
+    them) in the oracle's FP32 V-cycle's bits: both take every sum and division in the
+    reference's order."""
+    radius, depth, top, dx, dims = DENSE[case]
+    print("case: %s sweeps %d queued %d" % (case, sweeps, queued), flush=True)
+    g = orc.flipgrid(radius, depth, top, dx)
+    assert g.dims == dims
+    s = mael.FlipBasin(mael.Basin(radius=radius, depth=depth, rimwall=top), dx=dx, capacity=16)
+    rng = np.random.default_rng(3)
+    shape = orc.cells_shape(g)
+    types = rng.choice(np.array([0, 1, 2], np.uint8), shape, p=[0.25, 0.65, 0.1])
+    phi = (rng.uniform(0.01, 1.0, shape) * np.where(types == 1, -1, 1)).astype(np.float32)
+    r = np.where(types == 1, rng.normal(0, 1, shape), 0).astype(np.float32)
+    for name, a in (("TYPES", types), ("PHI", phi), ("RHS", r)):
+        s.set(name, a)
+    opts = mael.dense.solve_options(sweeps=sweeps)
+    s.ctx.check(mael.lib().mael_dense_vcycle(s.h, C.byref(opts), queued))
+    z = s.get("P")
+    ref = orc.dense_vcycle(g, types, phi, r, sweeps=sweeps, fp32=True)
+    assert np.array_equal(z.view(np.uint32), ref.view(np.uint32)), int((z.view(np.uint32) != ref.view(np.uint32)).sum())
