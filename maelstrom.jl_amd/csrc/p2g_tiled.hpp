@@ -624,45 +624,221 @@ struct G2PAdjSource {
 };
 struct PB12 { float* f[12]; };
 
+// The workgroup's largest v (floats >= 0 by their bits) into *bound: an atomic only from a
+// workgroup that raises it.
+__device__ inline void wg_raise(float m, int* bound, int* red) {
+    const int v = -wave_min(-__float_as_int(m));
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const int w = max(max(red[0], red[1]), max(red[2], red[3]));
+        if (w > __hip_atomic_load(bound, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(bound, w);
+    }
+}
+
+// A workgroup's 256 particles over boxes of faces in LDS, component by component, as
+// k_g2p_tiled: stage(k, idx) puts face idx (< 0: none there) of component a at k in the box;
+// take(a, k0, ex, exy, bx, by, bz, q0, q1, q2) reads the box for a particle whose first node
+// is at k0; done() follows a particle's three components. left(a, ...) is a component of a
+// particle that no box took (or that is not to be boxed).
+template <int CAP, class NodeMap, class Stage, class Take, class Left, class Done>
+__device__ __forceinline__ void over_boxes(bool live, bool boxed, float (&qo)[3], const NodeMap& map, int* red, int32_t* stab,
+                                           Stage stage, Take take, Left left, Done done) {
+    bool todo = live && boxed && NodeBoxes::fits(qo[0]) && NodeBoxes::fits(qo[1]) && NodeBoxes::fits(qo[2]);
+    const bool far = live && !todo;
+#pragma unroll 1
+    for (int round = 0; round < BOX_ROUNDS; ++round) {
+        asm volatile("" : "+v"(qo[0]), "+v"(qo[1]), "+v"(qo[2]));   // as in k_p2g_tiled: nothing moved out of the loop
+        bool act = todo;
+        const NodeBoxes B = fitting_boxes(act, qo, CAP, red);
+        if (!B.any) break;
+        todo = todo && !act;
+        int lo[3], hi[3];
+        B.nodes(lo, hi);
+        const typename NodeMap::Near near = map.near(true, lo, hi);
+        map.stage(near, stab);
+        __syncthreads();
+        auto component = [&](auto axis) __attribute__((always_inline)) {
+            constexpr int a = decltype(axis)::value;
+            const int x0 = B.first(a, 0), y0 = B.first(a, 1), z0 = B.first(a, 2);
+            const int ex = B.extent(a, 0), ey = B.extent(a, 1), size = B.size(a);
+            const BoxIndex at(ex, ey);
+            for (int k = threadIdx.x; k < size; k += P2G_THREADS) {
+                int i, j, kk;
+                at.at(k, i, j, kk);
+                stage(axis, k, map.at(near, stab, a, x0 + i, y0 + j, z0 + kk));
+            }
+            __syncthreads();
+            if (act) {
+                const float q0 = a == 0 ? qo[0] : qo[0] - 0.5f, q1 = a == 1 ? qo[1] : qo[1] - 0.5f,
+                            q2 = a == 2 ? qo[2] : qo[2] - 0.5f;
+                const BSpline bx = bspline(q0), by = bspline(q1), bz = bspline(q2);
+                take(axis, (bx.b - x0) + ex * ((by.b - y0) + ey * (bz.b - z0)), ex, ex * ey, bx, by, bz, q0, q1, q2);
+            }
+            __syncthreads();   // the box is reused
+        };
+        component(std::integral_constant<int, 0>{});
+        component(std::integral_constant<int, 1>{});
+        component(std::integral_constant<int, 2>{});
+        if (act) done();
+    }
+    if (todo || far) {   // far apart, not finite or far off the grid
+        auto component = [&](auto axis) __attribute__((always_inline)) {
+            constexpr int a = decltype(axis)::value;
+            const float q0 = a == 0 ? qo[0] : qo[0] - 0.5f, q1 = a == 1 ? qo[1] : qo[1] - 0.5f, q2 = a == 2 ? qo[2] : qo[2] - 0.5f;
+            left(axis, bspline(q0), bspline(q1), bspline(q2), q0, q1, q2);
+        };
+        component(std::integral_constant<int, 0>{});
+        component(std::integral_constant<int, 1>{});
+        component(std::integral_constant<int, 2>{});
+        done();
+    }
+}
+
+// Which particles took the grid's velocity in G2P (the three flag sums > 0.999, in the
+// gather's order of operations), and the largest contribution one of them makes to a node,
+// as float bits (for the deposit's scale). 1.6 M particles at 15 cm 176 -> 78 us against
+// reading the flags from global memory node by node.
+template <class NodeMap>
+__global__ __launch_bounds__(P2G_THREADS) void k_g2p_adj_reached(PView ps, int64_t n, NodeMap map, float lo0, float lo1, float lo2,
+                                                                 float dx, G2PFaces F, uint8_t* __restrict__ reached, PB12 pb,
+                                                                 int* __restrict__ bound) {
+    __shared__ float sflag[G2P_BOX];
+    __shared__ alignas(16) int red[6 * (P2G_THREADS / 64)];
+    __shared__ int32_t stab[NodeMap::TAB];
+    const int64_t p = (int64_t)xcd_tile(blockIdx.x, gridDim.x) * P2G_THREADS + threadIdx.x;
+    const bool live = p < n;
+    float qo[3] = {0.0f, 0.0f, 0.0f}, m = 0.0f;
+    if (live) {
+        qo[0] = ispace(ps.f[0][p], lo0, dx, 0.0f);
+        qo[1] = ispace(ps.f[1][p], lo1, dx, 0.0f);
+        qo[2] = ispace(ps.f[2][p], lo2, dx, 0.0f);
+    }
+    bool ok = true;
+    over_boxes<G2P_BOX>(
+        live, true, qo, map, red, stab,
+        [&](auto axis, int k, auto idx) {
+            constexpr int a = decltype(axis)::value;
+            sflag[k] = idx >= 0 ? (float)F.f[a][idx] : -1.0f;
+        },
+        [&](auto, int k0, int ex, int exy, const BSpline& bx, const BSpline& by, const BSpline& bz, float, float, float) {
+            const float wx[3] = {bx.w0, bx.w1, bx.w2}, wy[3] = {by.w0, by.w1, by.w2}, wz[3] = {bz.w0, bz.w1, bz.w2};
+            float f = 0.0f;
+#pragma unroll
+            for (int mz = 0; mz < 3; ++mz)
+#pragma unroll
+                for (int my = 0; my < 3; ++my)
+#pragma unroll
+                    for (int mx = 0; mx < 3; ++mx) {
+                        const float fl = sflag[k0 + mx + ex * my + exy * mz];
+                        const float wgt = (wx[mx] * wy[my]) * wz[mz];
+                        f += (NodeMap::HOLES && fl < 0.0f ? 0.0f : wgt) * fl;
+                    }
+            ok = ok && f > 0.999f;
+        },
+        [&](auto axis, const BSpline& bx, const BSpline& by, const BSpline& bz, float, float, float) {
+            constexpr int a = decltype(axis)::value;
+            const float x0 = bx.w0, x1 = bx.w1, x2 = bx.w2, y0 = by.w0, y1 = by.w1, y2 = by.w2, z0 = bz.w0, z1 = bz.w1, z2 = bz.w2;
+            float f = 0.0f;
+#pragma unroll 1
+            for (int q = 0; q < 27; ++q) {
+                const int mx = q % 3, my = (q / 3) % 3, mz = q / 9;
+                const auto idx = map.index(a, node_at(bx.b, mx), node_at(by.b, my), node_at(bz.b, mz));
+                if (NodeMap::HOLES && idx < 0) continue;
+                const float wgt = (mx == 0 ? x0 : (mx == 1 ? x1 : x2)) * (my == 0 ? y0 : (my == 1 ? y1 : y2)) *
+                                  (mz == 0 ? z0 : (mz == 1 ? z1 : z2));
+                f += wgt * (float)F.f[a][idx];
+            }
+            ok = ok && f > 0.999f;
+        },
+        [&] {
+            reached[p] = ok ? 1 : 0;
+            if (!ok) return;
+            const float cd = 6.0f / dx;   // |row . d| <= (4 / dx^2)(1.5 dx) sum |row|
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+                m = fmaxf(m, fabsf(pb.f[a][p]) +
+                                 cd * (fabsf(pb.f[3 + 3 * a][p]) + fabsf(pb.f[4 + 3 * a][p]) + fabsf(pb.f[5 + 3 * a][p])));
+            if (!(m <= 3.0e38f)) m = 3.0e38f;
+        });
+    wg_raise(m, bound, red);
+}
+
 // The P2G adjoint's particle part: each particle gathers the momentum cotangents s of the
 // nodes it deposited to (NodeMap as k_p2g_tiled's), with the deposit's weights and
-// offsets, and adds them to its v and row cotangents.
+// offsets, and adds them to its v and row cotangents. 1.6 M particles at 15 cm 310 -> 132 us
+// against reading the faces from global memory node by node.
+struct AdjFaces { const float* s[3]; };
 template <class NodeMap>
-__global__ __launch_bounds__(256) void k_p2g_adj_gather(PView ps, int64_t n, NodeMap map, float lo0, float lo1, float lo2,
-                                                        float dx, float dt, const float* __restrict__ s0,
-                                                        const float* __restrict__ s1, const float* __restrict__ s2, PB12 pb) {
-    int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    float xp = ps.f[0][p], yp = ps.f[1][p], zp = ps.f[2][p];
-    float wT = temporal(ps.f[15][p], dt);
-    const float* S[3] = {s0, s1, s2};
-    for (int a = 0; a < 3; ++a) {
-        float q0 = ispace(xp, lo0, dx, a == 0 ? 0.0f : 0.5f);
-        float q1 = ispace(yp, lo1, dx, a == 1 ? 0.0f : 0.5f);
-        float q2 = ispace(zp, lo2, dx, a == 2 ? 0.0f : 0.5f);
-        BSpline bx = bspline(q0), by = bspline(q1), bz = bspline(q2);
-        float v = 0.0f, c0 = 0.0f, c1 = 0.0f, c2 = 0.0f;
-        for (int mz = 0; mz < 3; ++mz) {
-            int K = node_at(bz.b, mz);
-            float wz = pick(bz, mz), d2 = ((float)K - q2) * dx;
-            for (int my = 0; my < 3; ++my) {
-                int J = node_at(by.b, my);
-                float wy = pick(by, my), d1 = ((float)J - q1) * dx;
-                for (int mx = 0; mx < 3; ++mx) {
-                    int I = node_at(bx.b, mx);
-                    int64_t idx = (int64_t)map.index(a, I, J, K);
-                    if (idx < 0) continue;
-                    float t = wT * pick(bx, mx) * wy * wz * S[a][idx];
-                    v += t;
-                    c0 += t * (((float)I - q0) * dx);
-                    c1 += t * d1;
-                    c2 += t * d2;
-                }
-            }
-        }
-        pb.f[a][p] += v;
-        pb.f[3 + 3 * a][p] += c0; pb.f[4 + 3 * a][p] += c1; pb.f[5 + 3 * a][p] += c2;
+__global__ __launch_bounds__(P2G_THREADS) void k_p2g_adj_gather(PView ps, int64_t n, NodeMap map, float lo0, float lo1, float lo2,
+                                                                float dx, float dt, AdjFaces S, PB12 pb) {
+    __shared__ float sval[G2P_BOX];
+    __shared__ alignas(16) int red[6 * (P2G_THREADS / 64)];
+    __shared__ int32_t stab[NodeMap::TAB];
+    const int64_t p = (int64_t)xcd_tile(blockIdx.x, gridDim.x) * P2G_THREADS + threadIdx.x;
+    const bool live = p < n;
+    float qo[3] = {0.0f, 0.0f, 0.0f}, wT = 0.0f;
+    if (live) {
+        qo[0] = ispace(ps.f[0][p], lo0, dx, 0.0f);
+        qo[1] = ispace(ps.f[1][p], lo1, dx, 0.0f);
+        qo[2] = ispace(ps.f[2][p], lo2, dx, 0.0f);
+        wT = temporal(ps.f[15][p], dt);
     }
+    over_boxes<G2P_BOX>(
+        live, wT == wT, qo, map, red, stab,
+        [&](auto axis, int k, auto idx) {   // (0 where there is no node: its terms vanish, unless wT is NaN)
+            constexpr int a = decltype(axis)::value;
+            sval[k] = idx >= 0 ? S.s[a][idx] : 0.0f;
+        },
+        [&](auto axis, int k0, int ex, int exy, const BSpline& bx, const BSpline& by, const BSpline& bz, float q0, float q1,
+            float q2) {
+            constexpr int a = decltype(axis)::value;
+            const float wx[3] = {bx.w0, bx.w1, bx.w2}, wy[3] = {by.w0, by.w1, by.w2}, wz[3] = {bz.w0, bz.w1, bz.w2};
+            float d0[3], d1[3], d2[3];
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+                d0[m] = ((float)(bx.b + m) - q0) * dx;
+                d1[m] = ((float)(by.b + m) - q1) * dx;
+                d2[m] = ((float)(bz.b + m) - q2) * dx;
+            }
+            float v = 0.0f, c0 = 0.0f, c1 = 0.0f, c2 = 0.0f;
+#pragma unroll
+            for (int mz = 0; mz < 3; ++mz)
+#pragma unroll
+                for (int my = 0; my < 3; ++my)
+#pragma unroll
+                    for (int mx = 0; mx < 3; ++mx) {
+                        const float t = (((wT * wx[mx]) * wy[my]) * wz[mz]) * sval[k0 + mx + ex * my + exy * mz];
+                        v += t;
+                        c0 += t * d0[mx];
+                        c1 += t * d1[my];
+                        c2 += t * d2[mz];
+                    }
+            pb.f[a][p] += v;
+            pb.f[3 + 3 * a][p] += c0; pb.f[4 + 3 * a][p] += c1; pb.f[5 + 3 * a][p] += c2;
+        },
+        [&](auto axis, const BSpline& bx, const BSpline& by, const BSpline& bz, float q0, float q1, float q2) {
+            constexpr int a = decltype(axis)::value;
+            const float x0 = bx.w0, x1 = bx.w1, x2 = bx.w2, y0 = by.w0, y1 = by.w1, y2 = by.w2, z0 = bz.w0, z1 = bz.w1, z2 = bz.w2;
+            float v = 0.0f, c0 = 0.0f, c1 = 0.0f, c2 = 0.0f;
+#pragma unroll 1
+            for (int q = 0; q < 27; ++q) {
+                const int mx = q % 3, my = (q / 3) % 3, mz = q / 9;
+                const int I = node_at(bx.b, mx), J = node_at(by.b, my), K = node_at(bz.b, mz);
+                const auto idx = map.index(a, I, J, K);
+                if (idx < 0) continue;
+                const float t = wT * (mx == 0 ? x0 : (mx == 1 ? x1 : x2)) * (my == 0 ? y0 : (my == 1 ? y1 : y2)) *
+                                (mz == 0 ? z0 : (mz == 1 ? z1 : z2)) * S.s[a][idx];
+                v += t;
+                c0 += t * (((float)I - q0) * dx);
+                c1 += t * (((float)J - q1) * dx);
+                c2 += t * (((float)K - q2) * dx);
+            }
+            pb.f[a][p] += v;
+            pb.f[3 + 3 * a][p] += c0; pb.f[4 + 3 * a][p] += c1; pb.f[5 + 3 * a][p] += c2;
+        },
+        [] {});
 }
 
 }  // namespace mael

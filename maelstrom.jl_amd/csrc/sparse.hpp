@@ -341,27 +341,6 @@ __device__ inline void finegather(const STopo& t, const V* __restrict__ u, int a
     float c = __fdiv_rn(4.0f, g.dx * g.dx);
     a0 *= c; a1 *= c; a2 *= c;
 }
-template <class V>
-__device__ inline float finegather_value(const STopo& t, const V* __restrict__ u, int a, float px, float py, float pz) {
-    const SGrid& g = t.g;
-    float q0 = ispace(px, g.lo[0], g.dx, a == 0 ? 0.0f : 0.5f);
-    float q1 = ispace(py, g.lo[1], g.dx, a == 1 ? 0.0f : 0.5f);
-    float q2 = ispace(pz, g.lo[2], g.dx, a == 2 ? 0.0f : 0.5f);
-    BSpline bx = bspline(q0), by = bspline(q1), bz = bspline(q2);
-    float vel = 0.0f;
-#pragma unroll
-    for (int mz = 0; mz < 3; ++mz)
-#pragma unroll
-        for (int my = 0; my < 3; ++my)
-#pragma unroll
-            for (int mx = 0; mx < 3; ++mx) {
-                int32_t idx = finefaceat(t, a, bx.b + mx, by.b + my, bz.b + mz);
-                float wgt = pick(bx, mx) * pick(by, my) * pick(bz, mz);
-                if (idx >= 0) vel += wgt * (float)u[idx];
-            }
-    return vel;
-}
-
 // Whether no point of the box of block w's cells widened by two cells is solid (the fluid
 // region, inside the wall's cylinder and above the floor, is convex: its eight corners
 // decide, and the margin covers the rounding of any cell centre or face position in it).

@@ -19,60 +19,6 @@ namespace mael {
 __global__ void k_adj_fromfix(float* __restrict__ ub, const unsigned long long* __restrict__ acc, size_t n, double inv);
 __global__ void k_g2p_adj_post(PB12 pb, const uint8_t* __restrict__ reached, int64_t n);
 
-// The flag sum of G2P's gather at (px, py, pz) for component a: the terms of
-// gather_component in its order, so the same bits as the forward's test.
-__device__ inline float flaggather(const STopo& t, const uint8_t* __restrict__ F, int a, float px, float py, float pz) {
-    const SGrid& g = t.g;
-    float q0 = ispace(px, g.lo[0], g.dx, a == 0 ? 0.0f : 0.5f);
-    float q1 = ispace(py, g.lo[1], g.dx, a == 1 ? 0.0f : 0.5f);
-    float q2 = ispace(pz, g.lo[2], g.dx, a == 2 ? 0.0f : 0.5f);
-    BSpline bx = bspline(q0), by = bspline(q1), bz = bspline(q2);
-    float flag = 0.0f;
-    for (int mz = 0; mz < 3; ++mz) {
-        float wz = pick(bz, mz);
-        for (int my = 0; my < 3; ++my) {
-            float wy = pick(by, my);
-            for (int mx = 0; mx < 3; ++mx) {
-                int32_t idx = finefaceat(t, a, bx.b + mx, by.b + my, bz.b + mz);
-                if (idx >= 0) {
-                    float wgt = pick(bx, mx) * wy * wz;
-                    flag += wgt * (float)F[idx];
-                }
-            }
-        }
-    }
-    return flag;
-}
-
-// Which particles took the grid's velocity in G2P (all three flag sums > 0.999,
-// flip.jl:1239), and the largest contribution one of them makes to a node, as float bits.
-__global__ __launch_bounds__(256) void k_sg2p_adj_reached(PView ps, int64_t n, STopo t, const uint8_t* __restrict__ fu,
-                                                          const uint8_t* __restrict__ fv, const uint8_t* __restrict__ fw,
-                                                          uint8_t* __restrict__ reached, PB12 pb, int* __restrict__ bound) {
-    __shared__ int red[4];
-    int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    float m = 0.0f;
-    if (p < n) {
-        float xp = ps.f[0][p], yp = ps.f[1][p], zp = ps.f[2][p];
-        bool k = flaggather(t, fu, 0, xp, yp, zp) > 0.999f && flaggather(t, fv, 1, xp, yp, zp) > 0.999f &&
-                 flaggather(t, fw, 2, xp, yp, zp) > 0.999f;
-        reached[p] = k ? 1 : 0;
-        if (k) {
-            float cd = 6.0f / t.g.dx;   // |row . d| <= (4 / dx^2)(1.5 dx) sum |row|
-            for (int a = 0; a < 3; ++a) {
-                float c = fabsf(pb.f[a][p]) + cd * (fabsf(pb.f[3 + 3 * a][p]) + fabsf(pb.f[4 + 3 * a][p]) + fabsf(pb.f[5 + 3 * a][p]));
-                m = fmaxf(m, c);
-            }
-            if (!(m <= 3.0e38f)) m = 3.0e38f;
-        }
-    }
-    int v = __float_as_int(m);   // non-negative: integer order is float order
-    for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) atomicMax(bound, max(max(red[0], red[1]), max(red[2], red[3])));
-}
-
 // The transpose of k_restrictfaces (sflip.jl:604-612) on cotangents: a coarse face
 // restricted from the 16 fine faces under it (the same faces, found the same way) passes
 // a sixteenth of its cotangent to each of them and keeps none (cout = 0); any other coarse
@@ -206,8 +152,9 @@ void SparseBasin::g2p_adjoint(float dt) {
     for (int f = 0; f < 12; ++f) P.f[f] = pb[f].p;
     int* bound = (int*)partials.p;
     fill_async(bound, (size_t)1, 0, s);
-    hipLaunchKernelGGL(k_sg2p_adj_reached, dim3(cdiv(n, 256)), dim3(256), 0, s, view(cur), n, t, fl[0].fine.p, fl[1].fine.p,
-                       fl[2].fine.p, reached.p, P, bound);
+    const G2PFaces Fl{{nullptr, nullptr, nullptr}, {fl[0].fine.p, fl[1].fine.p, fl[2].fine.p}};
+    hipLaunchKernelGGL(k_g2p_adj_reached<SparseNodes>, dim3(cdiv(n, P2G_THREADS)), dim3(P2G_THREADS), 0, s, view(cur), n,
+                       SparseNodes{t}, g.lo[0], g.lo[1], g.lo[2], g.dx, Fl, reached.p, P, bound);
     MAEL_HIP(hipMemcpyAsync(st.pinned, bound, sizeof(int), hipMemcpyDeviceToHost, s));
     st.sync();
     float m;
@@ -252,8 +199,8 @@ void SparseBasin::p2g_adjoint(float dt) {
     if (n > 0) {
         PB12 P;
         for (int f = 0; f < 12; ++f) P.f[f] = pb[f].p;
-        hipLaunchKernelGGL(k_p2g_adj_gather<SparseNodes>, dim3(cdiv(n, 256)), dim3(256), 0, s, view(cur), n, SparseNodes{t},
-                           g.lo[0], g.lo[1], g.lo[2], g.dx, dt, sm[0], sm[1], sm[2], P);
+        hipLaunchKernelGGL(k_p2g_adj_gather<SparseNodes>, dim3(cdiv(n, P2G_THREADS)), dim3(P2G_THREADS), 0, s, view(cur), n,
+                           SparseNodes{t}, g.lo[0], g.lo[1], g.lo[2], g.dx, dt, AdjFaces{{sm[0], sm[1], sm[2]}}, P);
     }
     MAEL_LAUNCH_CHECK();
 }

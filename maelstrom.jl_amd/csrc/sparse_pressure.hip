@@ -1702,20 +1702,25 @@ __device__ inline int32_t cellref(const STopo& t, int I, int J, int K, size_t& c
 }
 // The largest |cotangent| over the allocated fine face copies and the coarse faces, as
 // float bits (+inf for a nonfinite one).
+// (An atomic only from a workgroup that raises the bound: one from each of 17,000 workgroups
+// on the one address made it 54 us a launch for 4.4 M faces.)
 __global__ __launch_bounds__(256) void k_sadj_absmax(const float* __restrict__ x, size_t n, const int4* __restrict__ where,
                                                      int* __restrict__ bound) {
     __shared__ int red[4];
-    size_t l = (size_t)blockIdx.x * 256 + threadIdx.x;
     float m = 0.0f;
-    if (l < n && (!where || where[l / SBFACES].x >= 0)) {
-        float v = x[l];
-        m = isfinite(v) ? fabsf(v) : __int_as_float(0x7f800000);
-    }
+    for (size_t l = (size_t)blockIdx.x * 256 + threadIdx.x; l < n; l += (size_t)gridDim.x * 256)
+        if (!where || where[l / SBFACES].x >= 0) {
+            const float v = x[l];
+            m = fmaxf(m, isfinite(v) ? fabsf(v) : __int_as_float(0x7f800000));
+        }
     int v = __float_as_int(m);
     for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
-    if (threadIdx.x == 0) atomicMax(bound, max(max(red[0], red[1]), max(red[2], red[3])));
+    if (threadIdx.x == 0) {
+        const int w = max(max(red[0], red[1]), max(red[2], red[3]));
+        if (w > __hip_atomic_load(bound, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(bound, w);
+    }
 }
 // -G^T ub, scaled into fixed-point sums: each valid fine face copy (k_projectfine's test)
 // adds -ub dDl/dP / d to the cells whose pressures it differences (a fine cell, or the
@@ -2657,8 +2662,9 @@ void SparseBasin::project_adjoint(const SparseOpts& o, SparseStats& stats) {
     int* bound = (int*)partials.p;
     fill_async(bound, (size_t)1, 0, s);
     for (int a = 0; a < 3; ++a) {
-        if (F) hipLaunchKernelGGL(k_sadj_absmax, dim3(cdiv(F, 256)), dim3(256), 0, s, ub[a].fine.p, F, where.p, bound);
-        hipLaunchKernelGGL(k_sadj_absmax, dim3(cdiv(nfaces(a), 256)), dim3(256), 0, s, ub[a].coarse.p, nfaces(a),
+        auto groups = [](size_t m) { return dim3(std::min<unsigned>(cdiv(m, 256), 2048)); };
+        if (F) hipLaunchKernelGGL(k_sadj_absmax, groups(F), dim3(256), 0, s, ub[a].fine.p, F, where.p, bound);
+        hipLaunchKernelGGL(k_sadj_absmax, groups(nfaces(a)), dim3(256), 0, s, ub[a].coarse.p, nfaces(a),
                            (const int4*)nullptr, bound);
     }
     MAEL_HIP(hipMemcpyAsync(st.pinned, bound, sizeof(int), hipMemcpyDeviceToHost, s));

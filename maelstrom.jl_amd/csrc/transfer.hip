@@ -116,34 +116,6 @@ void DenseBasin::p2g(float dt) {
     MAEL_LAUNCH_CHECK();
 }
 
-// The value part of the gather, for the flags (flip.jl:401-405 `gathered`).
-template <class V>
-__device__ inline float gather_value(const V* __restrict__ u, int n1, int n2, int n3, const DGrid& g, int a, float px,
-                                     float py, float pz) {
-    float q0 = ispace(px, g.lo[0], g.dx, a == 0 ? 0.0f : 0.5f);
-    float q1 = ispace(py, g.lo[1], g.dx, a == 1 ? 0.0f : 0.5f);
-    float q2 = ispace(pz, g.lo[2], g.dx, a == 2 ? 0.0f : 0.5f);
-    BSpline bx = bspline(q0), by = bspline(q1), bz = bspline(q2);
-    float vel = 0.0f;
-    size_t s1 = (size_t)n1, s2 = (size_t)n1 * n2;
-#pragma unroll
-    for (int mz = 0; mz < 3; ++mz) {
-        int k = min(max(bz.b + mz, 0), n3 - 1);
-        float wz = pick(bz, mz);
-#pragma unroll
-        for (int my = 0; my < 3; ++my) {
-            int j = min(max(by.b + my, 0), n2 - 1);
-            float wy = pick(by, my);
-#pragma unroll
-            for (int mx = 0; mx < 3; ++mx) {
-                int i = min(max(bx.b + mx, 0), n1 - 1);
-                vel += pick(bx, mx) * wy * wz * (float)u[(size_t)i + s1 * j + s2 * k];
-            }
-        }
-    }
-    return vel;
-}
-
 // The gather's face nodes: indices clamped to the array (flip.jl:1210-1224).
 struct DenseClampNodes {
     static constexpr bool HOLES = false;
@@ -181,36 +153,6 @@ namespace mael {
 // a deposit (the tiled fixed-point scatter, so it is deterministic), the P2G adjoint a
 // gather.
 
-// Which particles took the grid's velocity in G2P (the flags' gathers, as k_dense_g2p),
-// and the largest contribution one of them makes to a node, as float bits (for the scale).
-__global__ __launch_bounds__(256) void k_g2p_adj_reached(PView ps, int64_t n, DGrid g, const uint8_t* __restrict__ fu,
-                                                         const uint8_t* __restrict__ fv, const uint8_t* __restrict__ fw,
-                                                         uint8_t* __restrict__ reached, PB12 pb, int* __restrict__ bound) {
-    __shared__ int red[4];
-    int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    float m = 0.0f;
-    if (p < n) {
-        float xp = ps.f[0][p], yp = ps.f[1][p], zp = ps.f[2][p];
-        int n1 = g.n[0], n2 = g.n[1], n3 = g.n[2];
-        bool k = gather_value(fu, n1 + 1, n2, n3, g, 0, xp, yp, zp) > 0.999f &&
-                 gather_value(fv, n1, n2 + 1, n3, g, 1, xp, yp, zp) > 0.999f &&
-                 gather_value(fw, n1, n2, n3 + 1, g, 2, xp, yp, zp) > 0.999f;
-        reached[p] = k ? 1 : 0;
-        if (k) {
-            float cd = 6.0f / g.dx;   // |row . d| <= (4 / dx^2)(1.5 dx) sum |row|
-            for (int a = 0; a < 3; ++a) {
-                float c = fabsf(pb.f[a][p]) + cd * (fabsf(pb.f[3 + 3 * a][p]) + fabsf(pb.f[4 + 3 * a][p]) + fabsf(pb.f[5 + 3 * a][p]));
-                m = fmaxf(m, c);
-            }
-            if (!(m <= 3.0e38f)) m = 3.0e38f;
-        }
-    }
-    int v = __float_as_int(m);   // non-negative: integer order is float order
-    for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) atomicMax(bound, max(max(red[0], red[1]), max(red[2], red[3])));
-}
 // u-bar = the accumulated deposit / scale.
 __global__ void k_adj_fromfix(float* __restrict__ ub, const unsigned long long* __restrict__ acc, size_t n, double inv) {
     size_t l = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -257,8 +199,9 @@ void DenseBasin::g2p_adjoint(float dt) {
     for (int f = 0; f < 12; ++f) P.f[f] = pb[f].p;
     int* bound = (int*)partials.p;
     fill_async(bound, (size_t)1, 0, s);
-    hipLaunchKernelGGL(k_g2p_adj_reached, dim3(cdiv(n, 256)), dim3(256), 0, s, view(cur), n, g, flag[0].p, flag[1].p,
-                       flag[2].p, reached.p, P, bound);
+    const G2PFaces F{{nullptr, nullptr, nullptr}, {flag[0].p, flag[1].p, flag[2].p}};
+    hipLaunchKernelGGL(k_g2p_adj_reached<DenseClampNodes>, dim3(cdiv(n, P2G_THREADS)), dim3(P2G_THREADS), 0, s, view(cur), n,
+                       DenseClampNodes{{g.n[0], g.n[1], g.n[2]}}, g.lo[0], g.lo[1], g.lo[2], g.dx, F, reached.p, P, bound);
     int bits = 0;
     MAEL_HIP(hipMemcpyAsync(st.pinned, bound, sizeof(int), hipMemcpyDeviceToHost, s));
     st.sync();
@@ -329,8 +272,9 @@ void DenseBasin::p2g_adjoint(float dt) {
     if (n > 0) {
         PB12 P;
         for (int f = 0; f < 12; ++f) P.f[f] = pb[f].p;
-        hipLaunchKernelGGL(k_p2g_adj_gather<DenseNodes>, dim3(cdiv(n, 256)), dim3(256), 0, s, view(cur), n,
-                           DenseNodes{{g.n[0], g.n[1], g.n[2]}}, g.lo[0], g.lo[1], g.lo[2], g.dx, dt, sf[0], sf[1], sf[2], P);
+        hipLaunchKernelGGL(k_p2g_adj_gather<DenseNodes>, dim3(cdiv(n, P2G_THREADS)), dim3(P2G_THREADS), 0, s, view(cur), n,
+                           DenseNodes{{g.n[0], g.n[1], g.n[2]}}, g.lo[0], g.lo[1], g.lo[2], g.dx, dt,
+                           AdjFaces{{sf[0], sf[1], sf[2]}}, P);
     }
     MAEL_LAUNCH_CHECK();
 }

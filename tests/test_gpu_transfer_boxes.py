@@ -61,3 +61,44 @@ def test_boxes(mael, orc, ctx, n, places, off):
     ref = orc.dense_g2p(g, sub, int(keep.sum()), u, v, w, *flags, dt, 9.81)
     for f in VN + tuple("C%d" % k for k in range(9)):
         assert np.array_equal(s.get(f)[keep].view(np.uint32), ref[f].view(np.uint32)), f
+
+
+# A particle's part of the adjoints does not depend on its workgroup's other particles: in
+# shuffled order (up to 200 clusters a workgroup, most left to the direct path) it has the
+# same bits as in the clusters' order, and so has the cotangent of the faces (whole numbers).
+@pytest.mark.parametrize("n,places,off", [(1, 1, 0), (257, 7, 1), (1000, 7, 0), (1000, 200, 3)])
+def test_adjoint_boxes(mael, orc, ctx, n, places, off):
+    print("case: adjoint boxes n=%d places=%d" % (n, places), flush=True)
+    b = mael.Basin(radius=18.0, depth=12.0, Γ=225.0, core=2.5)
+    s = mael.FlipBasin(b, dx=0.6, capacity=2000)
+    g = orc.dense_scene(18.0, 12.0, 3.0, 0.6, 225.0, 2.5)[0]
+    rng = np.random.default_rng(n + places)
+    ps = _particles(rng, g, n, places)
+    if off:
+        ps["PX"][n // 2] = np.float32(g.lo[0] - 30.0)
+        if off > 1:
+            ps["PY"][n // 3], ps["PZ"][n // 5] = np.float32(1e9), np.float32(np.inf)
+    names = VN + tuple("C%d" % k for k in range(9))
+    pbar = {f: rng.normal(0, 1, n).astype(np.float32) for f in names}
+    flags = {"F" + c: (rng.random(s.shape(c)) > 0.002).astype(np.uint8) for c in "UVW"}
+    ubar = {"UB_" + c: rng.normal(0, 1, s.shape(c)).astype(np.float32) for c in "UVW"}
+    dt, got = 0.04, []
+    for order in (np.arange(n), rng.permutation(n)):
+        s.set_particles({f: a[order] for f, a in ps.items()}, n)
+        for f, a in flags.items():
+            s.set(f, a)
+        for f, a in pbar.items():
+            s.set("PB_" + f, a[order])
+        mael.grid2particles_adjoint(s, dt)
+        back = np.argsort(order)
+        out = [s.get("PB_" + f)[back] for f in names] + [s.get("UB_" + c) for c in "UVW"]
+        s.set("PHI", np.zeros(s.shape("PHI"), np.float32))   # every face in the band
+        for f, a in ubar.items():
+            s.set(f, a)
+        for f in names:
+            s.set("PB_" + f, np.zeros(n, np.float32))
+        mael.particles2grid_adjoint(s, dt)
+        got.append(out + [s.get("PB_" + f)[back] for f in names])
+    assert any(a.any() for a in got[0][-12:])
+    for a, b in zip(*got):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
