@@ -559,18 +559,36 @@ template <class C> struct CompT {
     const C* dgf = nullptr; // FP32, level 0: the full diagonal per fine cell (mode 6)
 };
 
-// Flexible CG's fused step (mode 4 of the level-0 rows, sflip.jl:1884-1886 with
-// 1903): the new direction d = z + beta d_old (x is z) is applied and written, and
-// d.q is summed per workgroup over the unknowns.
-struct SearchArgs {
-    const float* dof;   // d_old, fine pool and coarse grid
-    const float* doc;
-    float* dnf;         // d_new
-    float* dnc;
-    double* partials;   // [4 nslots fine quarter tiles | coarse workgroups]
-    int32_t coarse0;    // where the coarse workgroups' sums start
-    const double* scal;
+// What the fused passes of the composite rows take besides x and b.
+template <class T> struct RowArgs {
+    // mode 4, flexible CG's fused step (sflip.jl:1884-1886 with 1903): the new direction
+    // d = z + beta d_old (x is z, or z / scal[zslot] in reduced precision) is applied and
+    // written, and d.q is summed per workgroup over the unknowns
+    const float* dof = nullptr;   // d_old, fine pool and coarse grid
+    const float* doc = nullptr;
+    float* dnf = nullptr;         // d_new
+    float* dnc = nullptr;
+    double* partials = nullptr;   // [4 nslots fine quarter tiles | coarse workgroups]
+    int32_t coarse0 = 0;          // where the coarse workgroups' sums start
+    const double* scal = nullptr;
+    int zslot = -1;
+    // mode 8: x is prolonged on the way in, x + boost y of the coarser level (its fine
+    // part, or the first dense level, and its coarse part)
+    const T* yf = nullptr;
+    const T* yc = nullptr;
+    float boost = 0.0f;
+    // mode 10: the right-hand side in FP32 and its reduced-precision copy (r / scal[zslot])
+    // that the pass writes, coarse part
+    const float* rc = nullptr;
+    T* bc = nullptr;
 };
+// k_convert's scale: scal[slot], or its inverse; 1 where that is no use
+__device__ inline float slot_scale(const double* __restrict__ scal, int slot, bool invert) {
+    float c = 1.0f;
+    if (slot >= 0) c = invert ? (float)(1.0 / scal[slot]) : (float)scal[slot];
+    if (!(c == c) || c == 0.0f || !(fabsf(c) <= 3.0e38f)) c = 1.0f;
+    return c;
+}
 
 // sflip.jl:1218-1269 on the fine cells of a level: mode 0 Jacobi (out = x + w (b - A x) /
 // diag), 1 residual (out = b - A x), 2 apply (out = A x), 3 Jacobi from x = 0 (x not
@@ -580,6 +598,14 @@ struct SearchArgs {
 // neighbours' couplings, only their products with x (the weights round to the storage
 // type once per solve; the FP32 sweep keeps the reference's division). That sweep relaxes
 // the operator with diagonal w / r, and the reduced-precision residual uses the same.
+//
+// A level-0 pass is bound by HBM (9 B a cell for a reduced-precision sweep, 43 us for
+// 4,200 slots), so two passes take in the one beside them: mode 7 is the residual
+// restricted to the next level in the workgroup (its 2 B are neither written nor read
+// back), mode 8 the first sweep after the prolongation, with x prolonged as it is loaded.
+// In FP16 there: 59 -> 46 and 74 -> 50 us. (The first two sweeps from zero in one
+// pass, the first made for the halo too, took 98 us, 13 more than the two: what a neighbour
+// slot's side costs is whole lines of every array it needs.)
 // Level 0, matrix-free and staged in LDS. A workgroup takes a quarter of a slot (4 z
 // planes of its 16^3 block), a thread 4 consecutive cells along x of one row. Level 0's
 // coupling of a LIQUID fine cell to a neighbour is 1 when the neighbour is a LIQUID fine
@@ -613,15 +639,17 @@ template <class T> __device__ inline void store4_nt(T* __restrict__ p, uint32_t 
 constexpr int RS = 24, PS = 18 * RS;   // LDS rows of 24: cell li (-1..16) at 4 + li; planes of 18 rows
 // NQ: quads a thread (a workgroup takes 4 NQ planes of its slot, its 16 / (4 NQ) tiles
 // cover the slot); more cells a workgroup keep more loads in flight.
-template <int MODE, class T, class C, int NQ = 1>
-__device__ __forceinline__ void rowfine16_wg(const uint32_t tile, T* __restrict__ out, const T* __restrict__ x,
-                                             const T* __restrict__ b, const T* __restrict__ xc, const CompT<C>& L,
-                                             const STopo& t, const SearchArgs& S) {
+template <int MODE, class T, class C, int NQ = 1, class X = T>
+__device__ __forceinline__ void rowfine16_wg(const uint32_t tile, T* __restrict__ out, const X* __restrict__ x,
+                                             const T* __restrict__ b, const X* __restrict__ xc, const CompT<C>& L,
+                                             const STopo& t, const RowArgs<T>& S) {
     constexpr bool Z = MODE == 3 || MODE == 5 || MODE == 6, SEARCH = MODE == 4;
+    constexpr bool RESTRICT = MODE == 7, PROLONG = MODE == 8;
+    constexpr bool JACOBI = MODE == 0 || PROLONG, RESID = MODE == 1 || RESTRICT;
     // reduced precision: the sweep and the residual take the weight r = omega / diag
-    constexpr bool RW = (MODE == 0 || MODE == 1) && !std::is_same<T, float>::value;
+    constexpr bool RW = (JACOBI || RESID) && !std::is_same<T, float>::value;
     // FP32: the rows take the full diagonal computed once a solve (mode 6), the same sum
-    constexpr bool FD = MODE <= 4 && std::is_same<T, float>::value;
+    constexpr bool FD = MODE != 5 && MODE != 6 && std::is_same<T, float>::value;
     constexpr bool NW = !RW && !FD;                                        // the couplings staged
     constexpr int PL = 4 * NQ, HV = (PL + 2) * PS, TPS = 4 / NQ;          // planes, LDS, tiles a slot
     static_assert(NQ == 1 || NQ == 2, "a tile is 4 or 8 planes");
@@ -634,16 +662,51 @@ __device__ __forceinline__ void rowfine16_wg(const uint32_t tile, T* __restrict_
     const uint32_t cb = (uint32_t)(s - 1) * 4096u;
     const uint8_t* __restrict__ tf = L.actf;   // level 0: the fine cell types
     const float beta = SEARCH ? (float)S.scal[SS_BETA] : 0.0f;
+    // z's scale (where it is kept in reduced precision)
+    const float zs = SEARCH && !std::is_same<X, T>::value ? slot_scale(S.scal, S.zslot, false) : 1.0f;
+    auto zat = [&](X v) -> float {
+        if constexpr (std::is_same<X, T>::value) return lf(v);
+        else return lf(v) * zs;
+    };
     // x as the row reads it: in the fused search the direction z + beta d_old, rounded to T
-    auto xat = [&](const T* __restrict__ xs, const float* __restrict__ ds, size_t i) -> float {
-        if constexpr (SEARCH) return lf(sf<T>(lf(xs[i]) + beta * ds[i]));
+    auto xat = [&](const X* __restrict__ xs, const float* __restrict__ ds, size_t i) -> float {
+        if constexpr (SEARCH) return lf(sf<T>(zat(xs[i]) + beta * ds[i]));
         else return lf(xs[i]);
+    };
+    // level 1's cell over level 0's cell i
+    auto parent = [](uint32_t i) {
+        return (i >> 12) * 512u + ((i & 15u) >> 1) + 8u * (((i >> 4) & 15u) >> 1) + 64u * (((i >> 8) & 15u) >> 1);
+    };
+    auto prolonged = [&](float xv, T y) { return lf(sf<T>(xv + S.boost * lf(y))); };
+    // a cell of the halo
+    auto xfine = [&](uint32_t i) -> float {
+        if constexpr (PROLONG) return prolonged(lf(x[i]), S.yf[parent(i)]);
+        else return xat(x, S.dof, i);
+    };
+    // four of them along x from i (a multiple of 4)
+    auto xfine4 = [&](uint32_t i, float (&xv)[4]) {
+        const Four<X> x4 = load4(x, i);
+        if constexpr (SEARCH) {
+            const float4 d4 = *reinterpret_cast<const float4*>(S.dof + i);
+            const float dv[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) xv[e] = lf(sf<T>(zat(x4.v[e]) + beta * dv[e]));
+        } else if constexpr (PROLONG) {
+            const uint32_t par = parent(i);
+            const T y[2] = {S.yf[par], S.yf[par + 1]};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) xv[e] = prolonged(lf(x4.v[e]), y[e >> 1]);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) xv[e] = lf(x4.v[e]);
+        }
     };
     const int tid = threadIdx.x, i4 = tid & 3, j = (tid >> 2) & 15, kk = tid >> 6;
     // quad q of the thread: plane kk + 4 q of the tile
     auto cell = [&](int q) { return cb + 256u * (uint32_t)(k0 + kk + 4 * q) + 16u * (uint32_t)j + 4u * (uint32_t)i4; };
     int4 w = t.where[s - 1];
     if (w.x < 0) {
+        if constexpr (RESTRICT) return;   // no right-hand side on a free slot
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
             const uint32_t n = cell(q);
@@ -671,24 +734,22 @@ __device__ __forceinline__ void rowfine16_wg(const uint32_t tile, T* __restrict_
         const uint32_t n = cell(q);
         tq[q] = *reinterpret_cast<const uint32_t*>(tf + n);
         dq[q] = load4(RW ? L.rwf : (FD ? L.dgf : L.dDf), n);   // the Dirichlet part, the weight or the diagonal
-        if constexpr (MODE == 2 || MODE == 4 || MODE == 5 || MODE == 6) {
+        if constexpr (!JACOBI && !RESID && MODE != 3) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) bq[q].v[e] = sf<T>(0.0f);
         } else {
             bq[q] = load4(b, n);
         }
-        if constexpr (!Z) {
-            const Four<T> xq = load4(x, n);
-            if constexpr (SEARCH) {
-                const float4 dold = *reinterpret_cast<const float4*>(S.dof + n);
-                const float dv[4] = {dold.x, dold.y, dold.z, dold.w};
+        if constexpr (PROLONG) {
+            const Four<X> xq = load4(x, n);
+            const uint32_t par = parent(n);
+            const T y[2] = {S.yf[par], S.yf[par + 1]};
 #pragma unroll
-                for (int e = 0; e < 4; ++e) x0[q][e] = lf(sf<T>(lf(xq.v[e]) + beta * dv[e]));
-                *reinterpret_cast<float4*>(S.dnf + n) = make_float4(x0[q][0], x0[q][1], x0[q][2], x0[q][3]);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) x0[q][e] = lf(xq.v[e]);
-            }
+            for (int e = 0; e < 4; ++e)
+                x0[q][e] = ((tq[q] >> (8 * e)) & 0xffu) == LIQUID ? prolonged(lf(xq.v[e]), y[e >> 1]) : lf(xq.v[e]);
+        } else if constexpr (!Z) {
+            xfine4(n, x0[q]);
+            if constexpr (SEARCH) *reinterpret_cast<float4*>(S.dnf + n) = make_float4(x0[q][0], x0[q][1], x0[q][2], x0[q][3]);
         } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e) x0[q][e] = 0.0f;
@@ -713,7 +774,9 @@ __device__ __forceinline__ void rowfine16_wg(const uint32_t tile, T* __restrict_
         bool in = ci >= 0 && cj >= 0 && ck >= 0 && ci < n0 && cj < n1 && ck < n2;
         size_t cidx = cl(min(max(ci, 0), n0 - 1), min(max(cj, 0), n1 - 1), min(max(ck, 0), n2 - 1), n0, n1);
         wc = (in ? L.tc[cidx] : SOLID) == LIQUID ? FINE_COARSE : 0.0f;
-        float xv = Z ? 0.0f : xat(xc, S.doc, cidx);
+        float xv = 0.0f;
+        if constexpr (PROLONG) xv = prolonged(lf(xc[cidx]), S.yc[cidx]);   // (of use on LIQUID cells only)
+        else if constexpr (!Z) xv = xat(xc, S.doc, cidx);
         pc = wc > 0.0f ? wc * xv : 0.0f;
     };
     // 4 cells along x from li0 (a multiple of 4) at row lj, plane lk, in this slot or else
@@ -726,18 +789,7 @@ __device__ __forceinline__ void rowfine16_wg(const uint32_t tile, T* __restrict_
             uint32_t idx = (uint32_t)(sn - 1) * 4096u + (uint32_t)(li0 + 16 * ((lj & 15) + 16 * (lk & 15)));
             uint32_t ty = *reinterpret_cast<const uint32_t*>(tf + idx);
             float xv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-            if constexpr (!Z) {
-                const Four<T> x4 = load4(x, idx);
-                if constexpr (SEARCH) {
-                    const float4 d4 = *reinterpret_cast<const float4*>(S.dof + idx);
-                    const float dv[4] = {d4.x, d4.y, d4.z, d4.w};
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) xv[e] = lf(sf<T>(lf(x4.v[e]) + beta * dv[e]));
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) xv[e] = lf(x4.v[e]);
-                }
-            }
+            if constexpr (!Z) xfine4(idx, xv);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 wv[e] = ((ty >> (8 * e)) & 0xffu) == LIQUID ? FINE_FINE : 0.0f;
@@ -767,7 +819,8 @@ __device__ __forceinline__ void rowfine16_wg(const uint32_t tile, T* __restrict_
             if (sn != 0) {
                 uint32_t idx = (uint32_t)(sn - 1) * 4096u + (uint32_t)((li & 15) + 16 * (lj + 16 * lk));
                 wv = tf[idx] == LIQUID ? FINE_FINE : 0.0f;
-                float xv = Z ? 0.0f : xat(x, S.dof, idx);
+                float xv = 0.0f;
+                if constexpr (!Z) xv = xfine(idx);
                 pv = wv > 0.0f ? wv * xv : 0.0f;
             } else {
                 coarse(li, lj, lk, wv, pv);
@@ -784,6 +837,7 @@ __device__ __forceinline__ void rowfine16_wg(const uint32_t tile, T* __restrict_
     __syncthreads();
 
     double pq = 0.0;
+    Four<T> res4[RESTRICT ? NQ : 1];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
         const int hq = 4 + 4 * i4 + RS * (j + 1) + PS * (kk + 4 * q + 1);
@@ -822,7 +876,7 @@ __device__ __forceinline__ void rowfine16_wg(const uint32_t tile, T* __restrict_
             const bool act = MODE == 6 ? true : ((MODE == 2 || SEARCH) ? t0 == LIQUID : t0 != 0);
             float res = 0.0f;
             if (act) {
-                if constexpr (RW && MODE == 0) {
+                if constexpr (RW && JACOBI) {
                     const float rw = dd;   // omega / diag
                     res = rw > 0.0f ? (1.0f - OMEGA) * x0[q][e] + rw * (bb + off) : 0.0f;
                 } else if constexpr (RW) {   // the residual of the operator the weighted sweep relaxes
@@ -834,15 +888,35 @@ __device__ __forceinline__ void rowfine16_wg(const uint32_t tile, T* __restrict_
                     res = diag;
                 } else {
                     float ax = diag * x0[q][e] - off;
-                    if (MODE == 0 || MODE == 3) res = diag > 0.0f ? x0[q][e] + __fdiv_rn(OMEGA * (bb - ax), diag) : 0.0f;
-                    else if (MODE == 1) res = bb - ax;
+                    if (JACOBI || MODE == 3) res = diag > 0.0f ? x0[q][e] + __fdiv_rn(OMEGA * (bb - ax), diag) : 0.0f;
+                    else if (RESID) res = bb - ax;
                     else res = ax;
                 }
                 if constexpr (SEARCH) pq += (double)x0[q][e] * (double)res;
             }
             oq.v[e] = sf<T>(res);
         }
-        store4_nt(out, cell(q), oq);
+        if constexpr (RESTRICT) res4[q] = oq;
+        else store4_nt(out, cell(q), oq);
+    }
+    if constexpr (RESTRICT) {   // the sums of 2^3 of them, x fastest, from LDS
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+            sp4[64 * (kk + 4 * q) + 4 * j + i4] =
+                make_float4(lf(res4[q].v[0]), lf(res4[q].v[1]), lf(res4[q].v[2]), lf(res4[q].v[3]));
+        __syncthreads();
+        if (tid < 128 * NQ) {
+            const int ci = tid & 7, cj = (tid >> 3) & 7, ck = tid >> 6;
+            float acc = 0.0f;
+#pragma unroll
+            for (int cz = 0; cz < 2; ++cz)
+#pragma unroll
+                for (int by = 0; by < 2; ++by)
+#pragma unroll
+                    for (int ax = 0; ax < 2; ++ax) acc += sp[256 * (2 * ck + cz) + 16 * (2 * cj + by) + 2 * ci + ax];
+            out[(uint32_t)(s - 1) * 512u + (uint32_t)(ci + 8 * (cj + 8 * (k0 / 2 + ck)))] = sf<T>(acc);
+        }
     }
     if constexpr (SEARCH) {
         double sum = block_sum_red(pq, lds);
@@ -851,44 +925,20 @@ __device__ __forceinline__ void rowfine16_wg(const uint32_t tile, T* __restrict_
 }
 template <int MODE, class T, class C, int NQ = 1>
 __global__ __launch_bounds__(256) void k_rowfine16(T* __restrict__ out, const T* __restrict__ x, const T* __restrict__ b,
-                                                   const T* __restrict__ xc, CompT<C> L, STopo t, SearchArgs S) {
+                                                   const T* __restrict__ xc, CompT<C> L, STopo t, RowArgs<T> S) {
     rowfine16_wg<MODE, T, C, NQ>(xcd_tile(blockIdx.x, gridDim.x), out, x, b, xc, L, t, S);
-}
-
-// The reduced-precision level-0 Jacobi sweep from x = 0: out = r b with r = omega / diag
-// per cell (mode 5 of k_rowfine16), on non-solid cells; four cells a thread.
-template <class T>
-__global__ __launch_bounds__(256) void k_jacobi0w(T* __restrict__ out, const T* __restrict__ b, const T* __restrict__ rw,
-                                                  const uint8_t* __restrict__ tf, const int4* __restrict__ where, int32_t nf) {
-    const uint32_t n = 4u * (uint32_t)(xcd_tile(blockIdx.x, gridDim.x) * 256u + threadIdx.x);
-    if (n >= (uint32_t)nf) return;
-    Four<T> o;
-    if (where[n >> 12].x < 0) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o.v[e] = sf<T>(0.0f);
-    } else {
-        const uint32_t ty = *reinterpret_cast<const uint32_t*>(tf + n);
-        const Four<T> bq = load4(b, n), rq = load4(rw, n);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float r = lf(rq.v[e]);
-            o.v[e] = sf<T>(((ty >> (8 * e)) & 0xffu) != 0 && r > 0.0f ? r * lf(bq.v[e]) : 0.0f);
-        }
-    }
-    *reinterpret_cast<Four<T>*>(out + n) = o;
 }
 
 // The reduced-precision V-cycle's entry on level 0's fine part in one pass: b = r c in T
 // with k_convert's scale (c = 1 / scal[slot], 1 when slot < 0) and rounding, stored for
-// the rest of the V-cycle, and k_jacobi0w's sweep from zero on it.
+// the rest of the V-cycle, and the Jacobi sweep from x = 0 on it, out = b omega / diag
+// (mode 5 of k_rowfine16), on non-solid cells; four cells a thread.
 template <class T>
 __device__ __forceinline__ void jacobi0w_cvt_wg(const uint32_t tile, T* __restrict__ out, T* __restrict__ bh,
                                                 const float* __restrict__ r, const T* __restrict__ rw,
                                                 const uint8_t* __restrict__ tf, const int4* __restrict__ where,
                                                 int32_t nf, const double* __restrict__ scal, int slot) {
-    float c = 1.0f;
-    if (slot >= 0) c = (float)(1.0 / scal[slot]);
-    if (!(c == c) || c == 0.0f || !(fabsf(c) <= 3.0e38f)) c = 1.0f;
+    const float c = slot_scale(scal, slot, true);
     const uint32_t n = 4u * (tile * 256u + threadIdx.x);
     if (n >= (uint32_t)nf) return;
     const float4 rv = *reinterpret_cast<const float4*>(r + n);
@@ -914,19 +964,22 @@ __device__ __forceinline__ void jacobi0w_cvt_wg(const uint32_t tile, T* __restri
 
 // Level 1 (8^3 a slot), staged in LDS: a workgroup per slot stages x of the block and its
 // face layers (face neighbours' slots, else the coarse cells, clamped), then each thread
-// computes 2 cells with finerow's couplings and order.
+// computes 2 cells with finerow's couplings and order. Modes 7 and 8 as on level 0, to and
+// from the first dense level (the coarse grid's cells).
 template <int MODE, class T, class C>
 __device__ __forceinline__ void rowfine8_wg(const uint32_t tile, T* __restrict__ out, const T* __restrict__ x,
                                             const T* __restrict__ b, const T* __restrict__ xc, const CompT<C>& L,
-                                            const STopo& t) {
-    constexpr bool Z = MODE == 3;
+                                            const STopo& t, const RowArgs<T>& S) {
+    constexpr bool Z = MODE == 3, RESTRICT = MODE == 7, PROLONG = MODE == 8;
     constexpr int H8 = 10;
     __shared__ T sx[Z ? 1 : H8 * H8 * H8];
+    __shared__ T sr[RESTRICT ? 512 : 1];
     const int s = (int)tile + 1;
     const uint32_t cb = (uint32_t)(s - 1) * 512u, fb = (uint32_t)(s - 1) * 576u;
     int4 w = t.where[s - 1];
     if (w.x < 0) {
-        for (int c = threadIdx.x; c < 512; c += 256) out[cb + c] = sf<T>(0.0f);
+        if constexpr (!RESTRICT)
+            for (int c = threadIdx.x; c < 512; c += 256) out[cb + c] = sf<T>(0.0f);
         return;
     }
     if constexpr (!Z) {
@@ -934,21 +987,31 @@ __device__ __forceinline__ void rowfine8_wg(const uint32_t tile, T* __restrict__
 #pragma unroll
         for (int d = 0; d < 6; ++d) nb[d] = nbslot(t, w, d);
         const int n0 = t.g.nc(0), n1 = t.g.nc(1), n2 = t.g.nc(2);
+        // x at cell (li, lj, lk) of the slot's block and the layers round it, prolonged in mode 8
+        auto xat = [&](T v, int li, int lj, int lk) -> T {
+            if constexpr (!PROLONG) return v;
+            const int ci = (w.x * 8 + li) >> 1, cj = (w.y * 8 + lj) >> 1, ck = (w.z * 8 + lk) >> 1;
+            const T y = S.yc[cl(min(max(ci, 0), n0 - 1), min(max(cj, 0), n1 - 1), min(max(ck, 0), n2 - 1), n0, n1)];
+            return sf<T>(lf(v) + S.boost * lf(y));
+        };
         for (int c = threadIdx.x; c < 512; c += 256) {
             int i = c & 7, j = (c >> 3) & 7, k = c >> 6;
-            sx[(i + 1) + H8 * ((j + 1) + H8 * (k + 1))] = x[cb + c];
+            const T v = x[cb + c];
+            sx[(i + 1) + H8 * ((j + 1) + H8 * (k + 1))] = !PROLONG || L.actf[cb + c] != 0 ? xat(v, i, j, k) : v;
         }
         for (int e = threadIdx.x; e < 6 * 64; e += 256) {
             int d = e >> 6, p = e & 7, q = (e >> 3) & 7, ax = d >> 1, hi = d & 1;
             int li = ax == 0 ? (hi ? 8 : -1) : p, lj = ax == 1 ? (hi ? 8 : -1) : (ax == 0 ? p : q), lk = ax == 2 ? (hi ? 8 : -1) : q;
             int h = (li + 1) + H8 * ((lj + 1) + H8 * (lk + 1));
             int32_t sn = nb[d];
+            T v;
             if (sn != 0) {
-                sx[h] = x[(uint32_t)(sn - 1) * 512u + (uint32_t)((li & 7) + 8 * ((lj & 7) + 8 * (lk & 7)))];
+                v = x[(uint32_t)(sn - 1) * 512u + (uint32_t)((li & 7) + 8 * ((lj & 7) + 8 * (lk & 7)))];
             } else {
                 int ci = (w.x * 8 + li) >> 1, cj = (w.y * 8 + lj) >> 1, ck = (w.z * 8 + lk) >> 1;
-                sx[h] = xc[cl(min(max(ci, 0), n0 - 1), min(max(cj, 0), n1 - 1), min(max(ck, 0), n2 - 1), n0, n1)];
+                v = xc[cl(min(max(ci, 0), n0 - 1), min(max(cj, 0), n1 - 1), min(max(ck, 0), n2 - 1), n0, n1)];
             }
+            sx[h] = xat(v, li, lj, lk);   // (only active neighbours couple)
         }
         __syncthreads();
     }
@@ -972,25 +1035,39 @@ __device__ __forceinline__ void rowfine8_wg(const uint32_t tile, T* __restrict__
                 }
             float x0 = Z ? 0.0f : lf(sx[Z ? 0 : h]);
             float ax = diag * x0 - off;
-            if (MODE == 0 || MODE == 3) res = diag > 0.0f ? x0 + __fdiv_rn(OMEGA * (lf(b[n]) - ax), diag) : 0.0f;
-            else if (MODE == 1) res = lf(b[n]) - ax;
+            if (MODE == 0 || PROLONG || MODE == 3) res = diag > 0.0f ? x0 + __fdiv_rn(OMEGA * (lf(b[n]) - ax), diag) : 0.0f;
+            else if (MODE == 1 || RESTRICT) res = lf(b[n]) - ax;
             else res = ax;
         }
-        out[n] = sf<T>(res);
+        if constexpr (RESTRICT) sr[c] = sf<T>(res);
+        else out[n] = sf<T>(res);
+    }
+    if constexpr (RESTRICT) {
+        __syncthreads();
+        if (threadIdx.x < 64) {   // (a fine block's coarse cells are all on the grid)
+            const int ci = threadIdx.x & 3, cj = (threadIdx.x >> 2) & 3, ck = threadIdx.x >> 4;
+            float acc = 0.0f;
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+#pragma unroll
+                for (int bb = 0; bb < 2; ++bb)
+#pragma unroll
+                    for (int a = 0; a < 2; ++a) acc += lf(sr[64 * (2 * ck + c) + 8 * (2 * cj + bb) + 2 * ci + a]);
+            out[cl(w.x * 4 + ci, w.y * 4 + cj, w.z * 4 + ck, t.g.nc(0), t.g.nc(1))] = sf<T>(acc);
+        }
     }
 }
-template <int MODE, class T, class C>
-__global__ __launch_bounds__(256) void k_rowfine8(T* __restrict__ out, const T* __restrict__ x, const T* __restrict__ b,
-                                                  const T* __restrict__ xc, CompT<C> L, STopo t) {
-    rowfine8_wg<MODE, T, C>(xcd_tile(blockIdx.x, gridDim.x), out, x, b, xc, L, t);
-}
-
 // Coarse cells 256 cb .. 256 cb + 255; the search's partial sum goes to slot `ps`.
-template <int N, int MODE, class T, class C>
+// Mode 10 is mode 3 with the right-hand side converted on the way in (reduced precision),
+// modes 7 and 8 the coarse rows of the fused passes: the residual (on level 1 into the
+// first dense level, whose covered cells the fine part restricts to) and the sweep on x
+// prolonged.
+template <int N, int MODE, class T, class C, class X = T>
 __device__ __forceinline__ void rowcoarse_wg(const uint32_t cb, const uint32_t ps, T* __restrict__ out,
-                                             const T* __restrict__ x, const T* __restrict__ b, const T* __restrict__ xf,
-                                             const CompT<C>& L, const STopo& t, const SearchArgs& S) {
-    constexpr bool SEARCH = MODE == 4;
+                                             const X* __restrict__ x, const T* __restrict__ b, const X* __restrict__ xf,
+                                             const CompT<C>& L, const STopo& t, const RowArgs<T>& S) {
+    constexpr bool SEARCH = MODE == 4, PROLONG = MODE == 8, Z = MODE == 3 || MODE == 10;
+    constexpr bool JACOBI = MODE == 0 || PROLONG || Z, RESID = MODE == 1 || MODE == 7;
     __shared__ double lds[4];
     int n0 = t.g.nc(0), n1 = t.g.nc(1), n2 = t.g.nc(2);
     size_t l = (size_t)cb * 256u + threadIdx.x;
@@ -1007,19 +1084,40 @@ __device__ __forceinline__ void rowcoarse_wg(const uint32_t cb, const uint32_t p
     const bool row = L.actc[l] != 0 && !(msk & 1u);
     const LevelTypes ty{L.actf, L.tc};   // level 0 (N = 16): the couplings from the types
     const LevelTypes* typ = N == 16 ? &ty : nullptr;
+    const float zs = SEARCH && !std::is_same<X, T>::value ? slot_scale(S.scal, S.zslot, false) : 1.0f;
+    const float rs = MODE == 10 ? slot_scale(S.scal, S.zslot, true) : 1.0f;
+    auto zat = [&](X v) -> float {
+        if constexpr (std::is_same<X, T>::value) return lf(v);
+        else return lf(v) * zs;
+    };
+    auto prolonged = [&](float xv, T y) { return lf(sf<T>(xv + S.boost * lf(y))); };
     auto fx = [&](uint32_t i) -> float {
-        if constexpr (SEARCH) return lf(xf[i]) + beta * S.dof[i];
-        else if constexpr (MODE == 3) return 0.0f;
-        else return lf(xf[i]);
+        if constexpr (SEARCH) return zat(xf[i]) + beta * S.dof[i];
+        else if constexpr (Z) return 0.0f;
+        else if constexpr (PROLONG && N == 16) {
+            return prolonged(lf(xf[i]), S.yf[(i >> 12) * 512u + ((i & 15u) >> 1) + 8u * (((i >> 4) & 15u) >> 1) +
+                                             64u * (((i >> 8) & 15u) >> 1)]);
+        } else if constexpr (PROLONG) {   // level 1: the dense level's cell over this one
+            const int4 w = t.where[i >> 9];
+            const int c = (int)(i & 511u);
+            return prolonged(lf(xf[i]), S.yc[cl((w.x * 8 + (c & 7)) >> 1, (w.y * 8 + ((c >> 3) & 7)) >> 1, (w.z * 8 + (c >> 6)) >> 1,
+                                                n0, n1)]);
+        } else return lf(xf[i]);
     };
     auto cx = [&](size_t i) -> float {
-        if constexpr (SEARCH) return lf(x[i]) + beta * S.doc[i];
-        else if constexpr (MODE == 3) return 0.0f;
+        if constexpr (SEARCH) return zat(x[i]) + beta * S.doc[i];
+        else if constexpr (Z) return 0.0f;
+        else if constexpr (PROLONG) return prolonged(lf(x[i]), S.yc[i]);
         else return lf(x[i]);
     };
     const CoarsePre<float> P = coarserow_pre<C, float>(t, cx, L.cc, L.dDc, I, J, K, typ);
     const float xl = cx(l);
-    const float bl = (MODE == 0 || MODE == 1 || MODE == 3) ? lf(b[l]) : 0.0f;
+    float bl = 0.0f;
+    if constexpr (MODE == 10) {
+        const T bt = sf<T>(S.rc[l] * rs);
+        S.bc[l] = bt;
+        bl = lf(bt);
+    } else if constexpr (JACOBI || RESID) bl = lf(b[l]);
     if constexpr (SEARCH) S.dnc[l] = xl;
     float diag, off;
     if (msk & 0x7eu) {
@@ -1031,23 +1129,23 @@ __device__ __forceinline__ void rowcoarse_wg(const uint32_t cb, const uint32_t p
     }
     const float ax = diag * xl - off;
     float res;
-    if (MODE == 0 || MODE == 3) res = diag > 0.0f ? xl + __fdiv_rn(OMEGA * (bl - ax), diag) : 0.0f;
-    else if (MODE == 1) res = bl - ax;
+    if (JACOBI) res = diag > 0.0f ? xl + __fdiv_rn(OMEGA * (bl - ax), diag) : 0.0f;
+    else if (RESID) res = bl - ax;
     else res = ax;
     res = row ? res : 0.0f;
     if constexpr (SEARCH) pq = row ? (double)xl * (double)res : 0.0;
-    out[l] = sf<T>(res);
+    if (!(N == 8 && MODE == 7 && (msk & 1u))) out[l] = sf<T>(res);
     }
     if constexpr (SEARCH) {
         double sum = block_sum_red(pq, lds);
         if (threadIdx.x == 0) S.partials[S.coarse0 + ps] = sum;
     }
 }
-template <int N, int MODE, class T, class C>
-__global__ __launch_bounds__(256) void k_rowcoarse(T* __restrict__ out, const T* __restrict__ x, const T* __restrict__ b,
-                                                   const T* __restrict__ xf, CompT<C> L, STopo t, SearchArgs S) {
+template <int N, int MODE, class T, class C, class X>
+__global__ __launch_bounds__(256) void k_rowcoarse(T* __restrict__ out, const X* __restrict__ x, const T* __restrict__ b,
+                                                   const X* __restrict__ xf, CompT<C> L, STopo t, RowArgs<T> S) {
     // neighbouring rows on one XCD
-    rowcoarse_wg<N, MODE, T, C>(xcd_tile(blockIdx.x, gridDim.x), blockIdx.x, out, x, b, xf, L, t, S);
+    rowcoarse_wg<N, MODE, T, C, X>(xcd_tile(blockIdx.x, gridDim.x), blockIdx.x, out, x, b, xf, L, t, S);
 }
 
 // One launch for a whole composite-level pass: the fine part's workgroups (tiles of
@@ -1056,28 +1154,28 @@ __global__ __launch_bounds__(256) void k_rowcoarse(T* __restrict__ out, const T*
 // overlap the fine tiles (bandwidth-bound) and the pass drains once. Workgroup g takes
 // coarse block floor(g C / G) when that count steps at g, else fine workgroup g minus
 // the coarse blocks before it: each index of either part is taken exactly once, in order.
-template <int N, int MODE, class T, class C, int NQ>
-__global__ __launch_bounds__(256) void k_rowcomp(T* __restrict__ outf, T* __restrict__ outc, const T* __restrict__ xf,
-                                                 const T* __restrict__ xc, const T* __restrict__ bf,
-                                                 const T* __restrict__ bc, CompT<C> L, STopo t, SearchArgs S, uint32_t ncb) {
+template <int N, int MODE, class T, class C, int NQ, class X>
+__global__ __launch_bounds__(256) void k_rowcomp(T* __restrict__ outf, T* __restrict__ outc, const X* __restrict__ xf,
+                                                 const X* __restrict__ xc, const T* __restrict__ bf,
+                                                 const T* __restrict__ bc, CompT<C> L, STopo t, RowArgs<T> S, uint32_t ncb) {
     const uint32_t G = gridDim.x, g = xcd_tile(blockIdx.x, G);
     const uint32_t c0 = (uint32_t)(((uint64_t)g * ncb) / G), c1 = (uint32_t)(((uint64_t)(g + 1) * ncb) / G);
-    if (c1 > c0) rowcoarse_wg<N, MODE, T, C>(c0, c0, outc, xc, bc, xf, L, t, S);
-    else if constexpr (N == 16) rowfine16_wg<MODE, T, C, NQ>(g - c0, outf, xf, bf, xc, L, t, S);
-    else rowfine8_wg<MODE, T, C>(g - c0, outf, xf, bf, xc, L, t);
+    if (c1 > c0) rowcoarse_wg<N, MODE, T, C, X>(c0, c0, outc, xc, bc, xf, L, t, S);
+    else if constexpr (N == 16) rowfine16_wg<MODE, T, C, NQ, X>(g - c0, outf, xf, bf, xc, L, t, S);
+    else rowfine8_wg<MODE, T, C>(g - c0, outf, xf, bf, xc, L, t, S);
 }
 // The reduced-precision V-cycle's entry as one launch in the same interleave: level 0's
 // fine part through jacobi0w_cvt_wg (r converted and stored, the sweep from zero) and the
-// coarse rows of that sweep (their r already converted).
+// coarse rows of that sweep, r converted on the way in.
 template <class T>
 __global__ __launch_bounds__(256) void k_head0(T* __restrict__ outf, T* __restrict__ outc, T* __restrict__ bh,
-                                               const float* __restrict__ r, const T* __restrict__ xc, const T* __restrict__ bc,
-                                               const T* __restrict__ xf, CompT<T> L, STopo t, int32_t nf,
-                                               const double* __restrict__ scal, int slot, uint32_t ncb) {
+                                               const float* __restrict__ r, CompT<T> L, STopo t, int32_t nf, RowArgs<T> S,
+                                               uint32_t ncb) {
     const uint32_t G = gridDim.x, g = xcd_tile(blockIdx.x, G);
     const uint32_t c0 = (uint32_t)(((uint64_t)g * ncb) / G), c1 = (uint32_t)(((uint64_t)(g + 1) * ncb) / G);
-    if (c1 > c0) rowcoarse_wg<16, 3, T, T>(c0, c0, outc, xc, bc, xf, L, t, SearchArgs{});
-    else jacobi0w_cvt_wg<T>(g - c0, outf, bh, r, L.rwf, L.actf, t.where, nf, scal, slot);
+    const T* none = nullptr;
+    if (c1 > c0) rowcoarse_wg<16, 10, T, T>(c0, c0, outc, none, none, none, L, t, S);
+    else jacobi0w_cvt_wg<T>(g - c0, outf, bh, r, L.rwf, L.actf, t.where, nf, S.scal, S.zslot);
 }
 
 // ─── dense levels (sflip.jl:1574-1657) ───────────────────────────────────────
@@ -1165,48 +1263,6 @@ __global__ void k_prolongdense(T* __restrict__ xf, const T* __restrict__ xc, con
 // ─── between the composite levels (sflip.jl:1661-1705) ───────────────────────
 
 template <class T>
-__device__ __forceinline__ void restrict01_el(const int32_t n, T* __restrict__ b1, const T* __restrict__ r0, const STopo& t,
-                                              int nslots) {
-    if (n >= nslots * SBCELLS1) return;
-    int s = (n >> 9) + 1, c = n & 511, i = c & 7, j = (c >> 3) & 7, k = c >> 6;
-    if (t.where[s - 1].x < 0) return;
-    float acc = 0.0f;
-    for (int cz = 0; cz < 2; ++cz)
-        for (int by = 0; by < 2; ++by)
-            for (int ax = 0; ax < 2; ++ax)
-                acc += lf(r0[(s - 1) * SBCELLS + (2 * i + ax) + 16 * ((2 * j + by) + 16 * (2 * k + cz))]);
-    b1[n] = sf<T>(acc);
-}
-// Level 1's right-hand side in one launch: the fine part restricted from level 0's
-// residual in the first `nfb` workgroups, the coarse part (shared by both levels) copied.
-template <class T>
-__global__ __launch_bounds__(256) void k_restrictcomp(T* __restrict__ b1f, const T* __restrict__ r0f, T* __restrict__ b1c,
-                                                      const T* __restrict__ r0c, size_t nc, STopo t, int nslots, uint32_t nfb) {
-    if (blockIdx.x < nfb) {
-        restrict01_el<T>((int32_t)(blockIdx.x * 256u + threadIdx.x), b1f, r0f, t, nslots);
-    } else {
-        const size_t l = (size_t)(blockIdx.x - nfb) * 256u + threadIdx.x;
-        if (l < nc) b1c[l] = r0c[l];
-    }
-}
-template <class T>
-__global__ void k_restrict12(T* __restrict__ b2, const T* __restrict__ r1f, const T* __restrict__ r1c, STopo t) {
-    int n0 = t.g.nc(0), n1 = t.g.nc(1), n2 = t.g.nc(2);
-    size_t l = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (l >= (size_t)n0 * n1 * n2) return;
-    int I, J, K;
-    unlin(l, n0, n1, I, J, K);
-    if (covered(t, I, J, K)) {
-        float acc = 0.0f;
-        for (int c = 0; c < 2; ++c)
-            for (int b = 0; b < 2; ++b)
-                for (int a = 0; a < 2; ++a) acc += lf(r1f[cellat<8>(t, 2 * I + a, 2 * J + b, 2 * K + c)]);
-        b2[l] = sf<T>(acc);
-    } else {
-        b2[l] = r1c[l];
-    }
-}
-template <class T>
 __device__ __forceinline__ void prolong21_el(const int32_t n, T* __restrict__ x1f, const T* __restrict__ x2,
                                              const uint8_t* __restrict__ act1, const STopo& t, float boost, int nslots) {
     if (n >= nslots * SBCELLS1) return;
@@ -1266,9 +1322,7 @@ __device__ __forceinline__ void prolong10_wg(const uint32_t tile, T* __restrict_
 template <class Y, class X>
 __global__ void k_convert(Y* __restrict__ yf, const X* __restrict__ xf, size_t nf, Y* __restrict__ yc, const X* __restrict__ xc,
                           size_t nc, const double* __restrict__ scal, int slot, int invert) {
-    float c = 1.0f;
-    if (slot >= 0) c = invert ? (float)(1.0 / scal[slot]) : (float)scal[slot];
-    if (!(c == c) || c == 0.0f || !(fabsf(c) <= 3.0e38f)) c = 1.0f;
+    const float c = slot_scale(scal, slot, invert != 0);
     size_t nf4 = nf / 4, ng = nf4 + nc / 4;
     for (size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x; g < ng; g += (size_t)gridDim.x * blockDim.x) {
         const Four<X>* xs = g < nf4 ? reinterpret_cast<const Four<X>*>(xf) + g : reinterpret_cast<const Four<X>*>(xc) + (g - nf4);
@@ -1444,28 +1498,25 @@ __global__ __launch_bounds__(256) void k_fcg_update(double* __restrict__ partial
     double s = block_sum_red(v, lds);
     if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
-// The reduced-precision V-cycle's correction back to FP32 (z = zh scal[slot], as k_convert)
-// fused with k_sdot2 on it: z.r and z.rold summed in k_sdot2's grouping (the same partials
-// for the same z).
+// k_sdot2 on the reduced-precision V-cycle's correction, z = zh scal[slot] (as k_convert)
+// taken on the way in; z itself is not stored, the next search converts it again (2 B read
+// twice a cell instead of 4 B written and read: 34 -> 26 us for 4,200 slots).
 template <class T>
-__global__ __launch_bounds__(256) void k_convert_dot2(double* __restrict__ partials, float* __restrict__ zf,
-                                                      float* __restrict__ zc, const T* __restrict__ hf, const T* __restrict__ hc,
+__global__ __launch_bounds__(256) void k_sdot2h(double* __restrict__ partials, const T* __restrict__ hf, const T* __restrict__ hc,
                                                       const float* __restrict__ rf, const float* __restrict__ rc,
                                                       const float* __restrict__ of, const float* __restrict__ oc,
                                                       const uint8_t* __restrict__ tf, const uint8_t* __restrict__ tc,
                                                       const uint8_t* __restrict__ cm, STopo t, int32_t nf,
                                                       const double* __restrict__ scal, int slot) {
     __shared__ double lds[4];
-    float c = (float)scal[slot];
-    if (!(c == c) || c == 0.0f || !(fabsf(c) <= 3.0e38f)) c = 1.0f;
+    const float c = slot_scale(scal, slot, false);
     size_t nf4 = (size_t)nf / 4, ng = nf4 + (size_t)t.g.nc(0) * t.g.nc(1) * t.g.nc(2) / 4;
     double v1 = 0, v2 = 0;
     for (size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x; g < ng; g += (size_t)gridDim.x * blockDim.x) {
-        const Four<T> h = g < nf4 ? reinterpret_cast<const Four<T>*>(hf)[g] : reinterpret_cast<const Four<T>*>(hc)[g - nf4];
-        const float4 z = make_float4(lf(h.v[0]) * c, lf(h.v[1]) * c, lf(h.v[2]) * c, lf(h.v[3]) * c);
-        grp(zf, zc, g, nf4) = z;
         unsigned m = unknown4(g, nf4, tf, tc, cm, t);
         if (!m) continue;
+        const Four<T> h = g < nf4 ? reinterpret_cast<const Four<T>*>(hf)[g] : reinterpret_cast<const Four<T>*>(hc)[g - nf4];
+        const float4 z = make_float4(lf(h.v[0]) * c, lf(h.v[1]) * c, lf(h.v[2]) * c, lf(h.v[3]) * c);
         v1 += dot4(m, z, grp(rf, rc, g, nf4));
         v2 += dot4(m, z, grp(of, oc, g, nf4));
     }
@@ -1895,7 +1946,7 @@ struct SparseSolver {
         if (s.nslots) {   // level 0's full diagonal (mode 6 of the level-0 rows)
             Hier<float, float> H = hier32();
             hipLaunchKernelGGL((k_rowfine16<6, float, float>), dim3(4 * s.nslots), dim3(256), 0, st, s.dgf.p, (const float*)nullptr,
-                               (const float*)nullptr, (const float*)nullptr, H.L0, t, SearchArgs{});
+                               (const float*)nullptr, (const float*)nullptr, H.L0, t, RowArgs<float>{});
         }
         MAEL_LAUNCH_CHECK();
     }
@@ -1926,7 +1977,7 @@ struct SparseSolver {
 
     // The hierarchy in one storage precision: its vectors and couplings.
     template <class T, class C> struct Hier {
-        SVecT<T> q, tmp, X1x, X1b, X1r, X1t;
+        SVecT<T> tmp, X1x, X1b, X1t;
         std::vector<T*> Dx, Db, Dt;
         CompT<C> L0, L1;
         std::vector<DViewT<C>> D;
@@ -1934,10 +1985,9 @@ struct SparseSolver {
     };
     Hier<float, float> hier32() {
         Hier<float, float> H;
-        H.q = {s.q.fine.p, s.q.coarse.p};
         H.tmp = {s.tmp.fine.p, s.tmp.coarse.p};
         H.X1x = {s.X1x.fine.p, s.X1x.coarse.p}; H.X1b = {s.X1b.fine.p, s.X1b.coarse.p};
-        H.X1r = {s.X1r.fine.p, s.X1r.coarse.p}; H.X1t = {s.X1t.fine.p, s.X1t.coarse.p};
+        H.X1t = {s.X1t.fine.p, s.X1t.coarse.p};
         for (auto& L : s.D) {
             H.Dx.push_back(L.x.p); H.Db.push_back(L.b.p); H.Dt.push_back(L.t.p);
             H.D.push_back(DViewT<float>{i3(L.n), {L.c[0].p, L.c[1].p, L.c[2].p}, L.dD.p, L.act.p});
@@ -1955,9 +2005,9 @@ struct SparseSolver {
         MPStore& m = s.mp;
         auto V = [&](DBuf<uint16_t>& f, DBuf<uint16_t>& c) { return SVecT<T>{(T*)f.p, (T*)c.p}; };
         Hier<T, T> H;
-        H.q = V(m.q[0], m.q[1]); H.tmp = V(m.tmp[0], m.tmp[1]);
+        H.tmp = V(m.tmp[0], m.tmp[1]);
         H.X1x = V(m.X1[0][0], m.X1[0][1]); H.X1b = V(m.X1[1][0], m.X1[1][1]);
-        H.X1r = V(m.X1[2][0], m.X1[2][1]); H.X1t = V(m.X1[3][0], m.X1[3][1]);
+        H.X1t = V(m.X1[2][0], m.X1[2][1]);
         for (size_t l = 0; l < s.D.size(); ++l) {
             H.Dx.push_back((T*)m.Dv[l][0].p); H.Db.push_back((T*)m.Dv[l][1].p);
             H.Dt.push_back((T*)m.Dv[l][2].p);
@@ -1996,7 +2046,7 @@ struct SparseSolver {
         if (s.nslots) {   // level 0's Jacobi weights, omega / diag (mode 5 of the level-0 rows)
             Hier<T, T> H = hier16<T>();
             hipLaunchKernelGGL((k_rowfine16<5, T, T>), dim3(4 * s.nslots), dim3(256), 0, st, (T*)m.rwf.p, (const T*)nullptr,
-                               (const T*)nullptr, (const T*)nullptr, H.L0, t, SearchArgs{});
+                               (const T*)nullptr, (const T*)nullptr, H.L0, t, RowArgs<T>{});
         }
         MAEL_LAUNCH_CHECK();
     }
@@ -2009,54 +2059,45 @@ struct SparseSolver {
     template <class T> void zero_t(SVecT<T> v, size_t nfine) { zero_t(v.f, nfine); zero_t(v.c, Cc); }
     void zero(SVec v, size_t nfine) { zero_t(SVecT<float>{v.f, v.c}, nfine); }
 
-    // One composite-level pass (MODE 0 Jacobi, 1 residual, 2 apply) over the fine part
-    // (N^3 a slot) and the coarse part.
-    template <int N, int MODE, class T, class C>
-    void rows(SVecT<T> out, SVecT<T> x, SVecT<T> b, const CompT<C>& L, SearchArgs S = SearchArgs{}) {
-        int32_t nfl = s.nslots * N * N * N;
-        // one launch for both parts, except the reduced-precision sweep from zero (pointwise)
-        constexpr bool FUSE = !(N == 16 && MODE == 3 && !std::is_same<T, float>::value);
-        if constexpr (FUSE) {
-            if (nfl) {
-                constexpr int NQ = (N == 16 && (std::is_same<T, float>::value || MODE == 0 || MODE == 1)) ? 2 : 1;
-                const uint32_t nfw = N == 16 ? (uint32_t)s.nslots * (uint32_t)(4 / NQ) : (uint32_t)s.nslots;
-                const uint32_t ncb = (uint32_t)cdiv(Cc, 256);
-                if (N == 16 && MODE == 0) s.kt.begin(K_RBGS, st);
-                hipLaunchKernelGGL((k_rowcomp<N, MODE, T, C, NQ>), dim3(nfw + ncb), dim3(256), 0, st, out.f, out.c, x.f, x.c,
-                                   b.f, b.c, L, t, S, ncb);
-                if (N == 16 && MODE == 0) s.kt.end(K_RBGS, st);
-                return;
-            }
+    // One composite-level pass (MODE 0 Jacobi, 1 residual, 2 apply, ...) over the fine part
+    // (N^3 a slot) and the coarse part, in one launch.
+    template <int N, int MODE, class T, class C, class X>
+    void rows(SVecT<T> out, SVecT<X> x, SVecT<T> b, const CompT<C>& L, RowArgs<T> S = RowArgs<T>{}) {
+        constexpr bool SWEEP = N == 16 && (MODE == 0 || MODE == 8);
+        const uint32_t ncb = (uint32_t)cdiv(Cc, 256);
+        if (SWEEP) s.kt.begin(K_RBGS, st);
+        if (s.nslots) {
+            constexpr int NQ = N == 16 ? 2 : 1;   // 8-plane tiles
+            const uint32_t nfw = N == 16 ? (uint32_t)s.nslots * (uint32_t)(4 / NQ) : (uint32_t)s.nslots;
+            hipLaunchKernelGGL((k_rowcomp<N, MODE, T, C, NQ, X>), dim3(nfw + ncb), dim3(256), 0, st, out.f, out.c, x.f, x.c, b.f,
+                               b.c, L, t, S, ncb);
+        } else {
+            if (MODE == 4) fill_async(S.partials, (size_t)1, 0.0, st);   // no fine workgroups: the finish reads one zero
+            hipLaunchKernelGGL((k_rowcoarse<N, MODE, T, C, X>), dim3(ncb), dim3(256), 0, st, out.c, x.c, b.c, x.f, L, t, S);
         }
-        if (nfl) {
-            if (N == 16 && MODE == 0) s.kt.begin(K_RBGS, st);
-            if constexpr (N == 16 && MODE == 3 && !std::is_same<T, float>::value)
-                hipLaunchKernelGGL((k_jacobi0w<T>), dim3(s.nslots * 4), dim3(256), 0, st, out.f, b.f, L.rwf, L.actf, t.where, nfl);
-            else if constexpr (N == 16 && (std::is_same<T, float>::value || MODE == 0 || MODE == 1))   // 8-plane tiles
-                hipLaunchKernelGGL((k_rowfine16<MODE, T, C, 2>), dim3(2 * s.nslots), dim3(256), 0, st, out.f, x.f, b.f, x.c, L, t,
-                                   S);
-            else if constexpr (N == 16)
-                hipLaunchKernelGGL((k_rowfine16<MODE, T, C>), dim3(4 * s.nslots), dim3(256), 0, st, out.f, x.f, b.f, x.c, L, t, S);
-            else
-                hipLaunchKernelGGL((k_rowfine8<MODE, T, C>), dim3(s.nslots), dim3(256), 0, st, out.f, x.f, b.f, x.c, L, t);
-            if (N == 16 && MODE == 0) s.kt.end(K_RBGS, st);
-        } else if (MODE == 4) {
-            fill_async(S.partials, (size_t)1, 0.0, st);   // no fine workgroups: the finish reads one zero
-        }
-        hipLaunchKernelGGL((k_rowcoarse<N, MODE, T, C>), dim3(cdiv(Cc, 256)), dim3(256), 0, st, out.c, x.c, b.c, x.f, L, t, S);
+        if (SWEEP) s.kt.end(K_RBGS, st);
     }
     // flexible CG's fused step: dn = z + beta d (beta on the device), q = A dn, and d.q
-    // (with the reference's checks) into alpha
-    void search(SVec q, SVec dn, SVec z, SVec d) {
+    // (with the reference's checks) into alpha. In reduced precision z is the V-cycle's,
+    // times scal[SS_RNORM].
+    template <class X> void search_z(SVec q, SVec dn, SVecT<X> z, SVec d) {
         Hier<float, float> H = hier32();
         int32_t fine_groups = s.nslots ? 2 * s.nslots : 1;   // the level-0 rows' 8-plane tiles
-        SearchArgs S{d.f, d.c, dn.f, dn.c, s.partials.p, fine_groups, s.scal.p};
+        RowArgs<float> S;
+        S.dof = d.f; S.doc = d.c; S.dnf = dn.f; S.dnc = dn.c;
+        S.partials = s.partials.p; S.coarse0 = fine_groups; S.scal = s.scal.p; S.zslot = SS_RNORM;
         s.kt.begin(K_SEARCH, st);
-        rows<16, 4>(SVecT<float>{q.f, q.c}, SVecT<float>{z.f, z.c}, SVecT<float>{z.f, z.c}, H.L0, S);
+        rows<16, 4>(SVecT<float>{q.f, q.c}, z, SVecT<float>{nullptr, nullptr}, H.L0, S);
         s.kt.end(K_SEARCH, st);
         hipLaunchKernelGGL(k_sfinish, dim3(1), dim3(FINISH_THREADS), 0, st, s.partials.p, fine_groups + (int)cdiv(Cc, 256), s.scal.p,
                            (int)SF_ALPHA, 0);
         MAEL_LAUNCH_CHECK();
+    }
+    void search(SVec q, SVec dn, SVec z, SVec d) {
+        MPStore& m = s.mp;
+        if (precision == 0) search_z(q, dn, SVecT<float>{z.f, z.c}, d);
+        else if (precision == 1) search_z(q, dn, SVecT<__half>{(__half*)m.z[0].p, (__half*)m.z[1].p}, d);
+        else search_z(q, dn, SVecT<bf16>{(bf16*)m.z[0].p, (bf16*)m.z[1].p}, d);
     }
     template <int N, class T, class C> void smooth(SVecT<T> x, SVecT<T> b, SVecT<T> tmp, const CompT<C>& L, int sweeps) {
         for (int k = 0; k < sweeps; ++k) {
@@ -2064,14 +2105,25 @@ struct SparseSolver {
             rows<N, 0>(x, tmp, b, L);
         }
     }
-    // The same from x = 0: the first sweep reads no x, and x needs no clearing (every cell
-    // of the level's slots and coarse part is written).
-    template <int N, class T, class C>
-    void smooth0(SVecT<T> x, SVecT<T> b, SVecT<T> tmp, const CompT<C>& L, int sweeps, size_t nfine, bool queued = false) {
-        if (sweeps < 1) { zero_t(x, nfine); return; }
-        if (!queued) rows<N, 3>(tmp, x, b, L);   // else already queued (queue_head)
-        rows<N, 0>(x, tmp, b, L);
-        smooth<N>(x, b, tmp, L, sweeps - 1);
+    // The same from level 1's x = 0: the first sweep reads no x, and x needs no clearing
+    // (every cell of the level's slots and coarse part is written).
+    template <class T, class C> void smooth1(Hier<T, C>& H, int sweeps) {
+        if (sweeps < 1) { zero_t(H.X1x, (size_t)s.nslots * SBCELLS1); return; }
+        rows<8, 3>(H.X1t, H.X1x, H.X1b, H.L1);
+        rows<8, 0>(H.X1x, H.X1t, H.X1b, H.L1);
+        smooth<8>(H.X1x, H.X1b, H.X1t, H.L1, sweeps - 1);
+    }
+    // Level 0's first sweep from zero into H.tmp. In reduced precision it takes r in FP32 and
+    // writes its copy b = r / scal[nslot] for the rest of the V-cycle.
+    template <class T, class C> void head0(Hier<T, C>& H, SVecT<T> z, SVecT<T> b, SVec r, int nslot) {
+        if constexpr (std::is_same<T, float>::value) {
+            rows<16, 3>(H.tmp, z, b, H.L0);
+        } else {
+            RowArgs<T> S;
+            S.rc = r.c; S.bc = b.c; S.scal = s.scal.p; S.zslot = nslot;
+            const uint32_t ncb = (uint32_t)cdiv(Cc, 256), nfw = (uint32_t)s.nslots * 4u;   // 1024 fine cells a workgroup
+            hipLaunchKernelGGL((k_head0<T>), dim3(nfw + ncb), dim3(256), 0, st, H.tmp.f, H.tmp.c, b.f, r.f, H.L0, t, nf, S, ncb);
+        }
     }
 
     // The dense levels of the V-cycle (from the right-hand side in Db[0]); returns the first
@@ -2148,48 +2200,63 @@ struct SparseSolver {
         }
     }
 
-    // sflip.jl:1722-1762 vcycle!: z = M^-1 r in the hierarchy H (coarsest in arithmetic A).
+    // sflip.jl:1722-1762 vcycle!: z = M^-1 b in the hierarchy H (coarsest in arithmetic A).
+    // In reduced precision b is the copy of r that the head makes (already made if `queued`;
+    // without sweeps the caller's).
     template <class T, class C, class A>
-    void vcycle_t(Hier<T, C>& H, SVecT<T> z, SVecT<T> r, int sweeps, int coarse, float boost, bool queued = false) {
-        int ns = s.nslots;
-        smooth0<16>(z, r, H.tmp, H.L0, sweeps, (size_t)nf, queued);
-        rows<16, 1>(H.q, z, r, H.L0);
-        const uint32_t nfr = (uint32_t)cdiv((size_t)ns * SBCELLS1, 256);
-        hipLaunchKernelGGL(k_restrictcomp<T>, dim3(nfr + (uint32_t)cdiv(Cc, 256)), dim3(256), 0, st, H.X1b.f, H.q.f, H.X1b.c, H.q.c,
-                           Cc, t, ns, nfr);
-        smooth0<8>(H.X1x, H.X1b, H.X1t, H.L1, sweeps, (size_t)ns * SBCELLS1);
-        rows<8, 1>(H.X1r, H.X1x, H.X1b, H.L1);
-        hipLaunchKernelGGL(k_restrict12<T>, dim3(cdiv(Cc, 256)), dim3(256), 0, st, H.Db[0], H.X1r.f, H.X1r.c, t);
+    void vcycle_t(Hier<T, C>& H, SVecT<T> z, SVecT<T> b, SVec r, int nslot, int sweeps, int coarse, float boost, bool queued) {
+        const int ns = s.nslots;
+        if (sweeps < 1) {
+            zero_t(z, (size_t)nf);
+        } else {
+            if (!queued) head0(H, z, b, r, nslot);
+            rows<16, 0>(z, H.tmp, b, H.L0);
+            smooth<16>(z, b, H.tmp, H.L0, sweeps - 1);
+        }
+        rows<16, 7>(H.X1b, z, b, H.L0);   // the residual, restricted
+        smooth1(H, sweeps);
+        rows<8, 7>(SVecT<T>{H.Db[0], H.Db[0]}, H.X1x, H.X1b, H.L1);
         T* x2 = dense_levels<T, C, A>(H, sweeps, coarse, boost);
         SLevel& D2 = s.D[0];
-        const uint32_t ncb = (uint32_t)cdiv(Cc, 256), nfb1 = (uint32_t)cdiv((size_t)ns * SBCELLS1, 256);
-        hipLaunchKernelGGL((k_prolongcomp<T, 1>), dim3(nfb1 + ncb), dim3(256), 0, st, H.X1x.f, x2, s.act1.p, H.X1x.c, x2,
-                           D2.act.p, t, boost, ns, nfb1);
-        smooth<8>(H.X1x, H.X1b, H.X1t, H.L1, sweeps);
-        const uint32_t nfb0 = (uint32_t)cdiv((size_t)nf, 1024);
-        hipLaunchKernelGGL((k_prolongcomp<T, 0>), dim3(nfb0 + ncb), dim3(256), 0, st, z.f, H.X1x.f, s.types.fine.p, z.c, H.X1x.c,
-                           D2.act.p, t, boost, nf, nfb0);
-        smooth<16>(z, r, H.tmp, H.L0, sweeps);
+        const uint32_t ncb = (uint32_t)cdiv(Cc, 256);
+        if (sweeps < 1) {   // the prolongations by themselves
+            const uint32_t nfb1 = (uint32_t)cdiv((size_t)ns * SBCELLS1, 256), nfb0 = (uint32_t)cdiv((size_t)nf, 1024);
+            hipLaunchKernelGGL((k_prolongcomp<T, 1>), dim3(nfb1 + ncb), dim3(256), 0, st, H.X1x.f, x2, s.act1.p, H.X1x.c, x2,
+                               D2.act.p, t, boost, ns, nfb1);
+            hipLaunchKernelGGL((k_prolongcomp<T, 0>), dim3(nfb0 + ncb), dim3(256), 0, st, z.f, H.X1x.f, s.types.fine.p, z.c,
+                               H.X1x.c, D2.act.p, t, boost, nf, nfb0);
+        } else {            // in the first sweep after each
+            RowArgs<T> S;
+            S.boost = boost;
+            S.yf = x2; S.yc = x2;
+            rows<8, 8>(H.X1t, H.X1x, H.X1b, H.L1, S);
+            rows<8, 0>(H.X1x, H.X1t, H.X1b, H.L1);
+            smooth<8>(H.X1x, H.X1b, H.X1t, H.L1, sweeps - 1);
+            S.yf = H.X1x.f; S.yc = H.X1x.c;
+            rows<16, 8>(H.tmp, z, b, H.L0, S);
+            rows<16, 0>(z, H.tmp, b, H.L0);
+            smooth<16>(z, b, H.tmp, H.L0, sweeps - 1);
+        }
         MAEL_LAUNCH_CHECK();
     }
 
     int precision = 0;   // 0 FP32, 1 FP16 storage, 2 BF16 storage
     // z = M^-1 r. In reduced precision r is scaled by 1 / scal[nslot] on the way in (its
     // norm, so its entries are at most 1) and z back on the way out. With `rold`
-    // (flexible CG), z.r and z.rold are also summed into the partials as k_sdot2 does
-    // (fused with the conversion back in reduced precision).
-    // The V-cycle's first launches (the reduced-precision copy of r and the level-0 sweep
-    // from zero) queued ahead of a host read that decides whether the V-cycle runs at
+    // (flexible CG), z.r and z.rold are also summed into the partials as k_sdot2 does, and
+    // in reduced precision z stays in the hierarchy's precision (the next search scales it).
+    // The V-cycle's first launch (level 0's sweep from zero and the reduced-precision copy of
+    // r) queued ahead of a host read that decides whether the V-cycle runs at
     // all, so the device works through the read's round trip; the next vcycle() on the
     // same z and r skips them. Whoever changes r (or leaves the solve) before that clears
-    // `head`, and the V-cycle then runs whole (overwriting what the queued launches wrote,
-    // all of it V-cycle scratch).
+    // `head`, and the V-cycle then runs whole (overwriting what the queued launch wrote, all
+    // of it V-cycle scratch).
     bool head = false;
     void queue_head(SVec z, SVec r, int sweeps, int nslot) {
         if (sweeps < 1) return;
         if (precision == 0) {
             Hier<float, float> H = hier32();
-            rows<16, 3>(H.tmp, SVecT<float>{z.f, z.c}, SVecT<float>{r.f, r.c}, H.L0);
+            head0(H, SVecT<float>{z.f, z.c}, SVecT<float>{r.f, r.c}, r, -1);
         } else if (precision == 1) {
             queue_head_mp<__half>(r, nslot);
         } else {
@@ -2197,26 +2264,17 @@ struct SparseSolver {
         }
         head = true;
     }
-    // r into the hierarchy's precision and level 0's sweep from zero on it: the coarse part
-    // of r converted, then one launch (k_head0) for the fine part's conversion and sweep
-    // and the coarse rows
     template <class T> void queue_head_mp(SVec r, int nslot) {
         Hier<T, T> H = hier16<T>();
         MPStore& m = s.mp;
-        SVecT<T> zh{(T*)m.z[0].p, (T*)m.z[1].p}, rh{(T*)m.r[0].p, (T*)m.r[1].p};
-        unsigned g = std::min<unsigned>(cdiv(Cc, 256), 8192);
-        hipLaunchKernelGGL((k_convert<T, float>), dim3(g), dim3(256), 0, st, rh.f, r.f, (size_t)0, rh.c, r.c, Cc, s.scal.p, nslot,
-                           1);
-        const uint32_t ncb = (uint32_t)cdiv(Cc, 256), nfw = (uint32_t)s.nslots * 4u;   // 1024 fine cells a workgroup
-        hipLaunchKernelGGL((k_head0<T>), dim3(nfw + ncb), dim3(256), 0, st, H.tmp.f, H.tmp.c, rh.f, r.f, zh.c, rh.c, zh.f, H.L0, t,
-                           nf, s.scal.p, nslot, ncb);
+        head0(H, SVecT<T>{(T*)m.z[0].p, (T*)m.z[1].p}, SVecT<T>{(T*)m.r[0].p, (T*)m.r[1].p}, r, nslot);
     }
     void vcycle(SVec z, SVec r, int sweeps, int coarse, float boost, int nslot = -1, const SVec* rold = nullptr) {
         const bool queued = head;
         head = false;
         if (precision == 0) {
             Hier<float, float> H = hier32();
-            vcycle_t<float, float, float>(H, SVecT<float>{z.f, z.c}, SVecT<float>{r.f, r.c}, sweeps, coarse, boost, queued);
+            vcycle_t<float, float, float>(H, SVecT<float>{z.f, z.c}, SVecT<float>{r.f, r.c}, r, -1, sweeps, coarse, boost, queued);
             if (rold)
                 hipLaunchKernelGGL(k_sdot2, dim3(DOT_BLOCKS), dim3(256), 0, st, s.partials.p, z.f, z.c, r.f, r.c, rold->f,
                                    rold->c, s.types.fine.p, s.types.coarse.p, s.cmask.p, t, nf);
@@ -2231,24 +2289,16 @@ struct SparseSolver {
         MPStore& m = s.mp;
         SVecT<T> zh{(T*)m.z[0].p, (T*)m.z[1].p}, rh{(T*)m.r[0].p, (T*)m.r[1].p};
         unsigned g = std::min<unsigned>(cdiv((size_t)nf + Cc, 256), 8192);
-        if (!queued && sweeps >= 1) {
-            queue_head_mp<T>(r, nslot);
-            queued = true;
-        } else if (!queued) {
+        if (sweeps < 1)
             hipLaunchKernelGGL((k_convert<T, float>), dim3(g), dim3(256), 0, st, rh.f, r.f, (size_t)nf, rh.c, r.c, Cc, s.scal.p,
                                nslot, 1);
-        }
-        vcycle_t<T, T, double>(H, zh, rh, sweeps, coarse, boost, queued);
-        if (rold && nslot >= 0)
-            hipLaunchKernelGGL((k_convert_dot2<T>), dim3(DOT_BLOCKS), dim3(256), 0, st, s.partials.p, z.f, z.c, zh.f, zh.c, r.f,
-                               r.c, rold->f, rold->c, s.types.fine.p, s.types.coarse.p, s.cmask.p, t, nf, s.scal.p, nslot);
-        else {
+        vcycle_t<T, T, double>(H, zh, rh, r, nslot, sweeps, coarse, boost, queued);
+        if (rold)   // z stays where it is: the dots and the next search convert it
+            hipLaunchKernelGGL((k_sdot2h<T>), dim3(DOT_BLOCKS), dim3(256), 0, st, s.partials.p, zh.f, zh.c, r.f, r.c, rold->f,
+                               rold->c, s.types.fine.p, s.types.coarse.p, s.cmask.p, t, nf, s.scal.p, nslot);
+        else
             hipLaunchKernelGGL((k_convert<float, T>), dim3(g), dim3(256), 0, st, z.f, zh.f, (size_t)nf, z.c, zh.c, Cc, s.scal.p,
                                nslot, 0);
-            if (rold)
-                hipLaunchKernelGGL(k_sdot2, dim3(DOT_BLOCKS), dim3(256), 0, st, s.partials.p, z.f, z.c, r.f, r.c, rold->f,
-                                   rold->c, s.types.fine.p, s.types.coarse.p, s.cmask.p, t, nf);
-        }
     }
 
     void apply(SVec q, SVec x) {

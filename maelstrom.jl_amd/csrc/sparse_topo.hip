@@ -31,7 +31,7 @@ SparseBasin::SparseBasin(const SGrid& grid, int nblk, int64_t cap, int32_t bnd, 
         c1[a].alloc((size_t)blocks * SBFACES1);
     }
     dD1.alloc((size_t)blocks * SBCELLS1); act1.alloc((size_t)blocks * SBCELLS1);
-    for (auto* f : {&X1x, &X1b, &X1r, &X1t}) f->alloc((size_t)blocks * SBCELLS1, Cc);
+    for (auto* f : {&X1x, &X1b, &X1t}) f->alloc((size_t)blocks * SBCELLS1, Cc);
     // the coarse grid and its halvings until a workgroup solves the coarsest (sflip.jl:319-326)
     int m[3] = {g.nc(0), g.nc(1), g.nc(2)};
     while (true) {
@@ -77,7 +77,7 @@ SparseBasin::SparseBasin(const SGrid& grid, int nblk, int64_t cap, int32_t bnd, 
         fill_async(fl2[a].fine.p, nfa, (uint8_t)0, s);
         fill_async(fl2[a].coarse.p, nfaces(a), (uint8_t)0, s);
     }
-    for (auto* f : {&X1x, &X1b, &X1r, &X1t}) {
+    for (auto* f : {&X1x, &X1b, &X1t}) {
         fill_async(f->fine.p, (size_t)blocks * SBCELLS1, 0.0f, s);
         fill_async(f->coarse.p, Cc, 0.0f, s);
     }
@@ -89,7 +89,7 @@ SparseBasin::SparseBasin(const SGrid& grid, int nblk, int64_t cap, int32_t bnd, 
 void SparseBasin::mp_alloc() {
     if (mp.ready) return;
     size_t nf = (size_t)blocks * SBCELLS, nfa = (size_t)blocks * SBFACES, n1 = (size_t)blocks * SBCELLS1, Cc = ncells();
-    for (auto* v : {mp.z, mp.r, mp.q, mp.tmp}) { v[0].alloc(nf); v[1].alloc(Cc); }
+    for (auto* v : {mp.z, mp.r, mp.tmp}) { v[0].alloc(nf); v[1].alloc(Cc); }
     for (auto& v : mp.X1) { v[0].alloc(n1); v[1].alloc(Cc); }
     mp.Dv.resize(D.size());
     mp.Dc.resize(D.size());
@@ -103,7 +103,7 @@ void SparseBasin::mp_alloc() {
     }
     mp.dDf.alloc(nf); mp.dDc.alloc(Cc); mp.dD1.alloc(n1); mp.rwf.alloc(nf);
     // every vector starts at zero: free slots are never written and must read as zero
-    for (auto* v : {mp.z, mp.r, mp.q, mp.tmp}) { fill_async(v[0].p, nf, (uint16_t)0, st.s); fill_async(v[1].p, Cc, (uint16_t)0, st.s); }
+    for (auto* v : {mp.z, mp.r, mp.tmp}) { fill_async(v[0].p, nf, (uint16_t)0, st.s); fill_async(v[1].p, Cc, (uint16_t)0, st.s); }
     for (auto& v : mp.X1) { fill_async(v[0].p, n1, (uint16_t)0, st.s); fill_async(v[1].p, Cc, (uint16_t)0, st.s); }
     st.sync();
     mp.ready = true;
