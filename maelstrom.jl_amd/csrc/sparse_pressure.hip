@@ -591,7 +591,7 @@ __device__ inline float slot_scale(const double* __restrict__ scal, int slot, bo
 }
 
 // sflip.jl:1218-1269 on the fine cells of a level: mode 0 Jacobi (out = x + w (b - A x) /
-// diag), 1 residual (out = b - A x), 2 apply (out = A x), 3 Jacobi from x = 0 (x not
+// diag), 7 residual (b - A x, sflip.jl:1661-1690 with its restriction), 2 apply (out = A x), 3 Jacobi from x = 0 (x not
 // read); inactive cells and the cells of free slots get 0. Mode 5 writes w / diag (0 where
 // diag is not positive): in reduced precision the level-0 Jacobi sweep takes that weight
 // r per cell, out = (1 - w) x + r (b + off), and needs neither the diagonal nor the
@@ -645,9 +645,9 @@ __device__ __forceinline__ void rowfine16_wg(const uint32_t tile, T* __restrict_
                                              const STopo& t, const RowArgs<T>& S) {
     constexpr bool Z = MODE == 3 || MODE == 5 || MODE == 6, SEARCH = MODE == 4;
     constexpr bool RESTRICT = MODE == 7, PROLONG = MODE == 8;
-    constexpr bool JACOBI = MODE == 0 || PROLONG, RESID = MODE == 1 || RESTRICT;
+    constexpr bool JACOBI = MODE == 0 || PROLONG;
     // reduced precision: the sweep and the residual take the weight r = omega / diag
-    constexpr bool RW = (JACOBI || RESID) && !std::is_same<T, float>::value;
+    constexpr bool RW = (JACOBI || RESTRICT) && !std::is_same<T, float>::value;
     // FP32: the rows take the full diagonal computed once a solve (mode 6), the same sum
     constexpr bool FD = MODE != 5 && MODE != 6 && std::is_same<T, float>::value;
     constexpr bool NW = !RW && !FD;                                        // the couplings staged
@@ -734,7 +734,7 @@ __device__ __forceinline__ void rowfine16_wg(const uint32_t tile, T* __restrict_
         const uint32_t n = cell(q);
         tq[q] = *reinterpret_cast<const uint32_t*>(tf + n);
         dq[q] = load4(RW ? L.rwf : (FD ? L.dgf : L.dDf), n);   // the Dirichlet part, the weight or the diagonal
-        if constexpr (!JACOBI && !RESID && MODE != 3) {
+        if constexpr (!JACOBI && !RESTRICT && MODE != 3) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) bq[q].v[e] = sf<T>(0.0f);
         } else {
@@ -889,7 +889,7 @@ __device__ __forceinline__ void rowfine16_wg(const uint32_t tile, T* __restrict_
                 } else {
                     float ax = diag * x0[q][e] - off;
                     if (JACOBI || MODE == 3) res = diag > 0.0f ? x0[q][e] + __fdiv_rn(OMEGA * (bb - ax), diag) : 0.0f;
-                    else if (RESID) res = bb - ax;
+                    else if (RESTRICT) res = bb - ax;
                     else res = ax;
                 }
                 if constexpr (SEARCH) pq += (double)x0[q][e] * (double)res;
@@ -1036,7 +1036,7 @@ __device__ __forceinline__ void rowfine8_wg(const uint32_t tile, T* __restrict__
             float x0 = Z ? 0.0f : lf(sx[Z ? 0 : h]);
             float ax = diag * x0 - off;
             if (MODE == 0 || PROLONG || MODE == 3) res = diag > 0.0f ? x0 + __fdiv_rn(OMEGA * (lf(b[n]) - ax), diag) : 0.0f;
-            else if (MODE == 1 || RESTRICT) res = lf(b[n]) - ax;
+            else if (RESTRICT) res = lf(b[n]) - ax;
             else res = ax;
         }
         if constexpr (RESTRICT) sr[c] = sf<T>(res);
@@ -1067,7 +1067,7 @@ __device__ __forceinline__ void rowcoarse_wg(const uint32_t cb, const uint32_t p
                                              const X* __restrict__ x, const T* __restrict__ b, const X* __restrict__ xf,
                                              const CompT<C>& L, const STopo& t, const RowArgs<T>& S) {
     constexpr bool SEARCH = MODE == 4, PROLONG = MODE == 8, Z = MODE == 3 || MODE == 10;
-    constexpr bool JACOBI = MODE == 0 || PROLONG || Z, RESID = MODE == 1 || MODE == 7;
+    constexpr bool JACOBI = MODE == 0 || PROLONG || Z, RESID = MODE == 7;
     __shared__ double lds[4];
     int n0 = t.g.nc(0), n1 = t.g.nc(1), n2 = t.g.nc(2);
     size_t l = (size_t)cb * 256u + threadIdx.x;
@@ -1260,69 +1260,14 @@ __global__ void k_prolongdense(T* __restrict__ xf, const T* __restrict__ xc, con
     unlin(l, nf.x, nf.y, i, j, k);
     if (actf[l] != 0) xf[l] = sf<T>(lf(xf[l]) + boost * lf(xc[cl(i >> 1, j >> 1, k >> 1, nc.x, nc.y)]));
 }
-// ─── between the composite levels (sflip.jl:1661-1705) ───────────────────────
-
-template <class T>
-__device__ __forceinline__ void prolong21_el(const int32_t n, T* __restrict__ x1f, const T* __restrict__ x2,
-                                             const uint8_t* __restrict__ act1, const STopo& t, float boost, int nslots) {
-    if (n >= nslots * SBCELLS1) return;
-    int s = (n >> 9) + 1, c = n & 511, i = c & 7, j = (c >> 3) & 7, k = c >> 6;
-    int4 w = t.where[s - 1];
-    if (w.x < 0 || act1[n] == 0) return;
-    x1f[n] = sf<T>(lf(x1f[n]) + boost * lf(x2[cl((w.x * 8 + i) >> 1, (w.y * 8 + j) >> 1, (w.z * 8 + k) >> 1, t.g.nc(0), t.g.nc(1))]));
-}
-// A composite level's prolongation in one launch: its fine part (level 0 from level 1,
-// 1024 cells a workgroup, LVL 0; level 1 from the first dense level, LVL 1) in the first
-// `nfb` workgroups, its coarse part (from the coarser grid's coarse part or level) after.
-template <class T, int LVL>
-__global__ __launch_bounds__(256) void k_prolongcomp(T* __restrict__ xf, const T* __restrict__ fromf,
-                                                     const uint8_t* __restrict__ maskf, T* __restrict__ xc,
-                                                     const T* __restrict__ fromc, const uint8_t* __restrict__ actc, STopo t,
-                                                     float boost, int32_t nfine, uint32_t nfb) {
-    if (blockIdx.x < nfb) {
-        if constexpr (LVL == 0) prolong10_wg<T>(xcd_tile(blockIdx.x, nfb), xf, fromf, maskf, t, boost, nfine);
-        else prolong21_el<T>((int32_t)(blockIdx.x * 256u + threadIdx.x), xf, fromf, maskf, t, boost, nfine);
-    } else {
-        prolongcoarse_el<T>((size_t)(blockIdx.x - nfb) * 256u + threadIdx.x, xc, fromc, actc, t, boost);
-    }
-}
-template <class T>
-__device__ __forceinline__ void prolongcoarse_el(const size_t l, T* __restrict__ xc, const T* __restrict__ from,
-                                                 const uint8_t* __restrict__ act, const STopo& t, float boost) {
-    int n0 = t.g.nc(0), n1 = t.g.nc(1), n2 = t.g.nc(2);
-    if (l >= (size_t)n0 * n1 * n2) return;
-    int I, J, K;
-    unlin(l, n0, n1, I, J, K);
-    if (act[l] != 0 && !covered(t, I, J, K)) xc[l] = sf<T>(lf(xc[l]) + boost * lf(from[l]));
-}
-// Four cells of an x row a thread (two level-1 parents); a workgroup's 1024 cells lie in
-// one slot, so the slot's place is uniform.
-template <class T>
-__device__ __forceinline__ void prolong10_wg(const uint32_t tile, T* __restrict__ x0f, const T* __restrict__ x1f,
-                                             const uint8_t* __restrict__ tf, const STopo& t, float boost, int32_t nf) {
-    int32_t n = (int32_t)(tile * 1024u) + 4 * (int32_t)threadIdx.x;
-    if ((int32_t)(tile * 1024u) >= nf) return;
-    int s = (int)((tile * 1024u) >> 12) + 1, c = n & 4095;
-    if (t.where[s - 1].x < 0) return;
-    int i = c & 15, j = (c >> 4) & 15, k = c >> 8;
-    uchar4 ty = *reinterpret_cast<const uchar4*>(tf + n);
-    if (ty.x != LIQUID && ty.y != LIQUID && ty.z != LIQUID && ty.w != LIQUID) return;
-    const T* par = x1f + (size_t)(s - 1) * SBCELLS1 + (i >> 1) + 8 * ((j >> 1) + 8 * (k >> 1));
-    float p0 = boost * lf(par[0]), p1 = boost * lf(par[1]);
-    T* xo = x0f + n;
-    if (ty.x == LIQUID) xo[0] = sf<T>(lf(xo[0]) + p0);
-    if (ty.y == LIQUID) xo[1] = sf<T>(lf(xo[1]) + p0);
-    if (ty.z == LIQUID) xo[2] = sf<T>(lf(xo[2]) + p1);
-    if (ty.w == LIQUID) xo[3] = sf<T>(lf(xo[3]) + p1);
-}
 
 // Conversions between the Krylov vectors (FP32) and the reduced-precision hierarchy:
 // y = x * mult * scal[slot] (or * mult when slot < 0), over the fine and the coarse range,
 // four values a thread (both parts are multiples of 4 long).
 template <class Y, class X>
 __global__ void k_convert(Y* __restrict__ yf, const X* __restrict__ xf, size_t nf, Y* __restrict__ yc, const X* __restrict__ xc,
-                          size_t nc, const double* __restrict__ scal, int slot, int invert) {
-    const float c = slot_scale(scal, slot, invert != 0);
+                          size_t nc, const double* __restrict__ scal, int slot) {
+    const float c = slot_scale(scal, slot, false);
     size_t nf4 = nf / 4, ng = nf4 + nc / 4;
     for (size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x; g < ng; g += (size_t)gridDim.x * blockDim.x) {
         const Four<X>* xs = g < nf4 ? reinterpret_cast<const Four<X>*>(xf) + g : reinterpret_cast<const Four<X>*>(xc) + (g - nf4);
@@ -2059,7 +2004,7 @@ struct SparseSolver {
     template <class T> void zero_t(SVecT<T> v, size_t nfine) { zero_t(v.f, nfine); zero_t(v.c, Cc); }
     void zero(SVec v, size_t nfine) { zero_t(SVecT<float>{v.f, v.c}, nfine); }
 
-    // One composite-level pass (MODE 0 Jacobi, 1 residual, 2 apply, ...) over the fine part
+    // One composite-level pass (MODE 0 Jacobi, 2 apply, ...) over the fine part
     // (N^3 a slot) and the coarse part, in one launch.
     template <int N, int MODE, class T, class C, class X>
     void rows(SVecT<T> out, SVecT<X> x, SVecT<T> b, const CompT<C>& L, RowArgs<T> S = RowArgs<T>{}) {
@@ -2104,14 +2049,6 @@ struct SparseSolver {
             rows<N, 0>(tmp, x, b, L);
             rows<N, 0>(x, tmp, b, L);
         }
-    }
-    // The same from level 1's x = 0: the first sweep reads no x, and x needs no clearing
-    // (every cell of the level's slots and coarse part is written).
-    template <class T, class C> void smooth1(Hier<T, C>& H, int sweeps) {
-        if (sweeps < 1) { zero_t(H.X1x, (size_t)s.nslots * SBCELLS1); return; }
-        rows<8, 3>(H.X1t, H.X1x, H.X1b, H.L1);
-        rows<8, 0>(H.X1x, H.X1t, H.X1b, H.L1);
-        smooth<8>(H.X1x, H.X1b, H.X1t, H.L1, sweeps - 1);
     }
     // Level 0's first sweep from zero into H.tmp. In reduced precision it takes r in FP32 and
     // writes its copy b = r / scal[nslot] for the rest of the V-cycle.
@@ -2178,7 +2115,6 @@ struct SparseSolver {
     template <class T, class C> void dense_down(Hier<T, C>& H, int l, int sweeps) {
         SLevel &Dl = s.D[l], &Cn = s.D[l + 1];
         size_t c = Dl.cells();
-        if (sweeps < 1) zero_t(H.Dx[l], c);
         for (int k = 0; k < sweeps; ++k) {   // from x = 0: the first sweep reads no x
             if (k == 0)
                 hipLaunchKernelGGL((k_rowdense<3, T, C>), dim3(cdiv(c, 256)), dim3(256), 0, st, H.Dt[l], H.Dx[l], H.Db[l], H.D[l]);
@@ -2200,43 +2136,30 @@ struct SparseSolver {
         }
     }
 
-    // sflip.jl:1722-1762 vcycle!: z = M^-1 b in the hierarchy H (coarsest in arithmetic A).
-    // In reduced precision b is the copy of r that the head makes (already made if `queued`;
-    // without sweeps the caller's).
+    // sflip.jl:1722-1762 vcycle!: z = M^-1 b in the hierarchy H (coarsest in arithmetic A),
+    // with at least one pair of sweeps a side. In reduced precision b is the copy of r that
+    // the head makes (already made if `queued`). The sweeps from zero read no x, and x needs
+    // no clearing: every cell of a level's slots and coarse part is written.
     template <class T, class C, class A>
     void vcycle_t(Hier<T, C>& H, SVecT<T> z, SVecT<T> b, SVec r, int nslot, int sweeps, int coarse, float boost, bool queued) {
-        const int ns = s.nslots;
-        if (sweeps < 1) {
-            zero_t(z, (size_t)nf);
-        } else {
-            if (!queued) head0(H, z, b, r, nslot);
-            rows<16, 0>(z, H.tmp, b, H.L0);
-            smooth<16>(z, b, H.tmp, H.L0, sweeps - 1);
-        }
+        if (!queued) head0(H, z, b, r, nslot);
+        rows<16, 0>(z, H.tmp, b, H.L0);
+        smooth<16>(z, b, H.tmp, H.L0, sweeps - 1);
         rows<16, 7>(H.X1b, z, b, H.L0);   // the residual, restricted
-        smooth1(H, sweeps);
+        rows<8, 3>(H.X1t, H.X1x, H.X1b, H.L1);
+        rows<8, 0>(H.X1x, H.X1t, H.X1b, H.L1);
+        smooth<8>(H.X1x, H.X1b, H.X1t, H.L1, sweeps - 1);
         rows<8, 7>(SVecT<T>{H.Db[0], H.Db[0]}, H.X1x, H.X1b, H.L1);
-        T* x2 = dense_levels<T, C, A>(H, sweeps, coarse, boost);
-        SLevel& D2 = s.D[0];
-        const uint32_t ncb = (uint32_t)cdiv(Cc, 256);
-        if (sweeps < 1) {   // the prolongations by themselves
-            const uint32_t nfb1 = (uint32_t)cdiv((size_t)ns * SBCELLS1, 256), nfb0 = (uint32_t)cdiv((size_t)nf, 1024);
-            hipLaunchKernelGGL((k_prolongcomp<T, 1>), dim3(nfb1 + ncb), dim3(256), 0, st, H.X1x.f, x2, s.act1.p, H.X1x.c, x2,
-                               D2.act.p, t, boost, ns, nfb1);
-            hipLaunchKernelGGL((k_prolongcomp<T, 0>), dim3(nfb0 + ncb), dim3(256), 0, st, z.f, H.X1x.f, s.types.fine.p, z.c,
-                               H.X1x.c, D2.act.p, t, boost, nf, nfb0);
-        } else {            // in the first sweep after each
-            RowArgs<T> S;
-            S.boost = boost;
-            S.yf = x2; S.yc = x2;
-            rows<8, 8>(H.X1t, H.X1x, H.X1b, H.L1, S);
-            rows<8, 0>(H.X1x, H.X1t, H.X1b, H.L1);
-            smooth<8>(H.X1x, H.X1b, H.X1t, H.L1, sweeps - 1);
-            S.yf = H.X1x.f; S.yc = H.X1x.c;
-            rows<16, 8>(H.tmp, z, b, H.L0, S);
-            rows<16, 0>(z, H.tmp, b, H.L0);
-            smooth<16>(z, b, H.tmp, H.L0, sweeps - 1);
-        }
+        RowArgs<T> S;   // the prolongations, in the first sweep after each
+        S.boost = boost;
+        S.yf = S.yc = dense_levels<T, C, A>(H, sweeps, coarse, boost);
+        rows<8, 8>(H.X1t, H.X1x, H.X1b, H.L1, S);
+        rows<8, 0>(H.X1x, H.X1t, H.X1b, H.L1);
+        smooth<8>(H.X1x, H.X1b, H.X1t, H.L1, sweeps - 1);
+        S.yf = H.X1x.f; S.yc = H.X1x.c;
+        rows<16, 8>(H.tmp, z, b, H.L0, S);
+        rows<16, 0>(z, H.tmp, b, H.L0);
+        smooth<16>(z, b, H.tmp, H.L0, sweeps - 1);
         MAEL_LAUNCH_CHECK();
     }
 
@@ -2252,8 +2175,7 @@ struct SparseSolver {
     // `head`, and the V-cycle then runs whole (overwriting what the queued launch wrote, all
     // of it V-cycle scratch).
     bool head = false;
-    void queue_head(SVec z, SVec r, int sweeps, int nslot) {
-        if (sweeps < 1) return;
+    void queue_head(SVec z, SVec r, int nslot) {
         if (precision == 0) {
             Hier<float, float> H = hier32();
             head0(H, SVecT<float>{z.f, z.c}, SVecT<float>{r.f, r.c}, r, -1);
@@ -2289,16 +2211,13 @@ struct SparseSolver {
         MPStore& m = s.mp;
         SVecT<T> zh{(T*)m.z[0].p, (T*)m.z[1].p}, rh{(T*)m.r[0].p, (T*)m.r[1].p};
         unsigned g = std::min<unsigned>(cdiv((size_t)nf + Cc, 256), 8192);
-        if (sweeps < 1)
-            hipLaunchKernelGGL((k_convert<T, float>), dim3(g), dim3(256), 0, st, rh.f, r.f, (size_t)nf, rh.c, r.c, Cc, s.scal.p,
-                               nslot, 1);
         vcycle_t<T, T, double>(H, zh, rh, r, nslot, sweeps, coarse, boost, queued);
         if (rold)   // z stays where it is: the dots and the next search convert it
             hipLaunchKernelGGL((k_sdot2h<T>), dim3(DOT_BLOCKS), dim3(256), 0, st, s.partials.p, zh.f, zh.c, r.f, r.c, rold->f,
                                rold->c, s.types.fine.p, s.types.coarse.p, s.cmask.p, t, nf, s.scal.p, nslot);
         else
             hipLaunchKernelGGL((k_convert<float, T>), dim3(g), dim3(256), 0, st, z.f, zh.f, (size_t)nf, z.c, zh.c, Cc, s.scal.p,
-                               nslot, 0);
+                               nslot);
     }
 
     void apply(SVec q, SVec x) {
@@ -2458,7 +2377,7 @@ struct SparseSolver {
                 raise_flags((long long)flags);
             } else {
                 // the next V-cycle's head runs during the read
-                if (it < maxiter) queue_head(z, r, sweeps, SS_RNORM);
+                if (it < maxiter) queue_head(z, r, SS_RNORM);
                 wait_read2(SS_RNORM, rnorm, flags);
                 if (flags != 0.0) head = false;
                 raise_flags((long long)flags);
@@ -2594,7 +2513,7 @@ void SparseBasin::precondition(const SparseOpts& o, bool queued) {
     SVec bv = S.vec(b), rv = S.vec(r), z = S.vec(P);
     S.copy(rv, bv);
     S.dot(rv, rv, SF_NORM, SS_RNORM);
-    if (queued) S.queue_head(z, rv, o.sweeps, SS_RNORM);
+    if (queued) S.queue_head(z, rv, SS_RNORM);
     S.vcycle(z, rv, o.sweeps, o.coarse, o.boost, SS_RNORM);
     MAEL_LAUNCH_CHECK();
     st.sync();

@@ -365,6 +365,31 @@ def test_vcycle_matches_oracle(M, precision):
     assert err < VCYCLE_BAR[precision], err
 
 
+@pytest.mark.parametrize("precision,sweeps", [(0, 2), (1, 2), (2, 3)])
+def test_vcycle_sweeps(M, precision, sweeps):
+    """The composite V-cycle with several pairs of sweeps, the first of which after a
+    prolongation takes it in."""
+    from maelstrom_amd import _lib as L
+    print("case: sparse vcycle precision %d sweeps %d" % (precision, sweeps), flush=True)
+    o = _scene()
+    s = _upload(M, o)
+    ns = o.nslots
+    rng = np.random.default_rng(22)
+    tf, tc = _fine(o, "types_f", BCELLS), o.array("types_c")
+    rf = np.where(tf == 1, rng.normal(0, 1, tf.size), 0).astype(np.float32)
+    rc = np.where(tc == 1, rng.normal(0, 1, tc.size), 0).astype(np.float32)
+    s.set("RHS_F", rf)
+    s.set("RHS_C", rc)
+    opts = M.sparse.solve_options(precision=precision, boost=1.0, sweeps=sweeps)
+    s.ctx.check(L.lib().mael_sparse_vcycle(s.h, C.byref(opts), 0))
+    got = np.concatenate([s.get("P_F"), s.get("P_C").ravel()])
+    zf, zc = o.vcycle(np.concatenate([rf, np.zeros(o.array("P_f").size - rf.size, np.float32)]), rc, sweeps=sweeps,
+                      coarse=opts.coarse, boost=1.0)
+    err = rel_l2(got, np.concatenate([zf[:ns * BCELLS], zc]))
+    print("rel L2 vs FP64 oracle %.3e" % err, flush=True)
+    assert err < VCYCLE_BAR[precision], err
+
+
 @pytest.mark.parametrize("precision,refine", [(1, 0), (2, 0), (0, 10), (1, 10), (2, 10)])
 def test_project_mixed_precision(M, precision, refine):
     """The FP16 / BF16 hierarchy (FP32 CG, FP64 sums and coarsest solve), with and without
