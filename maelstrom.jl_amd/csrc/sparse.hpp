@@ -383,7 +383,7 @@ struct MPStore {
     DBuf<uint16_t> z[2], r[2], tmp[2];              // fine pool, coarse
     DBuf<uint16_t> X1[3][2];                        // level-1 x, b, t
     std::vector<std::array<DBuf<uint16_t>, 3>> Dv;  // dense levels: x, b, t
-    DBuf<uint16_t> cc[3], c1[3], dDf, dDc, dD1;   // level 0's couplings follow from the types
+    DBuf<uint16_t> c1[3], dDf, dDc, dD1;          // level 0's couplings follow from the types
     DBuf<uint16_t> rwf;                             // level 0's omega / diag (the Jacobi weights)
     std::vector<std::array<DBuf<uint16_t>, 4>> Dc;  // dense levels: couplings x, y, z, diagonal
 };
@@ -457,6 +457,7 @@ struct SparseBasin {
     DBuf<float> c1[3], dD1;                   // level 1 (8^3 a block)
     DBuf<uint8_t> act1;
     DBuf<uint8_t> cmask;                      // coarse cells' cover masks (k_covermask), per solve
+    DBuf<uint16_t> crow;                      // the same with their rows' couplings
     SField<float> X1x, X1b, X1t;              // level-1 vectors (fine 512 a slot, coarse part)
     std::vector<SLevel> D;                    // D[0] = the coarse grid as level 2, then halvings
     std::vector<SField<float>> V, Z;          // FGMRES bases, allocated on first use
