@@ -642,7 +642,16 @@ template <class T> __device__ inline void store4_nt(T* __restrict__ p, uint32_t 
         __builtin_nontemporal_store(w, reinterpret_cast<U4*>(p + i));
     }
 }
-constexpr int RS = 24, PS = 18 * RS;   // LDS rows of 24: cell li (-1..16) at 4 + li; planes of 18 rows
+// LDS rows of the 16 cells (four lanes' quads of a row and the next row's follow each other:
+// no bank conflicts), planes of 18 rows; the cells beyond a row's ends lie apart, two a row.
+constexpr int RS = 16, PS = 18 * RS;
+// lane i's value from lane i - 1 (i + 1), within 16 lanes
+__device__ inline float lane_below(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x111, 0xf, 0xf, true));
+}
+__device__ inline float lane_above(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x101, 0xf, 0xf, true));
+}
 // NQ: quads a thread (a workgroup takes 4 NQ planes of its slot, its 16 / (4 NQ) tiles
 // cover the slot); more cells a workgroup keep more loads in flight.
 template <int MODE, class T, class C, int NQ = 1, class X = T>
@@ -661,8 +670,8 @@ __device__ __forceinline__ void rowfine16_wg(const uint32_t tile, T* __restrict_
     static_assert(NQ == 1 || NQ == 2, "a tile is 4 or 8 planes");
     __shared__ float4 sw4[NW ? HV / 4 : 1];    // the couplings
     __shared__ float4 sp4[Z ? 1 : HV / 4];     // coupling times x
+    __shared__ float swx[NW ? 32 * PL : 1], spx[Z ? 1 : 32 * PL];   // of the x sides
     __shared__ double lds[4];
-    float* sw = reinterpret_cast<float*>(sw4);
     float* sp = reinterpret_cast<float*>(sp4);
     const int s = (int)(tile / TPS) + 1, k0 = (int)(tile % TPS) * PL;
     const uint32_t cb = (uint32_t)(s - 1) * 4096u;
@@ -765,7 +774,7 @@ __device__ __forceinline__ void rowfine16_wg(const uint32_t tile, T* __restrict_
             w0[q][e] = ((tq[q] >> (8 * e)) & 0xffu) == LIQUID ? FINE_FINE : 0.0f;
             p0[q][e] = w0[q][e] > 0.0f ? w0[q][e] * x0[q][e] : 0.0f;
         }
-        const int hq = 4 + 4 * i4 + RS * (j + 1) + PS * (kk + 4 * q + 1);   // LDS place of its first cell
+        const int hq = 4 * i4 + RS * (j + 1) + PS * (kk + 4 * q + 1);   // LDS place of its first cell
         if constexpr (NW) sw4[hq >> 2] = make_float4(w0[q][0], w0[q][1], w0[q][2], w0[q][3]);
         if constexpr (!Z) sp4[hq >> 2] = make_float4(p0[q][0], p0[q][1], p0[q][2], p0[q][3]);
     }
@@ -813,13 +822,13 @@ __device__ __forceinline__ void rowfine16_wg(const uint32_t tile, T* __restrict_
     if (tid < 128) {   // the z layers below and above the tile: 2 x 16 rows x 4 quads
         int top = tid >> 6, lj = (tid >> 2) & 15, q = tid & 3;
         int lk = top ? k0 + PL : k0 - 1;
-        stage4(4 * q, lj, lk, top ? nb[5] : nb[4], 4 + 4 * q + RS * (lj + 1) + PS * (top ? PL + 1 : 0));
+        stage4(4 * q, lj, lk, top ? nb[5] : nb[4], 4 * q + RS * (lj + 1) + PS * (top ? PL + 1 : 0));
     } else {           // the x sides: 2 x 16 rows x PL planes, one cell each
 #pragma unroll
         for (int r = 0; r < NQ; ++r) {
             int e = tid - 128 + 128 * r, side = e & 1, lj = (e >> 1) & 15, p = e >> 5;
             int li = side ? 16 : -1, lk = k0 + p;
-            int h = 4 + li + RS * (lj + 1) + PS * (p + 1);
+            int h = side + 2 * (lj + 16 * p);
             int32_t sn = side ? nb[1] : nb[0];
             float wv, pv;
             if (sn != 0) {
@@ -831,14 +840,14 @@ __device__ __forceinline__ void rowfine16_wg(const uint32_t tile, T* __restrict_
             } else {
                 coarse(li, lj, lk, wv, pv);
             }
-            if constexpr (NW) sw[h] = wv;
-            if constexpr (!Z) sp[h] = pv;
+            if constexpr (NW) swx[h] = wv;
+            if constexpr (!Z) spx[h] = pv;
         }
     }
     if (tid < 32 * NQ) {   // the y sides: 2 x PL planes x 4 quads
         int side = tid & 1, q = (tid >> 1) & 3, p = tid >> 3;
         int lj = side ? 16 : -1;
-        stage4(4 * q, lj, k0 + p, side ? nb[3] : nb[2], 4 + 4 * q + RS * (lj + 1) + PS * (p + 1));
+        stage4(4 * q, lj, k0 + p, side ? nb[3] : nb[2], 4 * q + RS * (lj + 1) + PS * (p + 1));
     }
     __syncthreads();
 
@@ -846,20 +855,26 @@ __device__ __forceinline__ void rowfine16_wg(const uint32_t tile, T* __restrict_
     Four<T> res4[RESTRICT ? NQ : 1];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-        const int hq = 4 + 4 * i4 + RS * (j + 1) + PS * (kk + 4 * q + 1);
-        // the neighbours' couplings and products: x within the quad from registers, the
-        // quad's x ends, y and z from LDS; order -x, +x, -y, +y, -z, +z
+        const int hq = 4 * i4 + RS * (j + 1) + PS * (kk + 4 * q + 1);
+        // the neighbours' couplings and products: x within the quad from registers, across
+        // its ends from the next lanes (at a row's ends from LDS), y and z from LDS; order
+        // -x, +x, -y, +y, -z, +z
+        const int hx = (i4 == 3) + 2 * (j + 16 * (kk + 4 * q));   // (the lanes between read one too)
         float4 wym = make_float4(0, 0, 0, 0), wyp = wym, wzm = wym, wzp = wym;
         float wl = 0.0f, wr = 0.0f;
         if constexpr (NW) {
             wym = sw4[(hq - RS) >> 2]; wyp = sw4[(hq + RS) >> 2]; wzm = sw4[(hq - PS) >> 2]; wzp = sw4[(hq + PS) >> 2];
-            wl = sw[hq - 1]; wr = sw[hq + 4];
+            const float we = swx[hx], wb = lane_below(w0[q][3]), wa = lane_above(w0[q][0]);
+            wl = i4 == 0 ? we : wb;
+            wr = i4 == 3 ? we : wa;
         }
         float4 pym = make_float4(0, 0, 0, 0), pyp = pym, pzm = pym, pzp = pym;
         float pl = 0.0f, pr = 0.0f;
         if constexpr (!Z) {
             pym = sp4[(hq - RS) >> 2]; pyp = sp4[(hq + RS) >> 2]; pzm = sp4[(hq - PS) >> 2]; pzp = sp4[(hq + PS) >> 2];
-            pl = sp[hq - 1]; pr = sp[hq + 4];
+            const float pe = spx[hx], pb = lane_below(p0[q][3]), pa = lane_above(p0[q][0]);
+            pl = i4 == 0 ? pe : pb;
+            pr = i4 == 3 ? pe : pa;
         }
         const float wy0[4] = {wym.x, wym.y, wym.z, wym.w}, wy1[4] = {wyp.x, wyp.y, wyp.z, wyp.w};
         const float wz0[4] = {wzm.x, wzm.y, wzm.z, wzm.w}, wz1[4] = {wzp.x, wzp.y, wzp.z, wzp.w};
@@ -1172,15 +1187,26 @@ __global__ __launch_bounds__(256) void k_rowcoarse(T* __restrict__ out, const X*
 // overlap the fine tiles (bandwidth-bound) and the pass drains once. Workgroup g takes
 // coarse block floor(g C / G) when that count steps at g, else fine workgroup g minus
 // the coarse blocks before it: each index of either part is taken exactly once, in order.
+// The host makes `share` = ceil(2^32 C / G), so the count is floor(g share / 2^32): it is C
+// at G and steps by at most one as long as C < G (a 64-bit division here took every
+// wavefront some hundred scalar instructions).
+inline uint32_t coarse_share(uint32_t ncb, uint32_t G) {
+    return (uint32_t)((((uint64_t)ncb << 32) + G - 1) / G);
+}
+struct Place { uint32_t index; bool coarse; };
+__device__ inline Place place_of(uint32_t share) {
+    const uint32_t g = xcd_tile(blockIdx.x, gridDim.x);
+    const uint32_t c0 = __umulhi(g, share), c1 = (uint32_t)(((uint64_t)g * share + share) >> 32);
+    return c1 > c0 ? Place{c0, true} : Place{g - c0, false};
+}
 template <int N, int MODE, class T, class C, int NQ, class X>
 __global__ __launch_bounds__(256) void k_rowcomp(T* __restrict__ outf, T* __restrict__ outc, const X* __restrict__ xf,
                                                  const X* __restrict__ xc, const T* __restrict__ bf,
-                                                 const T* __restrict__ bc, CompT<C> L, STopo t, RowArgs<T> S, uint32_t ncb) {
-    const uint32_t G = gridDim.x, g = xcd_tile(blockIdx.x, G);
-    const uint32_t c0 = (uint32_t)(((uint64_t)g * ncb) / G), c1 = (uint32_t)(((uint64_t)(g + 1) * ncb) / G);
-    if (c1 > c0) rowcoarse_wg<N, MODE, T, C, X>(c0, c0, outc, xc, bc, xf, L, t, S);
-    else if constexpr (N == 16) rowfine16_wg<MODE, T, C, NQ, X>(g - c0, outf, xf, bf, xc, L, t, S);
-    else rowfine8_wg<MODE, T, C>(g - c0, outf, xf, bf, xc, L, t, S);
+                                                 const T* __restrict__ bc, CompT<C> L, STopo t, RowArgs<T> S, uint32_t share) {
+    const Place at = place_of(share);
+    if (at.coarse) rowcoarse_wg<N, MODE, T, C, X>(at.index, at.index, outc, xc, bc, xf, L, t, S);
+    else if constexpr (N == 16) rowfine16_wg<MODE, T, C, NQ, X>(at.index, outf, xf, bf, xc, L, t, S);
+    else rowfine8_wg<MODE, T, C>(at.index, outf, xf, bf, xc, L, t, S);
 }
 // The reduced-precision V-cycle's entry as one launch in the same interleave: level 0's
 // fine part through jacobi0w_cvt_wg (r converted and stored, the sweep from zero) and the
@@ -1188,12 +1214,11 @@ __global__ __launch_bounds__(256) void k_rowcomp(T* __restrict__ outf, T* __rest
 template <class T>
 __global__ __launch_bounds__(256) void k_head0(T* __restrict__ outf, T* __restrict__ outc, T* __restrict__ bh,
                                                const float* __restrict__ r, CompT<T> L, STopo t, int32_t nf, RowArgs<T> S,
-                                               uint32_t ncb) {
-    const uint32_t G = gridDim.x, g = xcd_tile(blockIdx.x, G);
-    const uint32_t c0 = (uint32_t)(((uint64_t)g * ncb) / G), c1 = (uint32_t)(((uint64_t)(g + 1) * ncb) / G);
+                                               uint32_t share) {
+    const Place at = place_of(share);
     const T* none = nullptr;
-    if (c1 > c0) rowcoarse_wg<16, 10, T, T>(c0, c0, outc, none, none, none, L, t, S);
-    else jacobi0w_cvt_wg<T>(g - c0, outf, bh, r, L.rwf, L.actf, t.where, nf, S.scal, S.zslot);
+    if (at.coarse) rowcoarse_wg<16, 10, T, T>(at.index, at.index, outc, none, none, none, L, t, S);
+    else jacobi0w_cvt_wg<T>(at.index, outf, bh, r, L.rwf, L.actf, t.where, nf, S.scal, S.zslot);
 }
 
 // ─── dense levels (sflip.jl:1574-1657) ───────────────────────────────────────
@@ -2033,7 +2058,7 @@ struct SparseSolver {
             constexpr int NQ = N == 16 ? 2 : 1;   // 8-plane tiles
             const uint32_t nfw = N == 16 ? (uint32_t)s.nslots * (uint32_t)(4 / NQ) : (uint32_t)s.nslots;
             hipLaunchKernelGGL((k_rowcomp<N, MODE, T, C, NQ, X>), dim3(nfw + ncb), dim3(256), 0, st, out.f, out.c, x.f, x.c, b.f,
-                               b.c, L, t, S, ncb);
+                               b.c, L, t, S, coarse_share(ncb, nfw + ncb));
         } else {
             if (MODE == 4) fill_async(S.partials, (size_t)1, 0.0, st);   // no fine workgroups: the finish reads one zero
             hipLaunchKernelGGL((k_rowcoarse<N, MODE, T, C, X>), dim3(ncb), dim3(256), 0, st, out.c, x.c, b.c, x.f, L, t, S);
@@ -2077,7 +2102,11 @@ struct SparseSolver {
             RowArgs<T> S;
             S.rc = r.c; S.bc = b.c; S.scal = s.scal.p; S.zslot = nslot;
             const uint32_t ncb = (uint32_t)cdiv(Cc, 256), nfw = (uint32_t)s.nslots * 4u;   // 1024 fine cells a workgroup
-            hipLaunchKernelGGL((k_head0<T>), dim3(nfw + ncb), dim3(256), 0, st, H.tmp.f, H.tmp.c, b.f, r.f, H.L0, t, nf, S, ncb);
+            if (nfw)
+                hipLaunchKernelGGL((k_head0<T>), dim3(nfw + ncb), dim3(256), 0, st, H.tmp.f, H.tmp.c, b.f, r.f, H.L0, t, nf, S,
+                                   coarse_share(ncb, nfw + ncb));
+            else
+                hipLaunchKernelGGL((k_rowcoarse<16, 10, T, C, T>), dim3(ncb), dim3(256), 0, st, H.tmp.c, z.c, b.c, z.f, H.L0, t, S);
         }
     }
 
