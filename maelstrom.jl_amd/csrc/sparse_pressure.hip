@@ -1134,7 +1134,9 @@ __device__ __forceinline__ void rowcoarse_wg(const uint32_t cb, const uint32_t p
         S.dnc[l] = xl;
     }
     if constexpr (MODE == 10) {
-        const T bt = sf<T>(S.rc[l] * rs);
+        float r = S.rc[l] * rs;
+        asm("" : "+v"(r));   // rounded to FP32 first (not one rounding to FP16 with the product)
+        const T bt = sf<T>(r);
         S.bc[l] = bt;
         bl = lf(bt);
     }
