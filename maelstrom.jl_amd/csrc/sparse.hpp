@@ -364,6 +364,13 @@ __device__ inline void stage27(const STopo& t, int4 w, int32_t* s27) {
     }
 }
 
+// The kernels that go over a slot's 17 x 256 faces take them in one workgroup's 17 rounds
+// (a number the compiler knows: their template parameter) while those workgroups fill half
+// of the chip's 2048 places (8 a CU), else a workgroup a round. 60 cm, 120 slots: a
+// projection's difference 17 us with one workgroup a slot, 4 with 17.
+constexpr int SLOT_ROUNDS = 17;
+inline bool slots_few(int groups) { return groups <= 1024; }
+
 // sflip.jl:1030-1031 walledface: a wall on either side of the face at p (cells h wide).
 __device__ inline bool walledface_dev(const SGrid& g, const float p[3], int a, float h) {
     float e = 0.5f * h;

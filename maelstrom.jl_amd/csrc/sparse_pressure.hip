@@ -79,12 +79,15 @@ struct SlotFaces {
     }
 };
 
-// A workgroup per live slot (block order), a thread per 17 of its faces along a.
+// A workgroup (or one a round, slots_few) per live slot (block order): 256 of its faces along
+// a a round.
+template <int ROUNDS>
 __global__ __launch_bounds__(256) void k_finecoef(float* __restrict__ c, const uint8_t* __restrict__ tf,
                                                   const uint8_t* __restrict__ tc, STopo t, int a,
                                                   const int32_t* __restrict__ order) {
     const SlotFaces F(t, order[blockIdx.x], a);
-    for (int r = 0; r < SBFACES / 256; ++r) {
+    for (int q = 0; q < ROUNDS; ++q) {
+        const int r = ROUNDS == 1 ? (int)blockIdx.y : q;
         const int f = r * 256 + (int)threadIdx.x;
         int i, j, k;
         F.face(f, i, j, k);
@@ -1640,13 +1643,13 @@ __device__ inline float pdiff(double a, double b) { return (float)(a - b); }
 __device__ inline float pdiv(float a, float b) { return __fdiv_rn(a, b); }
 __device__ inline float pdiv(double a, float b) { return (float)(a / (double)b); }
 
-template <class PT>
+template <class PT, int ROUNDS>
 __global__ __launch_bounds__(256) void k_projectfine(float* __restrict__ u, uint8_t* __restrict__ valid,
                                                      const PT* __restrict__ P, const PT* __restrict__ Pc,
                                                      const uint8_t* __restrict__ tf, const uint8_t* __restrict__ tc,
                                                      const float* __restrict__ phi, const float* __restrict__ phic, STopo t, int a,
                                                      const int32_t* __restrict__ order) {
-    // a workgroup per live slot (block order), a thread per 17 of its faces along a: a
+    // a workgroup (or one a round, slots_few) per live slot (block order), 256 of its faces along a a round: a
     // face's two cells lie in the slot's block or in the blocks below and above it along
     // a, looked up once (fineat's index, or -1 where there is no block)
     const int s = order[blockIdx.x];
@@ -1671,7 +1674,8 @@ __global__ __launch_bounds__(256) void k_projectfine(float* __restrict__ u, uint
     auto coarsei = [&](int I, int J, int K) -> size_t {   // fineorcoarse's clamped coarse cell
         return cl(min(max(I >> 2, 0), n0 - 1), min(max(J >> 2, 0), n1 - 1), min(max(K >> 2, 0), n2 - 1), n0, n1);
     };
-    for (int r = 0; r < SBFACES / 256; ++r) {
+    for (int q = 0; q < ROUNDS; ++q) {
+        const int r = ROUNDS == 1 ? (int)blockIdx.y : q;
         const int f = r * 256 + (int)threadIdx.x;
         int i, j, k;
         if (a == 0) { i = f % 17; int q = f / 17; j = q & 15; k = q >> 4; }
@@ -1920,7 +1924,8 @@ struct SparseSolver {
     void coefficients() {
         for (int a = 0; a < 3; ++a) {
             if (s.nlive > 0)
-                hipLaunchKernelGGL(k_finecoef, dim3((unsigned)s.nlive), dim3(256), 0, st, s.cf[a].p, s.types.fine.p,
+                hipLaunchKernelGGL(slots_few(s.nlive) ? k_finecoef<1> : k_finecoef<SLOT_ROUNDS>,
+                                   dim3((unsigned)s.nlive, slots_few(s.nlive) ? SLOT_ROUNDS : 1), dim3(256), 0, st, s.cf[a].p, s.types.fine.p,
                                    s.types.coarse.p, t, a, s.sorder.p);
             hipLaunchKernelGGL(k_coarsecoef, dim3(cdiv(s.nfaces(a), 256)), dim3(256), 0, st, s.cc[a].p, s.types.coarse.p, t, a);
         }
@@ -2641,11 +2646,13 @@ void SparseBasin::project(float gamma, const SparseOpts& o, SparseStats& stats) 
     for (int a = 0; a < 3; ++a) {
         if (S.nf && nlive > 0) {
             if (o.refine > 0)
-                hipLaunchKernelGGL(k_projectfine<double>, dim3((unsigned)nlive), dim3(256), 0, s, u[a].fine.p, fl[a].fine.p,
+                hipLaunchKernelGGL((slots_few(nlive) ? k_projectfine<double, 1> : k_projectfine<double, SLOT_ROUNDS>),
+                                   dim3((unsigned)nlive, slots_few(nlive) ? SLOT_ROUNDS : 1), dim3(256), 0, s, u[a].fine.p, fl[a].fine.p,
                                    Pd.fine.p, Pd.coarse.p, types.fine.p, types.coarse.p, phi.fine.p, phi.coarse.p, t, a,
                                    sorder.p);
             else
-                hipLaunchKernelGGL(k_projectfine<float>, dim3((unsigned)nlive), dim3(256), 0, s, u[a].fine.p, fl[a].fine.p,
+                hipLaunchKernelGGL((slots_few(nlive) ? k_projectfine<float, 1> : k_projectfine<float, SLOT_ROUNDS>),
+                                   dim3((unsigned)nlive, slots_few(nlive) ? SLOT_ROUNDS : 1), dim3(256), 0, s, u[a].fine.p, fl[a].fine.p,
                                    P.fine.p, P.coarse.p, types.fine.p, types.coarse.p, phi.fine.p, phi.coarse.p, t, a,
                                    sorder.p);
         }

@@ -465,18 +465,25 @@ void SparseBasin::set_stir(const StirParams& p, const float* waves, int nwaves, 
 
 // One layer: an unflagged face takes the mean of its flagged neighbours (fine faces;
 // neighbours through finefaceat's rule, the blocks read from a table of the 27 around
-// the slot). A workgroup per live slot (block order), a thread per 17 of its faces. The
-// output arrays hold the layer before the input's (or, with `fresh`, nothing yet). A
-// flagged face keeps its value from layer to layer, and so does an unflagged one until it
-// is flagged: a face whose flag is the same in both and that takes no neighbour's mean is
-// already this layer's there and is skipped. Neighbours' values are read only where
-// flagged.
-template <int A>
-__global__ __launch_bounds__(256) void k_sextrapfine(float* __restrict__ out, uint8_t* __restrict__ fout,
-                                                     const float* __restrict__ src, const uint8_t* __restrict__ fin,
-                                                     float* __restrict__ out2, const float* __restrict__ src2, STopo t,
-                                                     int fresh, const int32_t* __restrict__ order) {
-    __shared__ int32_t s27[27];
+// the slot). A workgroup, or a workgroup a round (slots_few), per live slot (block order) and
+// axis. The output arrays hold the layer before the input's (or, with `fresh`,
+// nothing yet). A flagged face keeps its value from layer to layer, and so does an unflagged
+// one until it is flagged: a face whose flag is the same in both and that takes no
+// neighbour's mean is already this layer's there and is skipped. Neighbours' values are read
+// only where flagged.
+struct ExtrapArrays {
+    float* out[3];
+    uint8_t* fout[3];
+    const float* src[3];
+    const uint8_t* fin[3];
+    float* out2[3];         // null: no second array
+    const float* src2[3];
+};
+template <int A, int ROUNDS>
+__device__ __forceinline__ void extrapfine_wg(float* __restrict__ out, uint8_t* __restrict__ fout, const float* __restrict__ src,
+                                              const uint8_t* __restrict__ fin, float* __restrict__ out2,
+                                              const float* __restrict__ src2, const STopo& t, int fresh,
+                                              const int32_t* __restrict__ order, int32_t* s27) {
     const int s = order[blockIdx.x];   // 1-based, live
     const int4 w = t.where[s - 1];
     stage27(t, w, s27);
@@ -494,7 +501,8 @@ __global__ __launch_bounds__(256) void k_sextrapfine(float* __restrict__ out, ui
         if (s2 == 0) return -1;
         return (s2 - 1) * SBFACES + ffn(16, A, A == 0 ? 16 : (GI & 15), A == 1 ? 16 : (GJ & 15), A == 2 ? 16 : (GK & 15));
     };
-    for (int r = 0; r < SBFACES / 256; ++r) {
+    for (int q = 0; q < ROUNDS; ++q) {
+        const int r = ROUNDS == 1 ? (int)blockIdx.y : q;
         const int f = r * 256 + (int)threadIdx.x;
         const int32_t n = (s - 1) * SBFACES + f;
         const uint8_t f0 = fin[n];
@@ -521,10 +529,10 @@ __global__ __launch_bounds__(256) void k_sextrapfine(float* __restrict__ out, ui
         uint8_t nf[6];
         bool any = false;
 #pragma unroll
-        for (int q = 0; q < 6; ++q) {
-            nidx[q] = walled ? -1 : face(I + NBX[q][0], J + NBX[q][1], K + NBX[q][2]);
-            nf[q] = nidx[q] >= 0 ? fin[nidx[q]] : 0;
-            any = any || nf[q] != 0;
+        for (int m = 0; m < 6; ++m) {
+            nidx[m] = walled ? -1 : face(I + NBX[m][0], J + NBX[m][1], K + NBX[m][2]);
+            nf[m] = nidx[m] >= 0 ? fin[nidx[m]] : 0;
+            any = any || nf[m] != 0;
         }
         if (!any) {   // stays as it is
             if (fo == 0) continue;
@@ -536,10 +544,10 @@ __global__ __launch_bounds__(256) void k_sextrapfine(float* __restrict__ out, ui
         float acc = 0.0f, acc2 = 0.0f;
         int cnt = 0;
 #pragma unroll
-        for (int q = 0; q < 6; ++q)
-            if (nf[q]) {
-                acc += src[nidx[q]];
-                if (out2) acc2 += src2[nidx[q]];
+        for (int m = 0; m < 6; ++m)
+            if (nf[m]) {
+                acc += src[nidx[m]];
+                if (out2) acc2 += src2[nidx[m]];
                 ++cnt;
             }
         out[n] = __fdiv_rn(acc, (float)cnt);
@@ -547,9 +555,26 @@ __global__ __launch_bounds__(256) void k_sextrapfine(float* __restrict__ out, ui
         fout[n] = 1;
     }
 }
-__global__ void k_sextrapcoarse(float* __restrict__ out, uint8_t* __restrict__ fout, const float* __restrict__ src,
-                                const uint8_t* __restrict__ fin, float* __restrict__ out2, const float* __restrict__ src2,
-                                SGrid g, int a) {
+template <int A>   // one axis, a workgroup a slot
+__global__ __launch_bounds__(256) void k_sextrapfine(ExtrapArrays E, STopo t, int fresh, const int32_t* __restrict__ order) {
+    __shared__ int32_t s27[27];
+    extrapfine_wg<A, SLOT_ROUNDS>(E.out[A], E.fout[A], E.src[A], E.fin[A], E.out2[A], E.src2[A], t, fresh, order, s27);
+}
+// the three axes (blockIdx.z), a workgroup a round
+__global__ __launch_bounds__(256) void k_sextrapfine3(ExtrapArrays E, STopo t, int fresh, const int32_t* __restrict__ order) {
+    __shared__ int32_t s27[27];
+    if (blockIdx.z == 0) extrapfine_wg<0, 1>(E.out[0], E.fout[0], E.src[0], E.fin[0], E.out2[0], E.src2[0], t, fresh, order, s27);
+    else if (blockIdx.z == 1) extrapfine_wg<1, 1>(E.out[1], E.fout[1], E.src[1], E.fin[1], E.out2[1], E.src2[1], t, fresh, order, s27);
+    else extrapfine_wg<2, 1>(E.out[2], E.fout[2], E.src[2], E.fin[2], E.out2[2], E.src2[2], t, fresh, order, s27);
+}
+__global__ void k_sextrapcoarse(ExtrapArrays E, SGrid g) {   // an axis per blockIdx.y
+    const int a = (int)blockIdx.y;
+    float* __restrict__ out = a == 0 ? E.out[0] : (a == 1 ? E.out[1] : E.out[2]);
+    uint8_t* __restrict__ fout = a == 0 ? E.fout[0] : (a == 1 ? E.fout[1] : E.fout[2]);
+    const float* __restrict__ src = a == 0 ? E.src[0] : (a == 1 ? E.src[1] : E.src[2]);
+    const uint8_t* __restrict__ fin = a == 0 ? E.fin[0] : (a == 1 ? E.fin[1] : E.fin[2]);
+    float* __restrict__ out2 = a == 0 ? E.out2[0] : (a == 1 ? E.out2[1] : E.out2[2]);
+    const float* __restrict__ src2 = a == 0 ? E.src2[0] : (a == 1 ? E.src2[1] : E.src2[2]);
     int n0 = g.nc(0) + (a == 0), n1 = g.nc(1) + (a == 1), n2 = g.nc(2) + (a == 2);
     size_t l = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (l >= (size_t)n0 * n1 * n2) return;
@@ -624,37 +649,60 @@ void SparseBasin::extrapolate(int layers, int coarselayers, bool withkick) {
     hipStream_t s = st.s;
     STopo t = topo();
     size_t F = finefaces();
+    // the layers of one part (fine or coarse): layer 1 writes over the input of layer 0; after
+    // an odd count the results are copied back. The three axes take a launch a layer together
+    // while few slots leave the chip idle (60 cm: 32 us an axis, 7 together), else one after
+    // the other (5 cm: 318 us for the three, 370 together, where the flags of three axes pass
+    // through the caches between layers and the kernel keeps fewer wavefronts).
+    auto run = [&](auto part, size_t (*size)(const SparseBasin&, int), int count, bool together, auto launch) {
+        ExtrapArrays E;
+        for (int a = 0; a < 3; ++a) {
+            E.src[a] = part(u[a]).p; E.out[a] = part(u0[a]).p;
+            E.fin[a] = part(fl[a]).p; E.fout[a] = part(fl2[a]).p;
+            E.src2[a] = withkick ? part(ur[a]).p : nullptr; E.out2[a] = withkick ? part(ur0[a]).p : nullptr;
+        }
+        const unsigned axes = together ? 3 : 1;
+        for (int axis = 0; axis < 3; axis += (int)axes)
+            for (int l = 0; l < count; ++l) {
+                launch(E, axis, axes, l);
+                for (int a = axis; a < axis + (int)axes; ++a) {
+                    float* x = const_cast<float*>(E.src[a]); E.src[a] = E.out[a]; E.out[a] = x;
+                    float* y = const_cast<float*>(E.src2[a]); E.src2[a] = E.out2[a]; E.out2[a] = y;
+                    uint8_t* m = const_cast<uint8_t*>(E.fin[a]); E.fin[a] = E.fout[a]; E.fout[a] = m;
+                }
+            }
+        if (count & 1)
+            for (int a = 0; a < 3; ++a) {
+                const size_t N = size(*this, a);
+                MAEL_HIP(hipMemcpyAsync(part(u[a]).p, E.src[a], N * sizeof(float), hipMemcpyDeviceToDevice, s));
+                if (withkick) MAEL_HIP(hipMemcpyAsync(part(ur[a]).p, E.src2[a], N * sizeof(float), hipMemcpyDeviceToDevice, s));
+                MAEL_HIP(hipMemcpyAsync(part(fl[a]).p, E.fin[a], N, hipMemcpyDeviceToDevice, s));
+            }
+    };
+    const bool few = slots_few(nlive);
+    run([](auto& x) -> auto& { return x.fine; }, [](const SparseBasin& b, int) { return b.finefaces(); }, layers, few,
+        [&](const ExtrapArrays& E, int axis, unsigned axes, int l) {
+            if (nlive == 0) return;   // (free slots: nothing reads their faces)
+            const int fresh = l == 0 ? 1 : 0;
+            if (few) {
+                hipLaunchKernelGGL(k_sextrapfine3, dim3((unsigned)nlive, SLOT_ROUNDS, axes), dim3(256), 0, s, E, t, fresh, sorder.p);
+            } else {
+                auto kern = axis == 0 ? k_sextrapfine<0> : (axis == 1 ? k_sextrapfine<1> : k_sextrapfine<2>);
+                hipLaunchKernelGGL(kern, dim3((unsigned)nlive), dim3(256), 0, s, E, t, fresh, sorder.p);
+            }
+        });
     for (int a = 0; a < 3; ++a) {
-        float *f = u[a].fine.p, *tmp = u0[a].fine.p, *k = withkick ? ur[a].fine.p : nullptr, *ktmp = withkick ? ur0[a].fine.p : nullptr;
-        uint8_t *fin = fl[a].fine.p, *fout = fl2[a].fine.p;
-        auto kern = a == 0 ? k_sextrapfine<0> : (a == 1 ? k_sextrapfine<1> : k_sextrapfine<2>);
-        for (int l = 0; l < layers; ++l) {   // layer 1 writes over the input of layer 0
-            if (nlive > 0)   // free slots: nothing reads their faces
-                hipLaunchKernelGGL(kern, dim3((unsigned)nlive), dim3(256), 0, s, tmp, fout, f, fin, ktmp, k, t, l == 0 ? 1 : 0,
-                                   sorder.p);
-            std::swap(f, tmp); std::swap(k, ktmp); std::swap(fin, fout);
-        }
-        if (f != u[a].fine.p) {   // an odd count: copy back
-            MAEL_HIP(hipMemcpyAsync(u[a].fine.p, f, F * sizeof(float), hipMemcpyDeviceToDevice, s));
-            if (withkick) MAEL_HIP(hipMemcpyAsync(ur[a].fine.p, k, F * sizeof(float), hipMemcpyDeviceToDevice, s));
-            MAEL_HIP(hipMemcpyAsync(fl[a].fine.p, fin, F, hipMemcpyDeviceToDevice, s));
-        }
         launch_restrictfaces_f(*this, u[a].coarse.p, u[a].fine.p, a);
         if (withkick) launch_restrictfaces_f(*this, ur[a].coarse.p, ur[a].fine.p, a);
         launch_restrictfaces_u8(*this, fl[a].coarse.p, fl[a].fine.p, a);
-        size_t Fc = nfaces(a);
-        float *fc = u[a].coarse.p, *tc = u0[a].coarse.p, *kc = withkick ? ur[a].coarse.p : nullptr,
-              *ktc = withkick ? ur0[a].coarse.p : nullptr;
-        uint8_t *finc = fl[a].coarse.p, *foutc = fl2[a].coarse.p;
-        for (int l = 0; l < coarselayers; ++l) {
-            hipLaunchKernelGGL(k_sextrapcoarse, dim3(cdiv(Fc, 256)), dim3(256), 0, s, tc, foutc, fc, finc, ktc, kc, g, a);
-            std::swap(fc, tc); std::swap(kc, ktc); std::swap(finc, foutc);
-        }
-        if (fc != u[a].coarse.p) {
-            MAEL_HIP(hipMemcpyAsync(u[a].coarse.p, fc, Fc * sizeof(float), hipMemcpyDeviceToDevice, s));
-            if (withkick) MAEL_HIP(hipMemcpyAsync(ur[a].coarse.p, kc, Fc * sizeof(float), hipMemcpyDeviceToDevice, s));
-            MAEL_HIP(hipMemcpyAsync(fl[a].coarse.p, finc, Fc, hipMemcpyDeviceToDevice, s));
-        }
+    }
+    run([](auto& x) -> auto& { return x.coarse; }, [](const SparseBasin& b, int a) { return b.nfaces(a); }, coarselayers, true,
+        [&](const ExtrapArrays& E, int, unsigned axes, int) {
+            hipLaunchKernelGGL(k_sextrapcoarse, dim3(cdiv(std::max({nfaces(0), nfaces(1), nfaces(2)}), 256), axes), dim3(256), 0, s, E,
+                               g);
+        });
+    for (int a = 0; a < 3; ++a) {
+        const size_t Fc = nfaces(a);
         for (int w = 0; w < (withkick ? 2 : 1); ++w) {
             SField<float>& x = w == 0 ? u[a] : ur[a];
             if (F) hipLaunchKernelGGL(k_unreached, dim3(cdiv(F, 256)), dim3(256), 0, s, x.fine.p, fl[a].fine.p, F);

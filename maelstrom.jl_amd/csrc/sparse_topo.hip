@@ -566,11 +566,13 @@ void SparseBasin::classify() {
 
 // A workgroup per live slot (block order), a thread per 17 of its faces; a block clear of
 // the walls has no walled face and leaves at once.
+template <int ROUNDS>
 __global__ __launch_bounds__(256) void k_solidfine(float* __restrict__ u, STopo t, int a, const int32_t* __restrict__ order) {
     const int s = order[blockIdx.x];
     const int4 w = t.where[s - 1];
     if (blockclear(t.g, w)) return;
-    for (int r = 0; r < SBFACES / 256; ++r) {
+    for (int q = 0; q < ROUNDS; ++q) {
+        const int r = ROUNDS == 1 ? (int)blockIdx.y : q;
         const int f = r * 256 + (int)threadIdx.x;
         int i, j, k;
         if (a == 0) { i = f % 17; int q = f / 17; j = q & 15; k = q >> 4; }
@@ -597,7 +599,8 @@ __global__ void k_solidcoarse(float* __restrict__ u, SGrid g, int a) {
 void SparseBasin::solidify() {
     for (int a = 0; a < 3; ++a) {
         if (nlive > 0)
-            hipLaunchKernelGGL(k_solidfine, dim3((unsigned)nlive), dim3(256), 0, st.s, u[a].fine.p, topo(), a, sorder.p);
+            hipLaunchKernelGGL(slots_few(nlive) ? k_solidfine<1> : k_solidfine<SLOT_ROUNDS>,
+                               dim3((unsigned)nlive, slots_few(nlive) ? SLOT_ROUNDS : 1), dim3(256), 0, st.s, u[a].fine.p, topo(), a, sorder.p);
         hipLaunchKernelGGL(k_solidcoarse, dim3(cdiv(nfaces(a), 256)), dim3(256), 0, st.s, u[a].coarse.p, g, a);
     }
     MAEL_LAUNCH_CHECK();
@@ -637,32 +640,38 @@ void SparseBasin::gravity(float dt, float gacc) {
 
 // ─── redistancing (sflip.jl:833-919) ─────────────────────────────────────────
 
-// A workgroup per slot: the block's 16^3 values and the layers of the six blocks across
-// its sides (the coarse cell where there is no block, as in the reference's nphi) are
-// staged in LDS once, then each thread takes a 16-cell column along z. A block clear of
-// the walls skips the solid tests.
+// A workgroup per slot, or per KP of its 16 planes where the slots alone leave the chip idle
+// (up to 512 live; 120: 22 us with one, 9 with four): the block's values there and the layers across its sides
+// (the block's own planes, else the neighbour's, else the coarse cell where there is no
+// block, as in the reference's nphi) are staged in LDS once, then each thread takes a KP-cell
+// column along z. A block clear of the walls skips the solid tests.
+template <int KP>
 __global__ __launch_bounds__(256) void k_sreinit(float* __restrict__ out, const float* __restrict__ phi,
                                                  const float* __restrict__ phic, STopo t, float phimax,
                                                  const int32_t* __restrict__ order) {
     __shared__ int32_t s27[27];
-    __shared__ float tv[4096];       // the block's cells, x fastest
-    __shared__ float hv[6][256];     // neighbour m's layer at (p, q), the other two axes in order
+    __shared__ float tv[256 * KP];   // the planes' cells, x fastest
+    __shared__ float hv[6][256];     // side m's layer at (p, q), the other two axes in order
     const int32_t slot = order[blockIdx.x] - 1;   // live slots in block order
     const int4 w = t.where[slot];
     stage27(t, w, s27);
     const SGrid& g = t.g;
     const int tid = (int)threadIdx.x, ti = tid & 15, tj = tid >> 4;
-    const float* __restrict__ bp = phi + (size_t)slot * 4096;
-    float own[16];
+    const int k0 = (int)blockIdx.y * KP;   // the first plane
+    const float* __restrict__ bp = phi + (size_t)slot * 4096 + 256 * k0;
+    float own[KP];
 #pragma unroll
-    for (int k = 0; k < 16; ++k) own[k] = bp[tid + 256 * k];
+    for (int k = 0; k < KP; ++k) own[k] = bp[tid + 256 * k];
     __syncthreads();
     const int n0 = g.nc(0), n1 = g.nc(1), n2 = g.nc(2);
     float hl[6];
 #pragma unroll
     for (int m = 0; m < 6; ++m) {   // entry (p, q) = (ti, tj) of each side's layer
-        const int a = m >> 1, e = NBS[m][a] > 0 ? 16 : -1;
-        const int li = a == 0 ? e : ti, lj = a == 1 ? e : (a == 0 ? ti : tj), lk = a == 2 ? e : tj;
+        const int a = m >> 1;
+        const bool hi = NBS[m][a] > 0;
+        // (the x and y sides have KP rows)
+        const int li = a == 0 ? (hi ? 16 : -1) : ti, lj = a == 1 ? (hi ? 16 : -1) : (a == 0 ? ti : tj),
+                  lk = a == 2 ? (hi ? k0 + KP : k0 - 1) : k0 + (KP == 16 ? tj : tj % KP);
         const int32_t sn = s27[((li >> 4) + 1) + 3 * ((lj >> 4) + 1) + 9 * ((lk >> 4) + 1)];
         const int I = w.x * 16 + li, J = w.y * 16 + lj, K = w.z * 16 + lk;
         const size_t ci = cl(min(max(I >> 2, 0), n0 - 1), min(max(J >> 2, 0), n1 - 1), min(max(K >> 2, 0), n2 - 1), n0, n1);
@@ -670,7 +679,7 @@ __global__ __launch_bounds__(256) void k_sreinit(float* __restrict__ out, const 
         hl[m] = sn != 0 ? phi[fi] : phic[ci];
     }
 #pragma unroll
-    for (int k = 0; k < 16; ++k) tv[tid + 256 * k] = own[k];
+    for (int k = 0; k < KP; ++k) tv[tid + 256 * k] = own[k];
 #pragma unroll
     for (int m = 0; m < 6; ++m) hv[m][tid] = hl[m];
     const bool clear = blockclear(g, w);
@@ -678,17 +687,17 @@ __global__ __launch_bounds__(256) void k_sreinit(float* __restrict__ out, const 
     // takes this one value: the same function of the same arguments
     const float dsat = jmin(eikonal(phimax, phimax, phimax, g.dx), phimax);
     __syncthreads();
-    float* __restrict__ op = out + (size_t)slot * 4096;
-    for (int k = 0; k < 16; ++k) {
+    float* __restrict__ op = out + (size_t)slot * 4096 + 256 * k0;
+    for (int k = 0; k < KP; ++k) {
         const int l = tid + 256 * k;
-        const int I = w.x * 16 + ti, J = w.y * 16 + tj, K = w.z * 16 + k;
+        const int I = w.x * 16 + ti, J = w.y * 16 + tj, K = w.z * 16 + k0 + k;
         const float cv = tv[l], h = g.dx;
         float nv[6];   // in the order of NBS: +x, -x, +y, -y, +z, -z
         nv[0] = ti < 15 ? tv[l + 1] : hv[0][tj + 16 * k];
         nv[1] = ti > 0 ? tv[l - 1] : hv[1][tj + 16 * k];
         nv[2] = tj < 15 ? tv[l + 16] : hv[2][ti + 16 * k];
         nv[3] = tj > 0 ? tv[l - 16] : hv[3][ti + 16 * k];
-        nv[4] = k < 15 ? tv[l + 256] : hv[4][tid];
+        nv[4] = k < KP - 1 ? tv[l + 256] : hv[4][tid];
         nv[5] = k > 0 ? tv[l - 256] : hv[5][tid];
         bool solid = false, nsolid[6] = {false, false, false, false, false, false};
         if (!clear) {
@@ -769,8 +778,8 @@ void SparseBasin::redistance(int iterations) {
     hipStream_t s = st.s;
     for (int it = 0; it < iterations && nslots > 0; ++it) {
         if (nlive > 0)   // free slots keep what they hold in both copies: nothing reads them
-            hipLaunchKernelGGL(k_sreinit, dim3((unsigned)nlive), dim3(256), 0, s, phi0.fine.p, phi.fine.p, phi.coarse.p,
-                               topo(), phimax, sorder.p);
+            hipLaunchKernelGGL(nlive <= 512 ? k_sreinit<4> : k_sreinit<16>, dim3((unsigned)nlive, nlive <= 512 ? 4 : 1), dim3(256),
+                               0, s, phi0.fine.p, phi.fine.p, phi.coarse.p, topo(), phimax, sorder.p);
         std::swap(phi.fine, phi0.fine);
     }
     hipLaunchKernelGGL(k_coarsewall, dim3(cdiv(ncells(), 256)), dim3(256), 0, s, phi0.coarse.p, phi.coarse.p, topo());
