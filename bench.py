@@ -59,13 +59,14 @@ def sparse_bytes(kernel, live_cells, n_particles, precision=0, coarse_cells=0, c
         # per fine cell: x, b, the Dirichlet diagonal (FP32) or the Jacobi weight
         # omega/diag (FP16/BF16) and the result (e B each), the type (1 B); level 0's
         # couplings follow from the types (the row is matrix-free). Per coarse cell outside
-        # the blocks: x, b, the Dirichlet diagonal and the result (e B each), the type, the
-        # activity and the cover mask (1 B each); under a block: activity, mask, result.
-        "jacobi": (4 * e + 1) * live_cells + (4 * e + 3) * (coarse_cells - covered) + (e + 2) * covered,
-        # the flexible CG's search (FP32): z, d read, d, q written, the full diagonal read
-        # (4 B each) and the type (1 B) per fine cell; per coarse cell outside the blocks the
-        # same and the activity and cover mask; under a block activity, mask and q
-        "search": 21 * live_cells + 23 * (coarse_cells - covered) + 6 * covered,
+        # the blocks: x, b, the Dirichlet diagonal and the result (e B each) and the row's
+        # mask (2 B); under a block: the mask and the result.
+        "jacobi": (4 * e + 1) * live_cells + (4 * e + 2) * (coarse_cells - covered) + (e + 2) * covered,
+        # the flexible CG's search: z read in the V-cycle's precision (e B), d read, d, q
+        # written, the full diagonal read (4 B each, FP32) and the type (1 B) per fine cell;
+        # per coarse cell outside the blocks the same with the mask (2 B) for the type; under
+        # a block the mask and q
+        "search": (17 + e) * live_cells + (18 + e) * (coarse_cells - covered) + 6 * covered,
         # the flexible CG's update: P read and written, r read, the new r written (over
         # the older residual buffer), d, q read (4 B each) and the type (1 B) per unknown;
         # the cover mask too on the coarse grid

@@ -2058,7 +2058,7 @@ struct SparseSolver {
     // (N^3 a slot) and the coarse part, in one launch.
     template <int N, int MODE, class T, class C, class X>
     void rows(SVecT<T> out, SVecT<X> x, SVecT<T> b, const CompT<C>& L, RowArgs<T> S = RowArgs<T>{}) {
-        constexpr bool SWEEP = N == 16 && (MODE == 0 || MODE == 8);
+        constexpr bool SWEEP = N == 16 && MODE == 0;
         const uint32_t ncb = (uint32_t)cdiv(Cc, 256);
         if (SWEEP) s.kt.begin(K_RBGS, st);
         if (s.nslots) {
