@@ -1228,23 +1228,25 @@ __global__ __launch_bounds__(256) void k_head0(T* __restrict__ outf, T* __restri
 
 // ─── dense levels (sflip.jl:1574-1657) ───────────────────────────────────────
 
-// A dense level's cell: diag and the neighbours' sum; all loads issued before any use
-// (an index off the grid reads the cell itself, and its coupling adds nothing).
-template <class T, class C, bool Z = false>
-__device__ inline void denserow(const DViewT<C>& L, const T* __restrict__ x, int i, int j, int k, float& diag, float& off) {
-    int n0 = L.n.x, n1 = L.n.y, n2 = L.n.z;
-    size_t own = cl(i, j, k, n0, n1), sy = (size_t)n0, sz = (size_t)n0 * n1;
-    float c0 = lf(L.c[0][cl(i, j, k, n0 + 1, n1)]), c1 = lf(L.c[0][cl(i + 1, j, k, n0 + 1, n1)]);
-    float c2 = lf(L.c[1][cl(i, j, k, n0, n1 + 1)]), c3 = lf(L.c[1][cl(i, j + 1, k, n0, n1 + 1)]);
-    float c4 = lf(L.c[2][cl(i, j, k, n0, n1)]), c5 = lf(L.c[2][cl(i, j, k + 1, n0, n1)]);
-    auto xv = [&](bool ok, size_t idx) -> float {
-        if constexpr (Z) return 0.0f;   // x = 0: nothing to read
-        return lf(x[ok ? idx : own]);
-    };
+// A dense level's cell l = (i, j, k): diag and the neighbours' sum, the neighbours' values
+// from xat(index, i, j, k); all loads issued before any use (an index off the grid reads the
+// cell itself, and its coupling adds nothing).
+template <class C, class X>
+__device__ inline void denserow(const DViewT<C>& L, X xat, uint32_t l, int i, int j, int k, float& diag, float& off) {
+    const int n0 = L.n.x, n1 = L.n.y, n2 = L.n.z;
+    const uint32_t sy = (uint32_t)n0, sz = (uint32_t)n0 * (uint32_t)n1;
+    const uint32_t fx = l + (uint32_t)j + (uint32_t)n1 * (uint32_t)k, fy = l + sy * (uint32_t)k;   // its x and y faces
+    float c0 = lf(L.c[0][fx]), c1 = lf(L.c[0][fx + 1]);
+    float c2 = lf(L.c[1][fy]), c3 = lf(L.c[1][fy + sy]);
+    float c4 = lf(L.c[2][l]), c5 = lf(L.c[2][l + sz]);
     bool b0 = i > 0, b1 = i < n0 - 1, b2 = j > 0, b3 = j < n1 - 1, b4 = k > 0, b5 = k < n2 - 1;
-    float x0 = xv(b0, own - 1), x1 = xv(b1, own + 1), x2 = xv(b2, own - sy), x3 = xv(b3, own + sy);
-    float x4 = xv(b4, own - sz), x5 = xv(b5, own + sz);
-    diag = lf(L.dD[own]);
+    auto xv = [&](bool ok, uint32_t n, int a, int b, int c) -> float {
+        return xat(ok ? n : l, ok ? a : i, ok ? b : j, ok ? c : k);
+    };
+    float x0 = xv(b0, l - 1, i - 1, j, k), x1 = xv(b1, l + 1, i + 1, j, k);
+    float x2 = xv(b2, l - sy, i, j - 1, k), x3 = xv(b3, l + sy, i, j + 1, k);
+    float x4 = xv(b4, l - sz, i, j, k - 1), x5 = xv(b5, l + sz, i, j, k + 1);
+    diag = lf(L.dD[l]);
     off = 0.0f;
     if (c0 > 0.0f && b0) { diag += c0; off += c0 * x0; }
     if (c1 > 0.0f && b1) { diag += c1; off += c1 * x1; }
@@ -1253,26 +1255,36 @@ __device__ inline void denserow(const DViewT<C>& L, const T* __restrict__ x, int
     if (c4 > 0.0f && b4) { diag += c4; off += c4 * x4; }
     if (c5 > 0.0f && b5) { diag += c5; off += c5 * x5; }
 }
-// mode 0 Jacobi, 1 residual, 3 Jacobi from x = 0 (x not read)
+// mode 0 Jacobi, 3 Jacobi from x = 0 (x not read), 8 Jacobi on x prolonged, x + boost xc of
+// the coarser level (where a cell couples to a neighbour, the neighbour is active). The grid
+// round the basin is mostly not active: a wavefront without an active cell stops at the
+// flags (2.9 M cells in FP16: a sweep 14.8 -> 12.4 us, the first one up with its prolongation
+// 23.5 -> 17.1).
 template <int MODE, class T, class C>
 __global__ __launch_bounds__(256) void k_rowdense(T* __restrict__ out, const T* __restrict__ x, const T* __restrict__ b,
-                                                  DViewT<C> L) {
-    size_t l = (size_t)xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;   // neighbouring rows on one XCD
-    if (l >= (size_t)L.n.x * L.n.y * L.n.z) return;
-    int i, j, k;
-    unlin(l, L.n.x, L.n.y, i, j, k);
-    // the row's loads issued with the activity flag's, the result selected after
-    const bool act = L.act[l] != 0;
-    float diag, off;
-    denserow<T, C, MODE == 3>(L, x, i, j, k, diag, off);
-    const float xl = MODE == 3 ? 0.0f : lf(x[l]), bl = lf(b[l]);
-    const float ax = diag * xl - off;
-    const float res = MODE != 1 ? (diag > 0.0f ? xl + __fdiv_rn(OMEGA * (bl - ax), diag) : 0.0f) : bl - ax;
-    out[l] = sf<T>(act ? res : 0.0f);
+                                                  DViewT<C> L, const T* __restrict__ xc, int3 nc, float boost) {
+    const uint32_t l = xcd_tile(blockIdx.x, gridDim.x) * 256u + threadIdx.x;   // neighbouring rows on one XCD
+    if (l >= (uint32_t)L.n.x * (uint32_t)L.n.y * (uint32_t)L.n.z) return;
+    float res = 0.0f;
+    if (L.act[l] != 0) {
+        int i, j, k;
+        unlin(l, L.n.x, L.n.y, i, j, k);
+        auto xat = [&](uint32_t n, int a, int bb, int c) -> float {
+            if constexpr (MODE == 3) return 0.0f;
+            else if constexpr (MODE == 8)
+                return lf(sf<T>(lf(x[n]) + boost * lf(xc[(uint32_t)(a >> 1) + (uint32_t)nc.x * ((uint32_t)(bb >> 1) +
+                                                                                          (uint32_t)nc.y * (uint32_t)(c >> 1))])));
+            else return lf(x[n]);
+        };
+        float diag, off;
+        denserow(L, xat, l, i, j, k, diag, off);
+        const float xl = xat(l, i, j, k), ax = diag * xl - off;
+        res = diag > 0.0f ? xl + __fdiv_rn(OMEGA * (lf(b[l]) - ax), diag) : 0.0f;
+    }
+    out[l] = sf<T>(res);
 }
 // The coarser level's right-hand side, the residual and its restriction in one pass:
-// each coarser cell forms its eight finer cells' residuals (k_rowdense mode 1's
-// arithmetic, rounded to T as that kernel would store them), sums them in x-fastest
+// each coarser cell forms its eight finer cells' residuals (rounded to T), sums them in x-fastest
 // order and multiplies by `scale` (1 in the reference's solve; the reduced-precision
 // hierarchy carries each dense level's equations divided by 4 per level, so its values
 // stay in FP16's range). No residual array is written.
@@ -1288,27 +1300,17 @@ __global__ void k_residrestrict(T* __restrict__ bc, const T* __restrict__ x, con
         for (int bb = 0; bb < 2; ++bb)
             for (int a = 0; a < 2; ++a) {
                 const int i = 2 * I + a, j = 2 * J + bb, k = 2 * K + c;
-                const size_t f = cl(i, j, k, L.n.x, L.n.y);
+                const uint32_t f = (uint32_t)i + (uint32_t)L.n.x * ((uint32_t)j + (uint32_t)L.n.y * (uint32_t)k);
                 float res = 0.0f;
                 if (L.act[f] != 0) {
                     float diag, off;
-                    denserow<T, C, false>(L, x, i, j, k, diag, off);
+                    denserow(L, [&](uint32_t n, int, int, int) { return lf(x[n]); }, f, i, j, k, diag, off);
                     res = lf(b[f]) - (diag * lf(x[f]) - off);
                 }
                 acc += lf(sf<T>(res));
             }
     bc[l] = sf<T>(acc * scale);
 }
-template <class T>
-__global__ void k_prolongdense(T* __restrict__ xf, const T* __restrict__ xc, const uint8_t* __restrict__ actf, int3 nf, int3 nc,
-                               float boost) {
-    size_t l = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (l >= (size_t)nf.x * nf.y * nf.z) return;
-    int i, j, k;
-    unlin(l, nf.x, nf.y, i, j, k);
-    if (actf[l] != 0) xf[l] = sf<T>(lf(xf[l]) + boost * lf(xc[cl(i >> 1, j >> 1, k >> 1, nc.x, nc.y)]));
-}
-
 // Conversions between the Krylov vectors (FP32) and the reduced-precision hierarchy:
 // y = x * mult * scal[slot] (or * mult when slot < 0), over the fine and the coarse range,
 // four values a thread (both parts are multiples of 4 long).
@@ -2165,28 +2167,30 @@ struct SparseSolver {
         for (int l = tiled - 1; l >= 0; --l) dense_up<T, C>(H, l, x[l + 1], sweeps, boost);
         return x[0];
     }
-    // a level's way down and up with any number of sweep pairs, a launch a sweep
+    // a level's way down and up with any number of sweep pairs, a launch a sweep; the first on
+    // the way down is from x = 0, the first on the way up takes the prolongation in
+    template <int MODE, class T, class C>
+    void rowdense(T* out, const T* x, const T* b, const DViewT<C>& L, size_t cells, const T* xc = nullptr, int3 nc = int3{},
+                  float boost = 0.0f) {
+        hipLaunchKernelGGL((k_rowdense<MODE, T, C>), dim3(cdiv(cells, 256)), dim3(256), 0, st, out, x, b, L, xc, nc, boost);
+    }
     template <class T, class C> void dense_down(Hier<T, C>& H, int l, int sweeps) {
         SLevel &Dl = s.D[l], &Cn = s.D[l + 1];
-        size_t c = Dl.cells();
-        for (int k = 0; k < sweeps; ++k) {   // from x = 0: the first sweep reads no x
-            if (k == 0)
-                hipLaunchKernelGGL((k_rowdense<3, T, C>), dim3(cdiv(c, 256)), dim3(256), 0, st, H.Dt[l], H.Dx[l], H.Db[l], H.D[l]);
-            else
-                hipLaunchKernelGGL((k_rowdense<0, T, C>), dim3(cdiv(c, 256)), dim3(256), 0, st, H.Dt[l], H.Dx[l], H.Db[l], H.D[l]);
-            hipLaunchKernelGGL((k_rowdense<0, T, C>), dim3(cdiv(c, 256)), dim3(256), 0, st, H.Dx[l], H.Dt[l], H.Db[l], H.D[l]);
+        const size_t c = Dl.cells();
+        for (int k = 0; k < sweeps; ++k) {
+            if (k == 0) rowdense<3>(H.Dt[l], (const T*)nullptr, (const T*)H.Db[l], H.D[l], c);
+            else rowdense<0>(H.Dt[l], (const T*)H.Dx[l], (const T*)H.Db[l], H.D[l], c);
+            rowdense<0>(H.Dx[l], (const T*)H.Dt[l], (const T*)H.Db[l], H.D[l], c);
         }
         hipLaunchKernelGGL((k_residrestrict<T, C>), dim3(cdiv(Cn.cells(), 256)), dim3(256), 0, st, H.Db[l + 1], H.Dx[l], H.Db[l],
                            H.D[l], i3(Cn.n), H.rscale);
     }
     template <class T, class C> void dense_up(Hier<T, C>& H, int l, const T* coarser, int sweeps, float boost) {
-        SLevel &Dl = s.D[l], &Cn = s.D[l + 1];
-        size_t c = Dl.cells();
-        hipLaunchKernelGGL(k_prolongdense<T>, dim3(cdiv(c, 256)), dim3(256), 0, st, H.Dx[l], coarser, Dl.act.p, i3(Dl.n), i3(Cn.n),
-                           boost);
+        const size_t c = s.D[l].cells();
         for (int k = 0; k < sweeps; ++k) {
-            hipLaunchKernelGGL((k_rowdense<0, T, C>), dim3(cdiv(c, 256)), dim3(256), 0, st, H.Dt[l], H.Dx[l], H.Db[l], H.D[l]);
-            hipLaunchKernelGGL((k_rowdense<0, T, C>), dim3(cdiv(c, 256)), dim3(256), 0, st, H.Dx[l], H.Dt[l], H.Db[l], H.D[l]);
+            if (k == 0) rowdense<8>(H.Dt[l], (const T*)H.Dx[l], (const T*)H.Db[l], H.D[l], c, coarser, i3(s.D[l + 1].n), boost);
+            else rowdense<0>(H.Dt[l], (const T*)H.Dx[l], (const T*)H.Db[l], H.D[l], c);
+            rowdense<0>(H.Dx[l], (const T*)H.Dt[l], (const T*)H.Db[l], H.D[l], c);
         }
     }
 
