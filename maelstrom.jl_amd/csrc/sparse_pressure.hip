@@ -1258,17 +1258,16 @@ __device__ inline void denserow(const DViewT<C>& L, X xat, uint32_t l, int i, in
 // mode 0 Jacobi, 3 Jacobi from x = 0 (x not read), 8 Jacobi on x prolonged, x + boost xc of
 // the coarser level (where a cell couples to a neighbour, the neighbour is active). The grid
 // round the basin is mostly not active: a wavefront without an active cell stops at the
-// flags (2.9 M cells in FP16: a sweep 14.8 -> 12.4 us, the first one up with its prolongation
-// 23.5 -> 17.1).
+// flags, and the launch is over 64 x 4 cells of a plane, so that no wavefront divides (2.9 M
+// cells in FP16: a sweep 14.8 -> 10.1 us, the first one up with its prolongation 23.5 -> 13.3).
 template <int MODE, class T, class C>
 __global__ __launch_bounds__(256) void k_rowdense(T* __restrict__ out, const T* __restrict__ x, const T* __restrict__ b,
                                                   DViewT<C> L, const T* __restrict__ xc, int3 nc, float boost) {
-    const uint32_t l = xcd_tile(blockIdx.x, gridDim.x) * 256u + threadIdx.x;   // neighbouring rows on one XCD
-    if (l >= (uint32_t)L.n.x * (uint32_t)L.n.y * (uint32_t)L.n.z) return;
+    const int i = 64 * (int)blockIdx.x + (int)(threadIdx.x & 63), j = 4 * (int)blockIdx.y + (int)(threadIdx.x >> 6), k = (int)blockIdx.z;
+    if (i >= L.n.x || j >= L.n.y) return;
+    const uint32_t l = (uint32_t)i + (uint32_t)L.n.x * ((uint32_t)j + (uint32_t)L.n.y * (uint32_t)k);
     float res = 0.0f;
     if (L.act[l] != 0) {
-        int i, j, k;
-        unlin(l, L.n.x, L.n.y, i, j, k);
         auto xat = [&](uint32_t n, int a, int bb, int c) -> float {
             if constexpr (MODE == 3) return 0.0f;
             else if constexpr (MODE == 8)
@@ -2178,27 +2177,25 @@ struct SparseSolver {
     // a level's way down and up with any number of sweep pairs, a launch a sweep; the first on
     // the way down is from x = 0, the first on the way up takes the prolongation in
     template <int MODE, class T, class C>
-    void rowdense(T* out, const T* x, const T* b, const DViewT<C>& L, size_t cells, const T* xc = nullptr, int3 nc = int3{},
-                  float boost = 0.0f) {
-        hipLaunchKernelGGL((k_rowdense<MODE, T, C>), dim3(cdiv(cells, 256)), dim3(256), 0, st, out, x, b, L, xc, nc, boost);
+    void rowdense(T* out, const T* x, const T* b, const DViewT<C>& L, const T* xc = nullptr, int3 nc = int3{}, float boost = 0.0f) {
+        hipLaunchKernelGGL((k_rowdense<MODE, T, C>), dim3(cdiv(L.n.x, 64), cdiv(L.n.y, 4), L.n.z), dim3(256), 0, st, out, x, b, L, xc,
+                           nc, boost);
     }
     template <class T, class C> void dense_down(Hier<T, C>& H, int l, int sweeps) {
-        SLevel &Dl = s.D[l], &Cn = s.D[l + 1];
-        const size_t c = Dl.cells();
+        SLevel& Cn = s.D[l + 1];
         for (int k = 0; k < sweeps; ++k) {
-            if (k == 0) rowdense<3>(H.Dt[l], (const T*)nullptr, (const T*)H.Db[l], H.D[l], c);
-            else rowdense<0>(H.Dt[l], (const T*)H.Dx[l], (const T*)H.Db[l], H.D[l], c);
-            rowdense<0>(H.Dx[l], (const T*)H.Dt[l], (const T*)H.Db[l], H.D[l], c);
+            if (k == 0) rowdense<3>(H.Dt[l], (const T*)nullptr, (const T*)H.Db[l], H.D[l]);
+            else rowdense<0>(H.Dt[l], (const T*)H.Dx[l], (const T*)H.Db[l], H.D[l]);
+            rowdense<0>(H.Dx[l], (const T*)H.Dt[l], (const T*)H.Db[l], H.D[l]);
         }
         hipLaunchKernelGGL((k_residrestrict<T, C>), dim3(cdiv(Cn.n[0], 32), Cn.n[1], Cn.n[2]), dim3(256), 0, st, H.Db[l + 1], H.Dx[l],
                            H.Db[l], H.D[l], i3(Cn.n), H.rscale);
     }
     template <class T, class C> void dense_up(Hier<T, C>& H, int l, const T* coarser, int sweeps, float boost) {
-        const size_t c = s.D[l].cells();
         for (int k = 0; k < sweeps; ++k) {
-            if (k == 0) rowdense<8>(H.Dt[l], (const T*)H.Dx[l], (const T*)H.Db[l], H.D[l], c, coarser, i3(s.D[l + 1].n), boost);
-            else rowdense<0>(H.Dt[l], (const T*)H.Dx[l], (const T*)H.Db[l], H.D[l], c);
-            rowdense<0>(H.Dx[l], (const T*)H.Dt[l], (const T*)H.Db[l], H.D[l], c);
+            if (k == 0) rowdense<8>(H.Dt[l], (const T*)H.Dx[l], (const T*)H.Db[l], H.D[l], coarser, i3(s.D[l + 1].n), boost);
+            else rowdense<0>(H.Dt[l], (const T*)H.Dx[l], (const T*)H.Db[l], H.D[l]);
+            rowdense<0>(H.Dx[l], (const T*)H.Dt[l], (const T*)H.Db[l], H.D[l]);
         }
     }
 
