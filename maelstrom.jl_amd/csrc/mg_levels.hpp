@@ -7,7 +7,7 @@
 // workgroup takes a tile with a halo of two cells, a thread keeps the rows of its cells in
 // registers through the sweeps and the values go through LDS; a neighbour's cells are
 // computed again in the halo. Every value goes through the same operations and roundings to
-// the storage type as in a launch of its own (k_rowdense, k_residrestrict, k_prolongdense;
+// the storage type as in a launch of its own (k_rowdense, k_residrestrict;
 // a face without a coupling adds a zero product instead of being skipped), so the V-cycle's
 // values do not change.
 //

@@ -1912,9 +1912,10 @@ struct SVec {   // a pressure-sized vector: fine pool part and coarse part
 };
 
 // Dense levels of at most MG_TILED cells take the tiled launches, with 8^3 tiles up to
-// MG_SMALL cells. At 2.9 M cells (FP16) the halo's repeated rows cost what the saved passes
-// gain (a 5 cm solve 18.1 ms tiled, 18.0 ms with a launch a sweep there); at 368,640 the tiles
-// are ahead (18.1 ms without them). 8^3 tiles put a level of up to 80,000 cells on more
+// MG_SMALL cells. At 2.9 M cells (FP16) the halo's repeated rows cost more than the saved
+// passes gain (two tiled launches against five took as long when a pass took 15 us; it takes
+// 10 now); at 368,640 the two are even (a 5 cm solve 14.80 ms tiled, 14.76 with a launch a
+// pass), and the tiles make fewer launches. 8^3 tiles put a level of up to 80,000 cells on more
 // CUs: 144 workgroups for 73,728 cells, where 16x8x8 would make 72.
 constexpr size_t MG_TILED = 500000, MG_SMALL = 80000;
 
