@@ -194,23 +194,46 @@ struct NodeBoxes {
     }
 };
 
+// The words of LDS for a workgroup's reductions: wg_mins' six, and a wavefront's counts.
+constexpr int BOX_RED = 7 * (P2G_THREADS / 64);
 // The boxes for the workgroup's `act` lanes: theirs if it has at most `cap`
-// nodes, else that of the lanes on the low side of the middle of the widest extent, halved
+// nodes, else that of the lanes on one side of the middle of the widest extent, halved
 // again until it fits (its least lane is below the middle and its greatest is not: both
-// sides hold particles, so this ends). act becomes the lanes of the box.
-__device__ inline NodeBoxes fitting_boxes(bool& act, const float (&qo)[3], int cap, int* red) {
+// sides hold particles, so this ends). act becomes the lanes of the box. With `left` 0 the low
+// side (the deposit, where a particle that no box takes costs global adds); else the side with
+// more lanes, and no box (`any` false) where `left` boxes of as many lanes would not take them
+// all: a gather's workgroup that leaves any particle to its own reads waits for those once,
+// whether they are few or all 256.
+__device__ inline NodeBoxes fitting_boxes(bool& act, const float (&qo)[3], int cap, int left, int* red) {
     NodeBoxes B(act, qo, red);
     const int s0 = NodeBoxes::sum(act, qo[0]), s1 = NodeBoxes::sum(act, qo[1]), s2 = NodeBoxes::sum(act, qo[2]);
+    int whole = 0;
     while (B.any && B.largest() > cap) {
         const int e0 = B.hi[0] - B.lo[0], e1 = B.hi[1] - B.lo[1], e2 = B.hi[2] - B.lo[2];
         const int k = e0 >= e1 && e0 >= e2 ? 0 : (e1 >= e2 ? 1 : 2);
         const int lo = k == 0 ? B.lo[0] : (k == 1 ? B.lo[1] : B.lo[2]), hi = k == 0 ? B.hi[0] : (k == 1 ? B.hi[1] : B.hi[2]);
-        act = act && (k == 0 ? s0 : (k == 1 ? s1 : s2)) < (lo + hi + 1) >> 1;
+        const bool below = (k == 0 ? s0 : (k == 1 ? s1 : s2)) < (lo + hi + 1) >> 1;
+        bool low = true;
+        if (left > 0) {
+            // (NodeBoxes' barriers lie between two uses of these words)
+            const int n = (int)(__popcll(__ballot(act)) << 16 | __popcll(__ballot(act && below)));
+            if ((threadIdx.x & 63) == 0) red[24 + (threadIdx.x >> 6)] = n;
+            __syncthreads();
+            const int4 r = *reinterpret_cast<const int4*>(red + 24);
+            const int both = __builtin_amdgcn_readfirstlane(r.x + r.y + r.z + r.w), all = both >> 16, under = both & 0xffff;
+            if (whole == 0) whole = all;
+            low = 2 * under >= all;
+            if ((low ? under : all - under) * left < whole) {
+                B.any = false;
+                break;
+            }
+        }
+        act = act && below == low;
         B = NodeBoxes(act, qo, red);
     }
     return B;
 }
-// Boxes a workgroup takes before what is left goes to global memory node by node.
+// Boxes a workgroup of the deposit takes before what is left goes to global memory node by node.
 constexpr int BOX_ROUNDS = 4;
 
 // NodeMap: `index(a, I, J, K)` of a face node, < 0 off the grid (the dense grid's array
@@ -233,7 +256,7 @@ template <class NodeMap, class Source, int BOX = P2G_BOX>
 __global__ __launch_bounds__(P2G_THREADS, 4) void k_p2g_tiled(PView ps, int64_t n, NodeMap map, Source src,
                                                                               P2GArgs A) {
     __shared__ unsigned long long smom[BOX], swt[Source::WEIGHTS ? BOX : 1];
-    __shared__ alignas(16) int red[12 * (P2G_THREADS / 64)];
+    __shared__ alignas(16) int red[BOX_RED];
     __shared__ int32_t stab[NodeMap::TAB];
     const int64_t p0 = (int64_t)xcd_tile(blockIdx.x, gridDim.x) * P2G_THREADS;   // neighbouring tiles on one XCD
     // A wavefront takes every eighth particle: particles of one cell (consecutive in cell
@@ -262,7 +285,7 @@ __global__ __launch_bounds__(P2G_THREADS, 4) void k_p2g_tiled(PView ps, int64_t 
         // same in every round, out of the loop and into registers that it does not have)
         asm volatile("" : "+v"(qo[0]), "+v"(qo[1]), "+v"(qo[2]));
         bool act = todo;
-        const NodeBoxes B = fitting_boxes(act, qo, BOX, red);
+        const NodeBoxes B = fitting_boxes(act, qo, BOX, 0, red);
         if (!B.any) break;   // none left (the bounds are the workgroup's)
         todo = todo && !act;
         int lo[3], hi[3];
@@ -353,6 +376,11 @@ inline dim3 p2g_grid(int64_t n) {
 // Every path takes the flags' sum and the value and affine row over the 27 nodes in the
 // reference's order (gather, sflip.jl:193-215 finegather), so the same bits.
 //
+// NodeMap::boxes() is how many a workgroup takes. Particles come in cell order from a step,
+// where several boxes pay, but a caller may set them in any: 98,000 (27 in cell order) and 1.6 M
+// (112) in random order on the sparse basin take 59 and 1,100 us, as many as without boxes,
+// and took 115 and 1,350 with up to four boxes whatever those held.
+//
 // NodeMap as k_p2g_tiled's; HOLES: a node may be missing (index < 0) and is skipped. In a
 // box, a missing node's flag is -1 and its value 0 and it adds zero products instead: the
 // sums start at +0 and are never -0, so adding a zero leaves them bit for bit as skipping.
@@ -372,7 +400,7 @@ template <class NodeMap>
 __global__ __launch_bounds__(P2G_THREADS, 4) void k_g2p_tiled(PView ps, int64_t n, NodeMap map, float lo0, float lo1, float lo2,
                                                               float dx, G2PFaces F, float dt, float gravity) {
     __shared__ float sval[G2P_BOX], sflag[G2P_BOX];
-    __shared__ alignas(16) int red[6 * (P2G_THREADS / 64)];
+    __shared__ alignas(16) int red[BOX_RED];
     __shared__ int32_t stab[NodeMap::TAB];
     const int64_t p = (int64_t)xcd_tile(blockIdx.x, gridDim.x) * P2G_THREADS + threadIdx.x;   // neighbouring tiles on one XCD
     const bool live = p < n;
@@ -398,12 +426,12 @@ __global__ __launch_bounds__(P2G_THREADS, 4) void k_g2p_tiled(PView ps, int64_t 
     };
 
     bool todo = live && NodeBoxes::fits(qo[0]) && NodeBoxes::fits(qo[1]) && NodeBoxes::fits(qo[2]);
-    bool left = live && !todo;
+    const bool far = live && !todo;
 #pragma unroll 1
-    for (int round = 0; round < BOX_ROUNDS; ++round) {
+    for (int left = NodeMap::boxes(); left > 0; --left) {
         asm volatile("" : "+v"(qo[0]), "+v"(qo[1]), "+v"(qo[2]));   // as in k_p2g_tiled: nothing moved out of the loop
         bool act = todo;
-        const NodeBoxes B = fitting_boxes(act, qo, G2P_BOX, red);
+        const NodeBoxes B = fitting_boxes(act, qo, G2P_BOX, left, red);
         if (!B.any) break;
         todo = todo && !act;
         int lo[3], hi[3];
@@ -477,31 +505,54 @@ __global__ __launch_bounds__(P2G_THREADS, 4) void k_g2p_tiled(PView ps, int64_t 
         }
         if (act) finish(reached, rec);
     }
-    if (todo || left) {   // far apart, not finite or far off the grid
-        float rec[12];
+    if (todo || far) {   // far apart, not finite or far off the grid
+        // (a component at a time in a loop, its sums kept in the box, which is free now: the
+        // nodes' reads of all three together would not fit the registers)
+        static_assert(6 * P2G_THREADS <= G2P_BOX, "the sums of a thread fit the box");
+        auto sums = [&](int f) -> float& {
+            return f < 6 ? sval[f * P2G_THREADS + threadIdx.x] : sflag[(f - 6) * P2G_THREADS + threadIdx.x];
+        };
         bool reached = true;
-#pragma unroll
+#pragma unroll 1
         for (int a = 0; a < 3; ++a) {
+            const float* __restrict__ u = a == 0 ? F.u[0] : (a == 1 ? F.u[1] : F.u[2]);
+            const uint8_t* __restrict__ fl = a == 0 ? F.f[0] : (a == 1 ? F.f[1] : F.f[2]);
             const float q0 = a == 0 ? qo[0] : qo[0] - 0.5f, q1 = a == 1 ? qo[1] : qo[1] - 0.5f, q2 = a == 2 ? qo[2] : qo[2] - 0.5f;
             const BSpline bx = bspline(q0), by = bspline(q1), bz = bspline(q2);
             float f_ = 0.0f, v_ = 0.0f, s0 = 0.0f, s1 = 0.0f, s2 = 0.0f;
-#pragma unroll 1
-            for (int m = 0; m < 27; ++m) {
-                const int mx = m % 3, my = (m / 3) % 3, mz = m / 9;
-                const int I = node_at(bx.b, mx), J = node_at(by.b, my), K = node_at(bz.b, mz);
-                const auto idx = map.index(a, I, J, K);
-                if (NodeMap::HOLES && idx < 0) continue;
-                const float wgt = pick(bx, mx) * pick(by, my) * pick(bz, mz);
-                f_ += wgt * (float)F.f[a][idx];
-                const float t = wgt * F.u[a][idx];
+            auto nodes = [&](auto each) {
+#pragma unroll
+                for (int mz = 0; mz < 3; ++mz)
+#pragma unroll
+                    for (int my = 0; my < 3; ++my)
+#pragma unroll
+                        for (int mx = 0; mx < 3; ++mx) {
+                            const int I = node_at(bx.b, mx), J = node_at(by.b, my), K = node_at(bz.b, mz);
+                            const auto idx = map.index(a, I, J, K);
+                            if (!NodeMap::HOLES || idx >= 0) each(idx, pick(bx, mx) * pick(by, my) * pick(bz, mz), I, J, K);
+                        }
+            };
+            auto flagsum = [&](auto idx, float wgt, int, int, int) { f_ += wgt * (float)fl[idx]; };
+            auto sum = [&](auto idx, float wgt, int I, int J, int K) {
+                const float t = wgt * u[idx];
                 v_ += t;
                 s0 += (t * ((float)I - q0)) * dx;
                 s1 += (t * ((float)J - q1)) * dx;
                 s2 += (t * ((float)K - q2)) * dx;
+            };
+            if (NodeMap::HOLES) {   // (looking a node's block up costs more than a read)
+                nodes([&](auto idx, float wgt, int I, int J, int K) { flagsum(idx, wgt, I, J, K); sum(idx, wgt, I, J, K); });
+            } else {
+                nodes(flagsum);
+                nodes(sum);
             }
             reached = reached && f_ > 0.999f;
-            rec[a] = v_; rec[3 + 3 * a] = s0 * c4; rec[4 + 3 * a] = s1 * c4; rec[5 + 3 * a] = s2 * c4;
+            sums(a) = v_;
+            sums(3 + 3 * a) = s0 * c4; sums(4 + 3 * a) = s1 * c4; sums(5 + 3 * a) = s2 * c4;
         }
+        float rec[12];
+#pragma unroll
+        for (int f = 0; f < 12; ++f) rec[f] = sums(f);
         finish(reached, rec);
     }
 }
@@ -521,7 +572,7 @@ template <class CellMap>
 __global__ __launch_bounds__(P2G_THREADS) void k_splat_tiled(PView ps, int64_t n, CellMap map, float lo0, float lo1, float lo2,
                                                             float dx, float dt, int32_t* __restrict__ phip) {
     __shared__ int32_t box[SPLAT_BOX];
-    __shared__ alignas(16) int red[6 * (P2G_THREADS / 64)];
+    __shared__ alignas(16) int red[BOX_RED];
     __shared__ int32_t stab[CellMap::TAB];
     const int64_t p0 = (int64_t)xcd_tile(blockIdx.x, gridDim.x) * P2G_THREADS;   // neighbouring tiles on one XCD
     // every eighth particle per lane group, as in k_p2g_tiled
@@ -555,7 +606,7 @@ __global__ __launch_bounds__(P2G_THREADS) void k_splat_tiled(PView ps, int64_t n
 #pragma unroll 1
     for (int round = 0; round < BOX_ROUNDS; ++round) {
         bool act = todo;
-        const NodeBoxes B = fitting_boxes(act, qo, SPLAT_BOX, red);
+        const NodeBoxes B = fitting_boxes(act, qo, SPLAT_BOX, 0, red);
         if (!B.any) break;
         todo = todo && !act;
         const int x0 = (B.lo[0] >> 1) - 1, y0 = (B.lo[1] >> 1) - 1, z0 = (B.lo[2] >> 1) - 1;
@@ -642,16 +693,16 @@ __device__ inline void wg_raise(float m, int* bound, int* red) {
 // take(a, k0, ex, exy, bx, by, bz, q0, q1, q2) reads the box for a particle whose first node
 // is at k0; done() follows a particle's three components. left(a, ...) is a component of a
 // particle that no box took (or that is not to be boxed).
-template <int CAP, class NodeMap, class Stage, class Take, class Left, class Done>
+template <int CAP, bool BOXED, class NodeMap, class Stage, class Take, class Left, class Done>
 __device__ __forceinline__ void over_boxes(bool live, bool boxed, float (&qo)[3], const NodeMap& map, int* red, int32_t* stab,
                                            Stage stage, Take take, Left left, Done done) {
     bool todo = live && boxed && NodeBoxes::fits(qo[0]) && NodeBoxes::fits(qo[1]) && NodeBoxes::fits(qo[2]);
     const bool far = live && !todo;
 #pragma unroll 1
-    for (int round = 0; round < BOX_ROUNDS; ++round) {
+    for (int left = BOXED ? NodeMap::boxes() : 0; left > 0; --left) {
         asm volatile("" : "+v"(qo[0]), "+v"(qo[1]), "+v"(qo[2]));   // as in k_p2g_tiled: nothing moved out of the loop
         bool act = todo;
-        const NodeBoxes B = fitting_boxes(act, qo, CAP, red);
+        const NodeBoxes B = fitting_boxes(act, qo, CAP, left, red);
         if (!B.any) break;
         todo = todo && !act;
         int lo[3], hi[3];
@@ -701,11 +752,11 @@ __device__ __forceinline__ void over_boxes(bool live, bool boxed, float (&qo)[3]
 // as float bits (for the deposit's scale). 1.6 M particles at 15 cm 176 -> 78 us against
 // reading the flags from global memory node by node.
 template <class NodeMap>
-__global__ __launch_bounds__(P2G_THREADS) void k_g2p_adj_reached(PView ps, int64_t n, NodeMap map, float lo0, float lo1, float lo2,
+__global__ __launch_bounds__(P2G_THREADS, 6) void k_g2p_adj_reached(PView ps, int64_t n, NodeMap map, float lo0, float lo1, float lo2,
                                                                  float dx, G2PFaces F, uint8_t* __restrict__ reached, PB12 pb,
                                                                  int* __restrict__ bound) {
     __shared__ float sflag[G2P_BOX];
-    __shared__ alignas(16) int red[6 * (P2G_THREADS / 64)];
+    __shared__ alignas(16) int red[BOX_RED];
     __shared__ int32_t stab[NodeMap::TAB];
     const int64_t p = (int64_t)xcd_tile(blockIdx.x, gridDim.x) * P2G_THREADS + threadIdx.x;
     const bool live = p < n;
@@ -716,7 +767,7 @@ __global__ __launch_bounds__(P2G_THREADS) void k_g2p_adj_reached(PView ps, int64
         qo[2] = ispace(ps.f[2][p], lo2, dx, 0.0f);
     }
     bool ok = true;
-    over_boxes<G2P_BOX>(
+    over_boxes<G2P_BOX, true>(
         live, true, qo, map, red, stab,
         [&](auto axis, int k, auto idx) {
             constexpr int a = decltype(axis)::value;
@@ -739,16 +790,19 @@ __global__ __launch_bounds__(P2G_THREADS) void k_g2p_adj_reached(PView ps, int64
         },
         [&](auto axis, const BSpline& bx, const BSpline& by, const BSpline& bz, float, float, float) {
             constexpr int a = decltype(axis)::value;
-            const float x0 = bx.w0, x1 = bx.w1, x2 = bx.w2, y0 = by.w0, y1 = by.w1, y2 = by.w2, z0 = bz.w0, z1 = bz.w1, z2 = bz.w2;
             float f = 0.0f;
 #pragma unroll 1
-            for (int q = 0; q < 27; ++q) {
-                const int mx = q % 3, my = (q / 3) % 3, mz = q / 9;
-                const auto idx = map.index(a, node_at(bx.b, mx), node_at(by.b, my), node_at(bz.b, mz));
-                if (NodeMap::HOLES && idx < 0) continue;
-                const float wgt = (mx == 0 ? x0 : (mx == 1 ? x1 : x2)) * (my == 0 ? y0 : (my == 1 ? y1 : y2)) *
-                                  (mz == 0 ? z0 : (mz == 1 ? z1 : z2));
-                f += wgt * (float)F.f[a][idx];
+            for (int r = 0; r < 9; ++r) {   // a row's three nodes are read together
+                const int my = r % 3, mz = r / 3;
+                float flag[3];
+#pragma unroll
+                for (int mx = 0; mx < 3; ++mx) {
+                    const auto idx = map.index(a, node_at(bx.b, mx), node_at(by.b, my), node_at(bz.b, mz));
+                    flag[mx] = !NodeMap::HOLES || idx >= 0 ? (float)F.f[a][idx] : -1.0f;
+                }
+#pragma unroll
+                for (int mx = 0; mx < 3; ++mx)
+                    if (!NodeMap::HOLES || flag[mx] >= 0.0f) f += pick(bx, mx) * pick(by, my) * pick(bz, mz) * flag[mx];
             }
             ok = ok && f > 0.999f;
         },
@@ -774,9 +828,10 @@ template <class NodeMap>
 __global__ __launch_bounds__(P2G_THREADS) void k_p2g_adj_gather(PView ps, int64_t n, NodeMap map, float lo0, float lo1, float lo2,
                                                                 float dx, float dt, AdjFaces S, PB12 pb) {
     __shared__ float sval[G2P_BOX];
-    __shared__ alignas(16) int red[6 * (P2G_THREADS / 64)];
+    __shared__ alignas(16) int red[BOX_RED];
     __shared__ int32_t stab[NodeMap::TAB];
-    const int64_t p = (int64_t)xcd_tile(blockIdx.x, gridDim.x) * P2G_THREADS + threadIdx.x;
+    const uint32_t tile = NodeMap::ADJ_BOXED ? xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
+    const int64_t p = (int64_t)tile * P2G_THREADS + threadIdx.x;
     const bool live = p < n;
     float qo[3] = {0.0f, 0.0f, 0.0f}, wT = 0.0f;
     if (live) {
@@ -785,7 +840,7 @@ __global__ __launch_bounds__(P2G_THREADS) void k_p2g_adj_gather(PView ps, int64_
         qo[2] = ispace(ps.f[2][p], lo2, dx, 0.0f);
         wT = temporal(ps.f[15][p], dt);
     }
-    over_boxes<G2P_BOX>(
+    over_boxes<G2P_BOX, NodeMap::ADJ_BOXED>(
         live, wT == wT, qo, map, red, stab,
         [&](auto axis, int k, auto idx) {   // (0 where there is no node: its terms vanish, unless wT is NaN)
             constexpr int a = decltype(axis)::value;
@@ -820,20 +875,29 @@ __global__ __launch_bounds__(P2G_THREADS) void k_p2g_adj_gather(PView ps, int64_
         },
         [&](auto axis, const BSpline& bx, const BSpline& by, const BSpline& bz, float q0, float q1, float q2) {
             constexpr int a = decltype(axis)::value;
-            const float x0 = bx.w0, x1 = bx.w1, x2 = bx.w2, y0 = by.w0, y1 = by.w1, y2 = by.w2, z0 = bz.w0, z1 = bz.w1, z2 = bz.w2;
             float v = 0.0f, c0 = 0.0f, c1 = 0.0f, c2 = 0.0f;
-#pragma unroll 1
-            for (int q = 0; q < 27; ++q) {
-                const int mx = q % 3, my = (q / 3) % 3, mz = q / 9;
-                const int I = node_at(bx.b, mx), J = node_at(by.b, my), K = node_at(bz.b, mz);
-                const auto idx = map.index(a, I, J, K);
-                if (idx < 0) continue;
-                const float t = wT * (mx == 0 ? x0 : (mx == 1 ? x1 : x2)) * (my == 0 ? y0 : (my == 1 ? y1 : y2)) *
-                                (mz == 0 ? z0 : (mz == 1 ? z1 : z2)) * S.s[a][idx];
-                v += t;
-                c0 += t * (((float)I - q0) * dx);
-                c1 += t * (((float)J - q1) * dx);
-                c2 += t * (((float)K - q2) * dx);
+            constexpr int PLANES = NodeMap::ADJ_BOXED ? 1 : 3;   // whose nodes are read together
+#pragma unroll PLANES
+            for (int mz = 0; mz < 3; ++mz) {
+                const int K = node_at(bz.b, mz);
+                float val[9];
+                int in = 0;
+#pragma unroll
+                for (int m = 0; m < 9; ++m) {
+                    const auto idx = map.index(a, node_at(bx.b, m % 3), node_at(by.b, m / 3), K);
+                    in |= (int)(idx >= 0) << m;
+                    val[m] = idx >= 0 ? S.s[a][idx] : 0.0f;
+                }
+#pragma unroll
+                for (int m = 0; m < 9; ++m) {
+                    if (!(in >> m & 1)) continue;
+                    const int mx = m % 3, my = m / 3;
+                    const float t = wT * pick(bx, mx) * pick(by, my) * pick(bz, mz) * val[m];
+                    v += t;
+                    c0 += t * (((float)node_at(bx.b, mx) - q0) * dx);
+                    c1 += t * (((float)node_at(by.b, my) - q1) * dx);
+                    c2 += t * (((float)K - q2) * dx);
+                }
             }
             pb.f[a][p] += v;
             pb.f[3 + 3 * a][p] += c0; pb.f[4 + 3 * a][p] += c1; pb.f[5 + 3 * a][p] += c2;

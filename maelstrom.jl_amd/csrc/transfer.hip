@@ -16,6 +16,11 @@ namespace mael {
 
 // flip.jl:513-537 p2g_kernel!: the tiled deposit over the dense grid's face arrays.
 struct DenseNodes {
+    // The adjoint's gather reads the faces directly: particles2grid_adjoint takes 265 us for
+    // 1.6 M particles on 256 x 256 x 128, in cell order and in two interleaved runs, and took
+    // 295 and 355 through boxes.
+    static constexpr bool ADJ_BOXED = false;
+    __device__ static int boxes() { return 0; }
     int n[3];
     __device__ int64_t index(int a, int I, int J, int K) const {
         int n1 = n[0] + (a == 0), n2 = n[1] + (a == 1), n3 = n[2] + (a == 2);
@@ -118,6 +123,12 @@ void DenseBasin::p2g(float dt) {
 
 // The gather's face nodes: indices clamped to the array (flip.jl:1210-1224).
 struct DenseClampNodes {
+    // Two boxes (a row of cells that crosses the funnel's ring), one while the launch's
+    // workgroups are all on the chip at once and its time is one's chain of boxes: 98,000
+    // particles in two interleaved runs 21 us with one box, 57 with up to four (18.9 and 18.4
+    // in cell order); 1.6 M 176 us with two, 211 with one and 186 with four (123, 163 and 125
+    // in cell order).
+    __device__ static int boxes() { return gridDim.x <= 512 ? 1 : 2; }
     static constexpr bool HOLES = false;
     int n[3];
     __device__ int64_t index(int a, int I, int J, int K) const {

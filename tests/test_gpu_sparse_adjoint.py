@@ -138,6 +138,43 @@ def test_sparse_p2g_adjoint_dot(M):
     assert _rel(lhs, rhs) < 1e-5, (lhs, rhs)
 
 
+def test_sparse_transfer_adjoints_any_order(M):
+    """A particle's part of the transfers' adjoints has the same bits in cell order (boxes of
+    faces) and shuffled (faces read directly), and so has the cotangent of the faces."""
+    print("case: sparse transfer adjoints in two orders", flush=True)
+    s = _basin(M)
+    rng = np.random.default_rng(6)
+    n = s.n
+    names = ["PX", "PY", "PZ", "LAG"] + VN + CN
+    ps = {f: s.get(f) for f in names}
+    for f in VN + CN:
+        ps[f] = rng.normal(0, 0.5, n).astype(np.float32)
+    pbar = {f: rng.normal(0, 1, n).astype(np.float32) for f in VN + CN}
+    ubar = _faces(s, rng)
+    fw = s.get("FW_F")
+    fw[rng.random(fw.shape) < 0.002] = 0
+    s.set("FW_F", fw)
+    got = []
+    for order in (np.arange(n), rng.permutation(n)):
+        for f in names:
+            s.set(f, ps[f][order])
+        M.sparse.particles2grid(s, 0.05)
+        for f in VN + CN:
+            s.set("PB_" + f, pbar[f][order])
+        M.sparse.grid2particles_adjoint(s, 0.05)
+        back = np.argsort(order)
+        out = [s.get("PB_" + f)[back] for f in VN + CN] + [s.get("UB_" + ax + "_F") for ax in AX]
+        for k, v in ubar.items():
+            s.set("UB_" + k, v)
+        for f in VN + CN:
+            s.set("PB_" + f, np.zeros(n, np.float32))
+        M.sparse.particles2grid_adjoint(s, 0.05)
+        got.append(out + [s.get("PB_" + f)[back] for f in VN + CN])
+    assert all(a.any() for a in got[0][-12:])
+    for a, b in zip(*got):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
 def test_sparse_project_adjoint_dot(M):
     print("case: sparse project adjoint", flush=True)
     s = _basin(M)

@@ -21,13 +21,15 @@ def _particles(rng, g, n, places):
     return ps
 
 
-# 1 and 7 clusters: one box and up to four; 200: left to the direct path. 1000 particles are
-# four workgroups, the last with 232.
-@pytest.mark.parametrize("n,places,off", [(1, 1, 0), (255, 1, 0), (257, 7, 1), (1000, 7, 0), (1000, 200, 3)])
+# 1 and 7 clusters: one box and up to four in the deposit; 200: left to the direct path. 1000
+# particles are four workgroups, the last with 232. 140,000 are 547, where the gather takes up
+# to two boxes: two clusters a workgroup, three or four, and five or six (left to the direct path).
+@pytest.mark.parametrize("n,places,off", [(1, 1, 0), (255, 1, 0), (257, 7, 1), (1000, 7, 0), (1000, 200, 3), (140000, 1094, 1),
+                                          (140000, 1800, 0), (140000, 2700, 3)])
 def test_boxes(mael, orc, ctx, n, places, off):
     print("case: boxes n=%d places=%d" % (n, places), flush=True)
     b = mael.Basin(radius=18.0, depth=12.0, Γ=225.0, core=2.5)
-    s = mael.FlipBasin(b, dx=0.6, capacity=2000)
+    s = mael.FlipBasin(b, dx=0.6, capacity=n + 1000)
     g, phi, u, v, w, _ = orc.dense_scene(18.0, 12.0, 3.0, 0.6, 225.0, 2.5)
     rng = np.random.default_rng(n + places)
     ps = _particles(rng, g, n, places)
@@ -66,11 +68,11 @@ def test_boxes(mael, orc, ctx, n, places, off):
 # A particle's part of the adjoints does not depend on its workgroup's other particles: in
 # shuffled order (up to 200 clusters a workgroup, most left to the direct path) it has the
 # same bits as in the clusters' order, and so has the cotangent of the faces (whole numbers).
-@pytest.mark.parametrize("n,places,off", [(1, 1, 0), (257, 7, 1), (1000, 7, 0), (1000, 200, 3)])
+@pytest.mark.parametrize("n,places,off", [(1, 1, 0), (257, 7, 1), (1000, 7, 0), (1000, 200, 3), (140000, 1800, 3)])
 def test_adjoint_boxes(mael, orc, ctx, n, places, off):
     print("case: adjoint boxes n=%d places=%d" % (n, places), flush=True)
     b = mael.Basin(radius=18.0, depth=12.0, Γ=225.0, core=2.5)
-    s = mael.FlipBasin(b, dx=0.6, capacity=2000)
+    s = mael.FlipBasin(b, dx=0.6, capacity=n + 1000)
     g = orc.dense_scene(18.0, 12.0, 3.0, 0.6, 225.0, 2.5)[0]
     rng = np.random.default_rng(n + places)
     ps = _particles(rng, g, n, places)
