@@ -52,8 +52,9 @@ DenseBasin::DenseBasin(const DGrid& grid, int lev, int64_t cap, int32_t bnd, int
         for (int a = 0; a < 3; ++a) lv[l].n[a] = g.n[a] >> l;
         if (l > 0) {
             size_t c = lv[l].cells();
-            lv[l].types.alloc(c); lv[l].x.alloc(c); lv[l].b.alloc(c); lv[l].r.alloc(c); lv[l].diag.alloc(c);
+            lv[l].types.alloc(c); lv[l].x.alloc(c); lv[l].b.alloc(c); lv[l].r.alloc(c);
         }
+        if (l > 0 || levels == 1) lv[l].diag.alloc(lv[l].cells());
     }
     size_t nparts = std::max<size_t>(1024, (size_t)cdiv(g.n[0] + 1, 64) * cdiv(g.n[1] + 1, 4) * (g.n[2] + 1));
     partials.alloc(nparts);

@@ -152,7 +152,7 @@ struct KTimer {
 struct DLevel {
     int n[3];
     DBuf<uint8_t> types;
-    DBuf<float> x, b, r, diag;   // diag: the LIQUID cells' diagonals, 0 elsewhere
+    DBuf<float> x, b, r, diag;   // diag: the LIQUID cells' neighbours that are not SOLID, 0 elsewhere
     size_t cells() const { return (size_t)n[0] * n[1] * n[2]; }
 };
 

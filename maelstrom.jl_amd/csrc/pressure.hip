@@ -117,8 +117,9 @@ __global__ void k_diag(float* __restrict__ diag, const uint8_t* __restrict__ typ
     diag[c] = d;
 }
 
-// flip.jl:838-848 celldiag of the coarse levels, up to CDIAG_LEVELS of them in one launch
-// (a level a row of workgroups): the neighbours that are not SOLID, 0 off the LIQUID cells.
+// flip.jl:838-848 celldiag of the coarse levels (and of a basin's only level, which the
+// coarsest solve takes like any other), up to CDIAG_LEVELS of them in one launch (a level a
+// row of workgroups): the neighbours that are not SOLID, 0 off the LIQUID cells.
 constexpr int CDIAG_LEVELS = 8;
 struct CoarseDiags {
     float* d[CDIAG_LEVELS];
@@ -501,7 +502,7 @@ struct DenseSolver {
     bool tiled(int l, int sweeps) const { return sweeps == 2 && s.lv[l].cells() <= RB_TILED; }
     unsigned tiles(int l) const { return cdiv(s.lv[l].n[0], RB) * cdiv(s.lv[l].n[1], RB) * cdiv(s.lv[l].n[2], RB); }
     float* scratch(int l) { return l == 0 ? s.rv.p : s.lv[l].r.p; }
-    const float* cdiag(int l) const { return l == 0 ? s.diag.p : s.lv[l].diag.p; }
+    const float* cdiag(int l) const { return l == 0 && L > 1 ? s.diag.p : s.lv[l].diag.p; }
     void down(int l, const float* b) {
         hipLaunchKernelGGL(k_rbdown, dim3(tiles(l)), dim3(RB_THREADS), 0, st, scratch(l), s.lv[l + 1].b.p, b, cdiag(l), types(l),
                            types(l + 1), dims(l), dims(l + 1));
@@ -689,10 +690,10 @@ void DenseBasin::operator_setup() {
         hipLaunchKernelGGL(k_coarsen, grid3(nc.x, nc.y, nc.z), dim3(BX, BY), 0, s, lv[l].types.p, S.types(l - 1), nc, nf);
     }
     hipLaunchKernelGGL(k_diag, grid3(n.x, n.y, n.z), dim3(BX, BY), 0, s, diag.p, types.p, phi.p, n);
-    for (int l = 1; l < levels; l += CDIAG_LEVELS) {
+    for (int l = levels == 1 ? 0 : 1; l < levels; l += CDIAG_LEVELS) {
         CoarseDiags A;
         const int m = std::min(CDIAG_LEVELS, levels - l);
-        for (int q = 0; q < m; ++q) { A.d[q] = lv[l + q].diag.p; A.t[q] = lv[l + q].types.p; A.n[q] = i3(lv[l + q].n); }
+        for (int q = 0; q < m; ++q) { A.d[q] = lv[l + q].diag.p; A.t[q] = S.types(l + q); A.n[q] = i3(lv[l + q].n); }
         hipLaunchKernelGGL(k_coarsediag, dim3(cdiv(lv[l].cells(), 256), m), dim3(256), 0, s, A);
     }
     MAEL_LAUNCH_CHECK();

@@ -54,18 +54,25 @@ DENSE = {
     "tile remainders and a 4,840-cell tail, 44x44x20 .. 11x11x5": (4.0, 2.0, 1.5, 0.2, (44, 44, 20)),
     "a level too wide for the tail, 128x128x4 .. 32x32x1": (36.9, 0.6, 0.9, 0.6, (128, 128, 4)),
     "tiles off by half, 40x40x24 .. 10x10x6": (10.2, 8.0, 5.0, 0.6, (40, 40, 24)),
+    "two levels, the tail the whole V-cycle, 18x18x8 .. 9x9x4": (4.0, 2.0, 1.5, 0.6, (18, 18, 8)),
+    "one level, the coarsest solve alone, 9x8x7": (4.0, 2.0, 1.5, 0.6, (9, 8, 7)),
 }
 
 
 @pytest.mark.parametrize("sweeps,queued", [(1, 0), (2, 0), (2, 1), (3, 1)])
 @pytest.mark.parametrize("case", sorted(DENSE))
-def test_dense_levels_bits(mael, orc, case, sweeps, queued):
+def test_dense_levels_bits(mael, orc, monkeypatch, case, sweeps, queued):
     """The dense basin's V-cycle on random cell types (empty rows and single-cell pools among
     them) in the oracle's FP32 V-cycle's bits: both take every sum and division in the
     reference's order."""
     radius, depth, top, dx, dims = DENSE[case]
     print("case: %s sweeps %d queued %d" % (case, sweeps, queued), flush=True)
     g = orc.flipgrid(radius, depth, top, dx)
+    if case.startswith("one level"):   # flipgrid makes two or more; the C ABI takes one
+        g.n[:], g.levels = dims, 1
+        one = mael.flipgrid(mael.Basin(radius=radius, depth=depth, rimwall=top), dx)
+        one.n[:], one.levels = dims, 1
+        monkeypatch.setattr(mael.dense, "flipgrid", lambda *a: one)
     assert g.dims == dims
     s = mael.FlipBasin(mael.Basin(radius=radius, depth=depth, rimwall=top), dx=dx, capacity=16)
     rng = np.random.default_rng(3)
