@@ -370,9 +370,12 @@ __device__ inline void stage27(const STopo& t, int4 w, int32_t* s27) {
 }
 
 // The kernels that go over a slot's 17 x 256 faces take them in one workgroup's 17 rounds
-// (a number the compiler knows: their template parameter) while those workgroups fill half
-// of the chip's 2048 places (8 a CU), else a workgroup a round. 60 cm, 120 slots: a
-// projection's difference 17 us with one workgroup a slot, 4 with 17.
+// (a number the compiler knows: their template parameter) where those workgroups fill half
+// of the chip's 2048 places (8 a CU), else a workgroup a round. With one workgroup a slot
+// and with 17, us: a projection's difference 24 and 12 for 408 slots, 28 and 20 for 876, 33
+// and 30 for 1,344; the walls' faces 6.1 and 4.1, 7.2 and 6.3, 7.7 and 8.0; a layer of the
+// extrapolation (three axes) 40 and 16, 51 and 34, 59 and 57. The couplings (k_finecoef)
+// always take a workgroup a slot: 16 and 19 for 84 slots, 30 and 45 for 876.
 constexpr int SLOT_ROUNDS = 17;
 inline bool slots_few(int groups) { return groups <= 1024; }
 

@@ -79,15 +79,12 @@ struct SlotFaces {
     }
 };
 
-// A workgroup (or one a round, slots_few) per live slot (block order): 256 of its faces along
-// a a round.
-template <int ROUNDS>
+// A workgroup per live slot (block order), a thread per 17 of its faces along a.
 __global__ __launch_bounds__(256) void k_finecoef(float* __restrict__ c, const uint8_t* __restrict__ tf,
                                                   const uint8_t* __restrict__ tc, STopo t, int a,
                                                   const int32_t* __restrict__ order) {
     const SlotFaces F(t, order[blockIdx.x], a);
-    for (int q = 0; q < ROUNDS; ++q) {
-        const int r = ROUNDS == 1 ? (int)blockIdx.y : q;
+    for (int r = 0; r < SLOT_ROUNDS; ++r) {
         const int f = r * 256 + (int)threadIdx.x;
         int i, j, k;
         F.face(f, i, j, k);
@@ -1915,7 +1912,8 @@ struct SVec {   // a pressure-sized vector: fine pool part and coarse part
 // MG_SMALL cells. At 2.9 M cells (FP16) the halo's repeated rows cost more than the saved
 // passes gain (two tiled launches against five took as long when a pass took 15 us; it takes
 // 10 now); at 368,640 the two are even (a 5 cm solve 14.80 ms tiled, 14.76 with a launch a
-// pass), and the tiles make fewer launches. 8^3 tiles put a level of up to 80,000 cells on more
+// pass), at 442,368 a V-cycle takes 223 us tiled and 229 not (FP16 300 and 307), at 602,112
+// 246 and 253 (323 and 330), and the tiles make fewer launches. 8^3 tiles put a level of up to 80,000 cells on more
 // CUs: 144 workgroups for 73,728 cells, where 16x8x8 would make 72.
 constexpr size_t MG_TILED = 500000, MG_SMALL = 80000;
 
@@ -1934,8 +1932,7 @@ struct SparseSolver {
     void coefficients() {
         for (int a = 0; a < 3; ++a) {
             if (s.nlive > 0)
-                hipLaunchKernelGGL(slots_few(s.nlive) ? k_finecoef<1> : k_finecoef<SLOT_ROUNDS>,
-                                   dim3((unsigned)s.nlive, slots_few(s.nlive) ? SLOT_ROUNDS : 1), dim3(256), 0, st, s.cf[a].p, s.types.fine.p,
+                hipLaunchKernelGGL(k_finecoef, dim3((unsigned)s.nlive), dim3(256), 0, st, s.cf[a].p, s.types.fine.p,
                                    s.types.coarse.p, t, a, s.sorder.p);
             hipLaunchKernelGGL(k_coarsecoef, dim3(cdiv(s.nfaces(a), 256)), dim3(256), 0, st, s.cc[a].p, s.types.coarse.p, t, a);
         }
