@@ -466,12 +466,13 @@ static inline dim3 grid3(int n1, int n2, int n3) { return dim3(cdiv(n1, BX), cdi
 static inline int3 i3(const int n[3]) { return make_int3(n[0], n[1], n[2]); }
 constexpr int RED_BLOCKS = 1024;   // workgroups of the 1-D reductions
 
-// Levels of at most RB_TILED cells take a launch down and one up: a level of 131,072 cells
-// is 256 tiles, one a CU (a backward pass on 128x128x64 1,700 us, 1,845 us with that level a
-// launch a pass), and one of 1 M cells is 2,048 of them (1,890 us tiled there too). The
+// Levels of at most RB_TILED cells take a launch down and one up. A whole V-cycle, us, with
+// its first level a launch a pass and tiled: 119 and 90 at 131,072 cells (256 tiles, one a
+// CU), 131 and 109 at 294,912, 146 and 133 at 442,368, 139 and 129 at 524,288, 159 and 154 at
+// 786,432; at 1 M cells 186 and 175, but a backward pass on 128x128x64 1,887 and 1,890. The
 // one-workgroup tail holds a level of RB_TAIL_SMALL or RB_TAIL_CELLS cells with the layer
 // round it.
-constexpr size_t RB_TILED = 300000;
+constexpr size_t RB_TILED = 600000;
 constexpr int RB_TAIL_SMALL = 4096, RB_TAIL_CELLS = 12288;
 
 struct DenseSolver {

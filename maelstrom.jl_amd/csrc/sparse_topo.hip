@@ -641,10 +641,11 @@ void SparseBasin::gravity(float dt, float gacc) {
 // ─── redistancing (sflip.jl:833-919) ─────────────────────────────────────────
 
 // A workgroup per slot, or per KP of its 16 planes where the slots alone leave the chip idle
-// (up to 512 live; 120: 22 us with one, 9 with four): the block's values there and the layers across its sides
-// (the block's own planes, else the neighbour's, else the coarse cell where there is no
-// block, as in the reference's nphi) are staged in LDS once, then each thread takes a KP-cell
-// column along z. A block clear of the walls skips the solid tests.
+// (slots_few; with one and with four, us: 28 and 18 for 408 slots, 35 and 26 for 876, 44 and
+// 35 for 1,344): the block's values there and the layers across its sides (the block's own
+// planes, else the neighbour's, else the coarse cell where there is no block, as in the
+// reference's nphi) are staged in LDS once, then each thread takes a KP-cell column along z.
+// A block clear of the walls skips the solid tests.
 template <int KP>
 __global__ __launch_bounds__(256) void k_sreinit(float* __restrict__ out, const float* __restrict__ phi,
                                                  const float* __restrict__ phic, STopo t, float phimax,
@@ -778,8 +779,8 @@ void SparseBasin::redistance(int iterations) {
     hipStream_t s = st.s;
     for (int it = 0; it < iterations && nslots > 0; ++it) {
         if (nlive > 0)   // free slots keep what they hold in both copies: nothing reads them
-            hipLaunchKernelGGL(nlive <= 512 ? k_sreinit<4> : k_sreinit<16>, dim3((unsigned)nlive, nlive <= 512 ? 4 : 1), dim3(256),
-                               0, s, phi0.fine.p, phi.fine.p, phi.coarse.p, topo(), phimax, sorder.p);
+            hipLaunchKernelGGL(slots_few(nlive) ? k_sreinit<4> : k_sreinit<16>, dim3((unsigned)nlive, slots_few(nlive) ? 4 : 1),
+                               dim3(256), 0, s, phi0.fine.p, phi.fine.p, phi.coarse.p, topo(), phimax, sorder.p);
         std::swap(phi.fine, phi0.fine);
     }
     hipLaunchKernelGGL(k_coarsewall, dim3(cdiv(ncells(), 256)), dim3(256), 0, s, phi0.coarse.p, phi.coarse.p, topo());
