@@ -17,6 +17,7 @@
 #pragma once
 #include "sparse.hpp"
 #include "precision.hpp"
+#include "quotient.hpp"
 
 namespace mael {
 
@@ -194,16 +195,6 @@ __global__ __launch_bounds__(MG_THREADS) void k_mgup(T* __restrict__ out, const 
 
 // ─── the last levels in one workgroup ────────────────────────────────────────
 
-// acc / d correctly rounded, from r = 1 / d: FP32 through FP64 (a quotient of two 24-bit
-// numbers is never so close to a rounding boundary as FP64's error), FP64 by two Newton
-// corrections of the quotient, each with the exact remainder of a fused multiply-add.
-__device__ inline float quotient(float acc, float, double r) { return (float)((double)acc * r); }
-__device__ inline double quotient(double acc, double d, double r) {
-    double q = acc * r;
-    q = __builtin_fma(__builtin_fma(-q, d, acc), r, q);
-    return __builtin_fma(__builtin_fma(-q, d, acc), r, q);
-}
-
 // The tail: up to three levels, the first of at most 2 THREADS cells, each next an eighth.
 // Bound by the 160 passes of the coarsest solve, one LDS round trip and barrier each: 1,152
 // and 144 FP32 cells 26 us, 512 cells 23 us (28 us with a thread per cell and a division a
@@ -293,7 +284,7 @@ __device__ inline void mg_rise(Fine& F, int3 nf, const Coarse& K, int3 nc, float
 // sflip.jl:1623-1657 coarsest_kernel!: red-black Gauss-Seidel from zero in arithmetic A
 // (FP64 in the mixed-precision solve), `sweeps` passes and as many in reverse colour order.
 // A thread has a cell of each colour of a row, so half the threads do a pass and the fewer
-// wavefronts meet sooner; the division by the same diagonal each pass is a product.
+// wavefronts meet sooner; the division by the same diagonal each pass is a product (quotient.hpp).
 template <class T, class A, int THREADS, class C, class Local>
 __device__ inline void mg_coarsest(Local& K, const DViewT<C>& L, A* X, const float* bs, int sweeps) {
     const int n0 = L.n.x, n1 = L.n.y, n2 = L.n.z, hx = (n0 + 1) >> 1, t = (int)threadIdx.x;

@@ -17,6 +17,7 @@
 // 256 cells) 21.8 us, against 58 us in twelve. A 64x64x32 solve 1,430 -> 707 us.
 #pragma once
 #include "dense.hpp"
+#include "quotient.hpp"
 #include <type_traits>
 
 namespace mael {
@@ -28,10 +29,6 @@ __device__ inline float rb_diag(const float* __restrict__ dg, const uint8_t* __r
     const float d = dg[l];
     return types[l] == LIQUID ? d : -1.0f;
 }
-
-// acc / d from r = 1 / d in FP64: a quotient of two 24-bit numbers is never so close to a
-// rounding boundary as FP64's error, so this is the correctly rounded division.
-__device__ inline float rb_quotient(float acc, double r) { return (float)((double)acc * r); }
 
 // A tile and H cells round it in LDS. The cells of one colour are numbered in rows of
 // pairs, and thread t has those numbered t, t + RB_THREADS, ...
@@ -228,7 +225,7 @@ struct RBLevel {
 // flip.jl:931-962 coarse_kernel!: `sweeps` sweeps from zero and as many in reverse colour
 // order, from the right-hand side in v (which becomes the result). A thread has a cell of
 // each colour of a row, so half the threads do a pass and the fewer wavefronts meet sooner,
-// and the division by the same diagonal each pass is a product.
+// and the division by the same diagonal (a count of neighbours) each pass is a product.
 __device__ inline void rb_coarsest(float* v, const float* dg, int3 n, int sweeps) {
     const int sx = n.x + 2, sxy = sx * (n.y + 2), hx = (n.x + 1) >> 1, t = (int)threadIdx.x;
     const int h = t % hx, j = (t / hx) % n.y, k = t / (hx * n.y);
@@ -259,7 +256,7 @@ __device__ inline void rb_coarsest(float* v, const float* dg, int3 n, int sweeps
             float acc = bv[c];
 #pragma unroll
             for (int m = 0; m < 6; ++m) acc += w[m];
-            v[at[c]] = rb_quotient(acc, rc[c]);
+            v[at[c]] = quotient_small(acc, rc[c]);
         }
         __syncthreads();
     };
