@@ -18,6 +18,7 @@
 #include "sparse.hpp"
 #include "precision.hpp"
 #include "quotient.hpp"
+#include <type_traits>
 
 namespace mael {
 
@@ -285,6 +286,9 @@ __device__ inline void mg_rise(Fine& F, int3 nf, const Coarse& K, int3 nc, float
 // (FP64 in the mixed-precision solve), `sweeps` passes and as many in reverse colour order.
 // A thread has a cell of each colour of a row, so half the threads do a pass and the fewer
 // wavefronts meet sooner; the division by the same diagonal each pass is a product (quotient.hpp).
+// An FP32 solve that came upon a subnormal quotient, where the product may round the wrong
+// way, is made again with divisions: to look at each quotient at once and divide took 36 us
+// instead of 29 for 1,152 and 144 cells.
 template <class T, class A, int THREADS, class C, class Local>
 __device__ inline void mg_coarsest(Local& K, const DViewT<C>& L, A* X, const float* bs, int sweeps) {
     const int n0 = L.n.x, n1 = L.n.y, n2 = L.n.z, hx = (n0 + 1) >> 1, t = (int)threadIdx.x;
@@ -312,23 +316,43 @@ __device__ inline void mg_coarsest(Local& K, const DViewT<C>& L, A* X, const flo
         }
         dg[colour] = d;
         rc[colour] = d > A(0) ? 1.0 / (double)d : 0.0;
+        act[colour] = act[colour] && d > A(0);   // (an empty row keeps its 0)
         if (in) X[at[colour]] = A(0);
     }
     __syncthreads();
-    auto pass = [&](int c) {
-        if (act[c]) {
-            A v[6];
+    auto solve = [&](auto divide) {
+        auto pass = [&](int c) {
+            if (act[c]) {
+                A v[6];
 #pragma unroll
-            for (int q = 0; q < 6; ++q) v[q] = X[nb[c][q]];
-            A acc = bi[c];
+                for (int q = 0; q < 6; ++q) v[q] = X[nb[c][q]];
+                A acc = bi[c];
 #pragma unroll
-            for (int q = 0; q < 6; ++q) acc += cw[c][q] * v[q];
-            X[at[c]] = dg[c] > A(0) ? quotient(acc, dg[c], rc[c]) : A(0);
-        }
-        __syncthreads();
+                for (int q = 0; q < 6; ++q) acc += cw[c][q] * v[q];
+                X[at[c]] = divide(acc, c);
+            }
+            __syncthreads();
+        };
+        for (int s = 0; s < sweeps; ++s) { pass(0); pass(1); }
+        for (int s = 0; s < sweeps; ++s) { pass(1); pass(0); }
     };
-    for (int s = 0; s < sweeps; ++s) { pass(0); pass(1); }
-    for (int s = 0; s < sweeps; ++s) { pass(1); pass(0); }
+    if constexpr (std::is_same<A, float>::value) {
+        uint32_t least = ~0u;
+        solve([&](float acc, int c) {
+            const float q = quotient(acc, dg[c], rc[c]);
+            least = min(least, subnormal_rank(q));
+            return q;
+        });
+        if (__syncthreads_or(least < SUBNORMALS)) {
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+                if (act[c]) X[at[c]] = 0.0f;
+            __syncthreads();
+            solve([&](float acc, int c) { return acc / dg[c]; });
+        }
+    } else {
+        solve([&](A acc, int c) { return quotient(acc, dg[c], rc[c]); });
+    }
     K.each([&](int m, int e) { K.x[e] = lf(sf<T>((float)X[e])); });
 }
 

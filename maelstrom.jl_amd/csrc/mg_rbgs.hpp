@@ -256,7 +256,7 @@ __device__ inline void rb_coarsest(float* v, const float* dg, int3 n, int sweeps
             float acc = bv[c];
 #pragma unroll
             for (int m = 0; m < 6; ++m) acc += w[m];
-            v[at[c]] = quotient_small(acc, rc[c]);
+            v[at[c]] = quotient(acc, 0.0f, rc[c]);
         }
         __syncthreads();
     };

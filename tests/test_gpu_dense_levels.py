@@ -48,6 +48,33 @@ def test_levels_match_oracle(mael, case, precision, sweeps):
     assert err < {0: 1e-5, 1: 3e-3, 2: 2e-2}[precision], err
 
 
+def test_levels_subnormal(mael):
+    """A right-hand side of 2^-140 and below: the coarsest solve meets subnormal quotients and is
+    made again with divisions. Its values are some hundreds of the smallest number, to half of
+    one in each of a few tens of passes."""
+    radius, depth, dims = CASES["one level, 16^3 halved once"]
+    print("case: subnormal right-hand side", flush=True)
+    o = O.SparseOracle(radius, depth, 3.0, 0.6, 2, 1, 16, 4, 8)
+    g = o.grid
+    rmax = np.float32(np.hypot(np.float32(g.lo[0]), np.float32(g.lo[1])))
+    o.init_coarse(O.surface_table(225.0, 2.5, 9.81, rmax), rmax, 225.0, 2.5)
+    o.classify()
+    s = mael.SparseBasin(mael.Basin(radius=radius, depth=depth, Γ=225.0, core=2.5), dx=0.6, blocks=1, capacity=16)
+    assert s.nc == dims
+    s.set("PHI_C", o.array("phi_c"))
+    s.set("TYPES_C", o.array("types_c"))
+    rng = np.random.default_rng(8)
+    rc = np.where(o.array("types_c") == 1, rng.uniform(0, 2.0 ** -140, o.array("types_c").size), 0).astype(np.float32)
+    s.set("RHS_C", rc)
+    opts = mael.sparse.solve_options(precision=0, boost=1.0, sweeps=1)
+    s.ctx.check(mael.lib().mael_sparse_vcycle(s.h, C.byref(opts), 0))
+    z = s.get("P_C").ravel().astype(np.float64)
+    _, ze = o.vcycle(np.zeros(o.array("P_f").size, np.float32), rc, sweeps=1, coarse=opts.coarse, boost=1.0)
+    err = np.linalg.norm(z - ze) / np.linalg.norm(ze)
+    print("rel L2 vs FP64 oracle %.3e, largest %.3g units" % (err, np.abs(ze).max() * 2.0 ** 149), flush=True)
+    assert err < 2e-2, err
+
+
 # radius, depth, top, dx -> cells; the dense V-cycle's levels halve them to at most 1024
 DENSE = {
     "tiles and a 2,048-cell tail, 64x64x32 .. 8x8x4": (18.0, 12.0, 3.0, 0.6, (64, 64, 32)),

@@ -1,5 +1,5 @@
 """The coarsest solves' division by a known diagonal (csrc/quotient.hpp), compiled for the host,
-against the division itself."""
+against the division itself. An FP32 quotient is right or told as subnormal."""
 import ctypes as C
 import os
 import subprocess
@@ -14,10 +14,13 @@ SOURCE = r"""
 #include "quotient.hpp"
 #include <cstdint>
 #include <cstring>
+static bool told(float q) { return mael::subnormal_rank(q) < mael::SUBNORMALS; }
+static bool told(double) { return false; }
 template <class T, class B> static int64_t wrong(const T* a, const T* d, int64_t n) {
     int64_t w = 0;
     for (int64_t k = 0; k < n; ++k) {
         const T q = mael::quotient(a[k], d[k], 1.0 / (double)d[k]), e = a[k] / d[k];
+        if (told(q)) continue;   // (FP32: the solve then divides)
         B x, y;
         std::memcpy(&x, &q, sizeof q);
         std::memcpy(&y, &e, sizeof e);
@@ -27,6 +30,7 @@ template <class T, class B> static int64_t wrong(const T* a, const T* d, int64_t
 }
 extern "C" int64_t wrong32(const float* a, const float* d, int64_t n) { return wrong<float, uint32_t>(a, d, n); }
 extern "C" int64_t wrong64(const double* a, const double* d, int64_t n) { return wrong<double, uint64_t>(a, d, n); }
+extern "C" int is_told(float q) { return told(q); }
 // every FP32 numerator whose quotient by 1 .. 6 is subnormal or the smallest normal
 extern "C" int64_t wrong_small() {
     int64_t w = 0;
@@ -34,7 +38,7 @@ extern "C" int64_t wrong_small() {
         for (uint32_t b = 0;; ++b) {
             float a;
             std::memcpy(&a, &b, 4);
-            const float q = mael::quotient_small(a, 1.0 / d), e = a / (float)d;
+            const float q = mael::quotient(a, 0.0f, 1.0 / d), e = a / (float)d;
             w += std::memcmp(&q, &e, 4) != 0;
             if (e > 1.17549435e-38f) break;
         }
@@ -52,6 +56,7 @@ def lib(tmp_path_factory):
     for f, t in ((L.wrong32, C.c_float), (L.wrong64, C.c_double)):
         f.restype, f.argtypes = C.c_int64, [C.POINTER(t), C.POINTER(t), C.c_int64]
     L.wrong_small.restype = C.c_int64
+    L.is_told.argtypes = [C.c_float]
     return L
 
 
@@ -74,13 +79,16 @@ def test_fp32(lib):
     u, m = 2 * rng.integers(1, 1 << 12, n) + 1, 2 * rng.integers(0, 1 << 10, n) + 1
     s = rng.integers(2, 14, n)
     assert _wrong(lib.wrong32, u * m * 2.0 ** (s - 150), u * 2.0 ** s) == 0
-    z = np.array([0.0, -0.0, 0.0, np.inf, -np.inf, np.nan])
-    with np.errstate(all="ignore"):
-        a, e = z.astype(np.float32), np.full(6, 3, np.float32)
-    assert _wrong(lib.wrong32, a[:5], e[:5]) == 0
+    assert _wrong(lib.wrong32, [0.0, -0.0, np.inf, -np.inf], [3.0] * 4) == 0
+
+
+def test_subnormal_is_told(lib):
+    q = np.array([0, -0.0, 2.0 ** -149, -2.0 ** -149, 2.0 ** -126 - 2.0 ** -149, 2.0 ** -126, -1, np.inf, np.nan], np.float32)
+    assert [bool(lib.is_told(float(x))) for x in q] == [False, False, True, True, True, False, False, False, False]
 
 
 def test_fp32_small_diagonals(lib):
+    """A count of neighbours as the diagonal: right whatever the quotient."""
     assert lib.wrong_small() == 0
 
 
