@@ -31,8 +31,7 @@ __device__ inline int wave_min(int v) {
 #undef MAEL_DPP_MIN
     return __builtin_amdgcn_readlane(v, 63);
 }
-__device__ inline int wave_max(int v) { return -wave_min(-v); }
-// K workgroup minima at once (one pair of barriers); red holds K x (P2G_THREADS / 64).
+// K workgroup minima at once (one pair of barriers); red, 16-byte aligned, holds K x (P2G_THREADS / 64).
 template <int K> __device__ inline void wg_mins(int (&v)[K], int* red) {
 #pragma unroll
     for (int k = 0; k < K; ++k) v[k] = wave_min(v[k]);
@@ -46,16 +45,6 @@ template <int K> __device__ inline void wg_mins(int (&v)[K], int* red) {
         const int4 r = *reinterpret_cast<const int4*>(red + 4 * k);
         v[k] = min(min(r.x, r.y), min(r.z, r.w));
     }
-}
-// The workgroup's bounds of (b0, b1, b2) over the `ok` lanes: x0 y0 z0 (BIG if none), x1 y1 z1.
-// red is 16-byte aligned.
-__device__ inline void wg_bounds(bool ok, int b0, int b1, int b2, int* red, int& x0, int& y0, int& z0, int& x1, int& y1,
-                                 int& z1) {
-    const int BIG = 1 << 30;
-    int v[6] = {ok ? b0 : BIG, ok ? b1 : BIG, ok ? b2 : BIG, ok ? -b0 : BIG, ok ? -b1 : BIG, ok ? -b2 : BIG};
-    wg_mins(v, red);
-    x0 = v[0]; y0 = v[1]; z0 = v[2];
-    x1 = v[3] == BIG ? -BIG : -v[3]; y1 = v[4] == BIG ? -BIG : -v[4]; z1 = v[5] == BIG ? -BIG : -v[5];
 }
 // (i, j, k) of entry l of a box of ex x ey columns: the quotients from float reciprocals,
 // exact for l < 2^21 (a quotient's distance from an integer, 1 / (2 ex), exceeds its
@@ -290,7 +279,7 @@ __global__ __launch_bounds__(P2G_THREADS, 4) void k_p2g_tiled(PView ps, int64_t 
         todo = todo && !act;
         int lo[3], hi[3];
         B.nodes(lo, hi);
-        const typename NodeMap::Near near = map.near(true, lo, hi);
+        const typename NodeMap::Near near = map.near(lo, hi);
         map.stage(near, stab);
         auto component = [&](auto axis) __attribute__((always_inline)) {
             constexpr int a = decltype(axis)::value;
@@ -436,7 +425,7 @@ __global__ __launch_bounds__(P2G_THREADS, 4) void k_g2p_tiled(PView ps, int64_t 
         todo = todo && !act;
         int lo[3], hi[3];
         B.nodes(lo, hi);
-        const typename NodeMap::Near near = map.near(true, lo, hi);
+        const typename NodeMap::Near near = map.near(lo, hi);
         map.stage(near, stab);
         __syncthreads();
         float rec[12];
@@ -612,7 +601,7 @@ __global__ __launch_bounds__(P2G_THREADS) void k_splat_tiled(PView ps, int64_t n
         const int x0 = (B.lo[0] >> 1) - 1, y0 = (B.lo[1] >> 1) - 1, z0 = (B.lo[2] >> 1) - 1;
         const int ex = ((B.hi[0] - B.lo[0]) >> 1) + 3, ey = ((B.hi[1] - B.lo[1]) >> 1) + 3, ez = ((B.hi[2] - B.lo[2]) >> 1) + 3;
         const int lo[3] = {x0, y0, z0}, hi[3] = {x0 + ex - 1, y0 + ey - 1, z0 + ez - 1};
-        const typename CellMap::Near near = map.near(true, lo, hi);
+        const typename CellMap::Near near = map.near(lo, hi);
         map.stage(near, stab);
         const int V = ex * ey * ez;
         // a thread clears the entries that it flushed before
@@ -707,7 +696,7 @@ __device__ __forceinline__ void over_boxes(bool live, bool boxed, float (&qo)[3]
         todo = todo && !act;
         int lo[3], hi[3];
         B.nodes(lo, hi);
-        const typename NodeMap::Near near = map.near(true, lo, hi);
+        const typename NodeMap::Near near = map.near(lo, hi);
         map.stage(near, stab);
         __syncthreads();
         auto component = [&](auto axis) __attribute__((always_inline)) {

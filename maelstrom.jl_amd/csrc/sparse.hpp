@@ -85,10 +85,10 @@ struct BlockTab {
     static constexpr int CAP = 64;
     int x, y, z, nx, ny, nz;
     bool use;
-    __device__ BlockTab(bool any, const int lo[3], const int hi[3]) {
+    __device__ BlockTab(const int lo[3], const int hi[3]) {
         x = (lo[0] - 1) >> 4; y = (lo[1] - 1) >> 4; z = (lo[2] - 1) >> 4;
         nx = (hi[0] >> 4) - x + 1; ny = (hi[1] >> 4) - y + 1; nz = (hi[2] >> 4) - z + 1;
-        use = any && nx <= CAP && ny <= CAP && nz <= CAP && nx * ny * nz <= CAP;
+        use = nx <= CAP && ny <= CAP && nz <= CAP && nx * ny * nz <= CAP;
     }
     __device__ void stage(const STopo& t, int32_t* tab) const {
         const int k = (int)threadIdx.x;
@@ -123,7 +123,7 @@ struct SparseNodes {
     __device__ int32_t index(int a, int I, int J, int K) const { return finefaceat(t, a, I, J, K); }
     static constexpr int TAB = BlockTab::CAP;
     using Near = BlockTab;
-    __device__ Near near(bool any, const int lo[3], const int hi[3]) const { return BlockTab(any, lo, hi); }
+    __device__ Near near(const int lo[3], const int hi[3]) const { return BlockTab(lo, hi); }
     __device__ void stage(const Near& b, int32_t* tab) const { b.stage(t, tab); }
     __device__ int32_t at(const Near& b, const int32_t* tab, int a, int I, int J, int K) const {
         return b.use ? b.face(tab, a, I, J, K) : index(a, I, J, K);

@@ -194,7 +194,7 @@ struct FineCellMap {
     __device__ int32_t index(int I, int J, int K) const { return fineat(t, I, J, K); }
     static constexpr int TAB = BlockTab::CAP;
     using Near = BlockTab;
-    __device__ Near near(bool any, const int lo[3], const int hi[3]) const { return BlockTab(any, lo, hi); }
+    __device__ Near near(const int lo[3], const int hi[3]) const { return BlockTab(lo, hi); }
     __device__ void stage(const Near& b, int32_t* tab) const { b.stage(t, tab); }
     __device__ int32_t at(const Near& b, const int32_t* tab, int I, int J, int K) const {
         return b.use ? b.cell(tab, I, J, K) : index(I, J, K);

@@ -333,7 +333,6 @@ __global__ void k_cellsdense(float* __restrict__ dDc, uint8_t* __restrict__ actc
 // one. Arithmetic is FP32 either way (the coarsest level's in A).
 
 template <class C> struct FineCoefT { const C* c[3]; };
-template <class C> struct CoarseCoefT { const C* c[3]; };
 
 // The slot of block w's face neighbour d (-x, +x, -y, +y, -z, +z), 0 for none.
 __device__ inline int32_t nbslot(const STopo& t, int4 w, int d) {
@@ -344,27 +343,24 @@ __device__ inline int32_t nbslot(const STopo& t, int4 w, int d) {
 
 // Level 0's couplings follow from the cell types (k_finecoef, k_coarsecoef,
 // sflip.jl:1323-1353): for a LIQUID uncovered cell, 4 to an uncovered LIQUID coarse
-// neighbour and 0.4 to a LIQUID fine cell across a sub-face, else 0. With `ty` set
-// (level 0), a coarse row takes them from the types (ty->tf fine, ty->tc coarse) instead of
-// the coupling arrays: the same values as the FP32 arrays hold.
-struct LevelTypes { const uint8_t* tf; const uint8_t* tc; };
-// A level's fine cell (N = 16 or 8) of slot s: diag and the neighbours' sum, A x = diag x
-// - off, summed in A (FP32, or FP64 for iterative refinement's residual). Neighbours in
-// the block index directly; across a face they are the neighbour block's (slots in nb)
-// or, without one, the coarse cell's. Every index is computed and all thirteen loads are
-// issued before any value is used (each index is in bounds whatever the couplings); a
-// coupling that is not positive adds nothing, in the reference's order.
-template <int N, class T, class C, class A = float, bool Z = false>
-__device__ inline void finerow(const STopo& t, const int32_t* nb, const T* __restrict__ x, const T* __restrict__ xc,
-                               const FineCoefT<C>& cf, const C* __restrict__ dD, int s, int i, int j, int k, int4 w, A& diag,
-                               A& off) {
-    constexpr int sh = N == 16 ? 2 : 1, V = N * N * N;
+// neighbour and 0.4 to a LIQUID fine cell across a sub-face, else 0: the values that the FP32
+// arrays hold.
+// A level-0 fine cell of slot s: diag and the neighbours' sum, A x = diag x - off, in FP64
+// (iterative refinement's residual). Neighbours in the block index directly; across a face
+// they are the neighbour block's (slots in nb) or, without one, the coarse cell's. Every
+// index is computed and all thirteen loads are issued before any value is used (each index
+// is in bounds whatever the couplings); a coupling that is not positive adds nothing, in the
+// reference's order.
+__device__ inline void finerow64(const STopo& t, const int32_t* nb, const double* __restrict__ x, const double* __restrict__ xc,
+                                 const FineCoefT<float>& cf, const float* __restrict__ dD, int s, int i, int j, int k, int4 w,
+                                 double& diag, double& off) {
+    using A = double;
+    constexpr int N = 16, sh = 2, V = N * N * N;
     constexpr uint32_t per = (N + 1) * N * N;
     int I = w.x * N + i, J = w.y * N + j, K = w.z * N + k;
     int n0 = t.g.nc(0), n1 = t.g.nc(1), n2 = t.g.nc(2);
     uint32_t own = (uint32_t)(s - 1) * V + (uint32_t)(i + N * (j + N * k));
     auto nbr = [&](bool inside, int delta, int d, int li, int lj, int lk, int In, int Jn, int Kn) -> A {
-        if constexpr (Z) return (A)0;   // x = 0: nothing to read
         int32_t sn = nb[d];
         uint32_t in_block = own + (uint32_t)delta;
         uint32_t in_nb = (uint32_t)(sn - 1) * V + (uint32_t)(li + N * (lj + N * lk));
@@ -372,17 +368,16 @@ __device__ inline void finerow(const STopo& t, const int32_t* nb, const T* __res
         uint32_t in_coarse = (uint32_t)ci + (uint32_t)n0 * ((uint32_t)cj + (uint32_t)n1 * (uint32_t)ck);
         bool fine = inside || sn != 0;
         uint32_t idx = inside ? in_block : (sn != 0 ? in_nb : in_coarse);
-        const T* p = fine ? x : xc;
-        return (A)lf(p[idx]);
+        return (fine ? x : xc)[idx];
     };
     uint32_t base = (uint32_t)(s - 1) * per;
-    A c0 = (A)lf(cf.c[0][base + ffn(N, 0, i, j, k)]), c1 = (A)lf(cf.c[0][base + ffn(N, 0, i + 1, j, k)]);
-    A c2 = (A)lf(cf.c[1][base + ffn(N, 1, i, j, k)]), c3 = (A)lf(cf.c[1][base + ffn(N, 1, i, j + 1, k)]);
-    A c4 = (A)lf(cf.c[2][base + ffn(N, 2, i, j, k)]), c5 = (A)lf(cf.c[2][base + ffn(N, 2, i, j, k + 1)]);
+    A c0 = (A)cf.c[0][base + ffn(N, 0, i, j, k)], c1 = (A)cf.c[0][base + ffn(N, 0, i + 1, j, k)];
+    A c2 = (A)cf.c[1][base + ffn(N, 1, i, j, k)], c3 = (A)cf.c[1][base + ffn(N, 1, i, j + 1, k)];
+    A c4 = (A)cf.c[2][base + ffn(N, 2, i, j, k)], c5 = (A)cf.c[2][base + ffn(N, 2, i, j, k + 1)];
     A x0 = nbr(i > 0, -1, 0, N - 1, j, k, I - 1, J, K), x1 = nbr(i < N - 1, 1, 1, 0, j, k, I + 1, J, K);
     A x2 = nbr(j > 0, -N, 2, i, N - 1, k, I, J - 1, K), x3 = nbr(j < N - 1, N, 3, i, 0, k, I, J + 1, K);
     A x4 = nbr(k > 0, -N * N, 4, i, j, N - 1, I, J, K - 1), x5 = nbr(k < N - 1, N * N, 5, i, j, 0, I, J, K + 1);
-    diag = (A)lf(dD[own]);
+    diag = (A)dD[own];
     off = (A)0;
     if (c0 > (A)0) { diag += c0; off += c0 * x0; }
     if (c1 > (A)0) { diag += c1; off += c1 * x1; }
@@ -415,44 +410,26 @@ __global__ void k_covermask(uint8_t* __restrict__ m, uint16_t* __restrict__ crow
     crow[l] = (uint16_t)(v | r);
 }
 
-// An uncovered coarse cell (cover mask msk): coarse faces, or towards a covered
+// An uncovered coarse cell (its mask from k_covermask): coarse faces, or towards a covered
 // neighbour its (N/4)^2 sub-faces. The uncovered neighbours' couplings and values are
-// loaded first (an index off the grid reads the cell itself); a covered neighbour is
-// always at the edge of its block, so its sub-faces and cells index from one slot
-// lookup (the upper block's copy of a face, or the lower block's high plane). Sums in
-// the reference's order. coarserow_pre issues the loads of the uncovered part (the six
-// neighbours' couplings and values, the Dirichlet diagonal), coarserow_post sums them
-// with the covered sides', so a caller can issue the first batch before it knows whether
-// the row is needed.
+// loaded first (coarserow_pre; 0 and the cell's own where there is no coupling); a covered
+// neighbour is always at the edge of its block, so its sub-faces and cells index from one
+// slot lookup (the upper block's copy of a face, or the lower block's high plane). Sums in
+// the reference's order.
 template <class A> struct CoarsePre {
     A cc[6], xv[6], dg;
-    bool in[6];
 };
-template <class C, class A, class CX>
-__device__ inline CoarsePre<A> coarserow_pre(const STopo& t, CX cx, const CoarseCoefT<C>& ccf, const C* __restrict__ dDc, int I,
-                                             int J, int K, const LevelTypes* ty) {
-    int n0 = t.g.nc(0), n1 = t.g.nc(1), n2 = t.g.nc(2);
-    size_t own = cl(I, J, K, n0, n1);
+template <class A, class CX>
+__device__ inline CoarsePre<A> coarserow_pre(const STopo& t, unsigned mask, uint32_t l, CX cx, A dg) {
+    const uint32_t step[3] = {1u, (uint32_t)t.g.nc(0), (uint32_t)t.g.nc(0) * (uint32_t)t.g.nc(1)};
     CoarsePre<A> P;
-    A* cc = P.cc;
-    A* xv = P.xv;
-    bool* in = P.in;
 #pragma unroll
     for (int d = 0; d < 6; ++d) {
-        int a = d >> 1, sg = (d & 1) ? 1 : -1;
-        int In = I + sg * (a == 0), Jn = J + sg * (a == 1), Kn = K + sg * (a == 2);
-        in[d] = In >= 0 && Jn >= 0 && Kn >= 0 && In < n0 && Jn < n1 && Kn < n2;
-        size_t nidx = in[d] ? cl(In, Jn, Kn, n0, n1) : own;
-        if (ty) {
-            cc[d] = (A)(ty->tc[nidx] == LIQUID ? COARSE_COARSE : 0.0f);
-        } else {
-            int f0 = n0 + (a == 0), f1 = n1 + (a == 1);
-            size_t fi = sg < 0 ? cl(I, J, K, f0, f1) : cl(I + (a == 0), J + (a == 1), K + (a == 2), f0, f1);
-            cc[d] = (A)lf(ccf.c[a][fi]);
-        }
-        xv[d] = cx(nidx);
+        const bool on = (mask & (CCOUPLED << d)) != 0;
+        P.cc[d] = on ? (A)COARSE_COARSE : (A)0;
+        P.xv[d] = cx(on ? ((d & 1) ? l + step[d >> 1] : l - step[d >> 1]) : l);
     }
-    P.dg = (A)lf(dDc[own]);
+    P.dg = dg;
     return P;
 }
 // The row of a cell none of whose neighbours is covered, branch-free: a zero coupling
@@ -462,26 +439,25 @@ template <class A> __device__ inline void coarserow_flat(const CoarsePre<A>& P, 
     off = (A)0;
 #pragma unroll
     for (int d = 0; d < 6; ++d) {
-        const A c = (P.in[d] && P.cc[d] > (A)0) ? P.cc[d] : (A)0;
-        diag += c;
-        off += c * P.xv[d];
+        diag += P.cc[d];
+        off += P.cc[d] * P.xv[d];
     }
 }
+// With covered neighbours; level 0's couplings to their cells (N = 16) from the types tf,
+// level 1's from the arrays.
 template <int N, class C, class A, class FX>
-__device__ inline void coarserow_post(const STopo& t, unsigned msk, FX fx, const FineCoefT<C>& cf, const CoarsePre<A>& P, int I,
-                                      int J, int K, A& diag, A& off, const LevelTypes* ty) {
+__device__ inline void coarserow_post(const STopo& t, unsigned mask, FX fx, const FineCoefT<C>& cf,
+                                      const uint8_t* __restrict__ tf, const CoarsePre<A>& P, int I, int J, int K, A& diag, A& off) {
     constexpr int R = N / 4, V = N * N * N, m = N - 1;
     constexpr uint32_t per = (N + 1) * N * N;
     const A* cc = P.cc;
     const A* xv = P.xv;
-    const bool* in = P.in;
     diag = P.dg;
     off = (A)0;
 #pragma unroll
     for (int d = 0; d < 6; ++d) {
-        if (!in[d]) continue;
         int a = d >> 1, sg = (d & 1) ? 1 : -1;
-        if (msk & (2u << d)) {
+        if (mask & (2u << d)) {
             int In = I + sg * (a == 0), Jn = J + sg * (a == 1), Kn = K + sg * (a == 2);
             int32_t sn = t.slot[blockid(t.g, In >> 2, Jn >> 2, Kn >> 2)];
             uint32_t cbase = (uint32_t)(sn - 1) * V, fbase = (uint32_t)(sn - 1) * per;
@@ -504,7 +480,7 @@ __device__ inline void coarserow_post(const STopo& t, unsigned msk, FX fx, const
                 for (int p = 0; p < R; ++p) {
                     const uint32_t cidx = c0 + (uint32_t)p * sp + (uint32_t)q * sq;
                     A c;
-                    if (ty) c = (A)(ty->tf[cidx] == LIQUID ? FINE_COARSE : 0.0f);
+                    if constexpr (N == 16) c = (A)(tf[cidx] == LIQUID ? FINE_COARSE : 0.0f);
                     else c = (A)lf(cf.c[a][f0 + (uint32_t)p * fp + (uint32_t)q * fq]);
                     diag += c;
                     off += c * fx(cidx);
@@ -514,24 +490,6 @@ __device__ inline void coarserow_post(const STopo& t, unsigned msk, FX fx, const
             off += cc[d] * xv[d];
         }
     }
-}
-
-template <int N, class C, class A, class FX, class CX>
-__device__ inline void coarserow_acc(const STopo& t, unsigned msk, FX fx, const FineCoefT<C>& cf, CX cx,
-                                     const CoarseCoefT<C>& ccf, const C* __restrict__ dDc, int I, int J, int K, A& diag,
-                                     A& off, const LevelTypes* ty = nullptr) {
-    const CoarsePre<A> P = coarserow_pre<C, A>(t, cx, ccf, dDc, I, J, K, ty);
-    coarserow_post<N, C, A>(t, msk, fx, cf, P, I, J, K, diag, off, ty);
-}
-
-// The same reading x from arrays (Z: x = 0, nothing read).
-template <int N, class T, class C, class A = float, bool Z = false>
-__device__ inline void coarserow(const STopo& t, unsigned msk, const T* __restrict__ xf, const FineCoefT<C>& cf,
-                                 const T* __restrict__ xc, const CoarseCoefT<C>& ccf, const C* __restrict__ dDc, int I, int J,
-                                 int K, A& diag, A& off, const LevelTypes* ty = nullptr) {
-    auto fx = [&](uint32_t i) -> A { if constexpr (Z) return (A)0; else return (A)lf(xf[i]); };
-    auto cx = [&](size_t i) -> A { if constexpr (Z) return (A)0; else return (A)lf(xc[i]); };
-    coarserow_acc<N, C, A>(t, msk, fx, cf, cx, ccf, dDc, I, J, K, diag, off, ty);
 }
 
 // The device scalars of the Krylov loops (slots of SparseBasin::scal).
@@ -550,16 +508,14 @@ __device__ inline double block_sum_red(double v, double* lds) {
     return s;
 }
 
-// Level views: fine couplings and diagonal at N, the coarse grid's level-0 couplings.
+// Level views: the fine part's couplings, Dirichlet diagonal and types (level 0) or activity,
+// the coarse grid's diagonal and row masks.
 template <class C> struct CompT {
     FineCoefT<C> cf;
     const C* dDf;
     const uint8_t* actf;
-    CoarseCoefT<C> cc;
     const C* dDc;
-    const uint8_t* actc;
-    const uint8_t* cmask;   // k_covermask
-    const uint16_t* crow;
+    const uint16_t* crow;   // k_covermask
     const uint8_t* tc;      // the coarse cell types (level 0's matrix-free couplings)
     const C* rwf = nullptr; // reduced precision, level 0: omega / diag per fine cell
     const C* dgf = nullptr; // FP32, level 0: the full diagonal per fine cell (mode 6)
@@ -574,7 +530,7 @@ template <class T> struct RowArgs {
     const float* doc = nullptr;
     float* dnf = nullptr;         // d_new
     float* dnc = nullptr;
-    double* partials = nullptr;   // [4 nslots fine quarter tiles | coarse workgroups]
+    double* partials = nullptr;   // [the fine tiles, two a slot | coarse workgroups]
     int32_t coarse0 = 0;          // where the coarse workgroups' sums start
     const double* scal = nullptr;
     int zslot = -1;
@@ -588,7 +544,8 @@ template <class T> struct RowArgs {
     const float* rc = nullptr;
     T* bc = nullptr;
 };
-// k_convert's scale: scal[slot], or its inverse; 1 where that is no use
+// The scale between a Krylov vector and the reduced-precision hierarchy: scal[slot], or its
+// inverse; 1 where that is no use.
 __device__ inline float slot_scale(const double* __restrict__ scal, int slot, bool invert) {
     float c = 1.0f;
     if (slot >= 0) c = invert ? (float)(1.0 / scal[slot]) : (float)scal[slot];
@@ -605,23 +562,24 @@ __device__ inline float slot_scale(const double* __restrict__ scal, int slot, bo
 // type once per solve; the FP32 sweep keeps the reference's division). That sweep relaxes
 // the operator with diagonal w / r, and the reduced-precision residual uses the same.
 //
-// A level-0 pass is bound by HBM (9 B a cell for a reduced-precision sweep, 43 us for
+// A level-0 pass is bound by HBM (9 B a cell for a reduced-precision sweep, 39 us for
 // 4,200 slots), so two passes take in the one beside them: mode 7 is the residual
 // restricted to the next level in the workgroup (its 2 B are neither written nor read
 // back), mode 8 the first sweep after the prolongation, with x prolonged as it is loaded.
-// In FP16 there: 59 -> 46 and 74 -> 50 us. (The first two sweeps from zero in one
-// pass, the first made for the halo too, took 98 us, 13 more than the two: what a neighbour
-// slot's side costs is whole lines of every array it needs.)
-// Level 0, matrix-free and staged in LDS. A workgroup takes a quarter of a slot (4 z
-// planes of its 16^3 block), a thread 4 consecutive cells along x of one row. Level 0's
+// In FP16 there, when a sweep took 43 us: 59 -> 46 and 74 -> 50 us. (The first two sweeps from
+// zero in one pass, the first made for the halo too, took 119 us with the coarse rows, against
+// 87 for the two: what a neighbour slot's side costs is whole lines of every array it needs.)
+// Level 0, matrix-free and staged in LDS. A workgroup takes half of a slot (8 z planes of
+// its 16^3 block; a quarter in modes 5 and 6), a thread 4 consecutive cells along x of one
+// row, twice. Level 0's
 // coupling of a LIQUID fine cell to a neighbour is 1 when the neighbour is a LIQUID fine
 // cell, 0.4 when it is a LIQUID coarse cell, else 0 (k_finecoef, sflip.jl:1323-1342), so
 // it depends on the neighbour alone: the workgroup stages, for its cells and the layers
 // around them (the block's other planes, the face neighbours' slots, or else the coarse
 // cells: the value clamped to the grid, the type SOLID off it), each cell's coupling w and
 // the product w x (0 where w is 0), once per cell. A LIQUID cell's row then adds its six
-// neighbours' w into the diagonal and their w x into the off-diagonal sum in finerow's
-// order; a zero coupling adds exactly nothing, so the sums equal those over the coupling
+// neighbours' w into the diagonal and their w x into the off-diagonal sum in the reference's
+// order (-x, +x, -y, +y, -z, +z); a zero coupling adds exactly nothing, so the sums equal those over the coupling
 // arrays bit for bit. Loads and stores of a thread's own cells are 4-wide.
 template <class T> struct alignas(4 * sizeof(T)) Four { T v[4]; };
 template <class T> __device__ inline Four<T> load4(const T* __restrict__ p, uint32_t i) {
@@ -951,7 +909,7 @@ __global__ __launch_bounds__(256) void k_rowfine16(T* __restrict__ out, const T*
 }
 
 // The reduced-precision V-cycle's entry on level 0's fine part in one pass: b = r c in T
-// with k_convert's scale (c = 1 / scal[slot], 1 when slot < 0) and rounding, stored for
+// with slot_scale's c = 1 / scal[slot] (1 when slot < 0), rounded to T and stored for
 // the rest of the V-cycle, and the Jacobi sweep from x = 0 on it, out = b omega / diag
 // (mode 5 of k_rowfine16), on non-solid cells; four cells a thread.
 template <class T>
@@ -985,7 +943,7 @@ __device__ __forceinline__ void jacobi0w_cvt_wg(const uint32_t tile, T* __restri
 
 // Level 1 (8^3 a slot), staged in LDS: a workgroup per slot stages x of the block and its
 // face layers (face neighbours' slots, else the coarse cells, clamped), then each thread
-// computes 2 cells with finerow's couplings and order. Modes 7 and 8 as on level 0, to and
+// computes 2 cells, the neighbours in the order of level 0. Modes 7 and 8 as on level 0, to and
 // from the first dense level (the coarse grid's cells).
 template <int MODE, class T, class C>
 __device__ __forceinline__ void rowfine8_wg(const uint32_t tile, T* __restrict__ out, const T* __restrict__ x,
@@ -1086,7 +1044,8 @@ __device__ __forceinline__ void rowfine8_wg(const uint32_t tile, T* __restrict__
 // unknowns: 2.9 M cells at 5 cm took half of the pass's vector instructions), so a cell's
 // mask (k_covermask) comes first: a wavefront without unknowns stops there, and the mask
 // has the couplings, without the neighbours' types, places and bounds.
-// 4,200 slots and 1.5 M cells in FP16: level 0's sweep 44 -> 41 us, level 1's 32 -> 25.
+// 4,200 slots and 1.5 M cells in FP16: level 0's sweep 44 -> 41 us (39 with the LDS rows
+// above), level 1's 32 -> 25.
 template <int N, int MODE, class T, class C, class X = T>
 __device__ __forceinline__ void rowcoarse_wg(const uint32_t cb, const uint32_t ps, T* __restrict__ out,
                                              const X* __restrict__ x, const T* __restrict__ b, const X* __restrict__ xf,
@@ -1141,25 +1100,14 @@ __device__ __forceinline__ void rowcoarse_wg(const uint32_t cb, const uint32_t p
         bl = lf(bt);
     }
     if (m & CROW) {
-        // the couplings to uncovered neighbours, whose index is the cell's own where there is none
-        const uint32_t step[3] = {1u, (uint32_t)n0, (uint32_t)n0 * (uint32_t)n1};
-        CoarsePre<float> P;
-#pragma unroll
-        for (int d = 0; d < 6; ++d) {
-            const bool on = (m & (CCOUPLED << d)) != 0;
-            P.in[d] = true;
-            P.cc[d] = on ? COARSE_COARSE : 0.0f;
-            P.xv[d] = cx(on ? ((d & 1) ? l + step[d >> 1] : l - step[d >> 1]) : l);
-        }
-        P.dg = lf(L.dDc[l]);
+        const CoarsePre<float> P = coarserow_pre<float>(t, m, l, cx, lf(L.dDc[l]));
         if constexpr (!SEARCH) xl = cx(l);
         if constexpr ((JACOBI && MODE != 10) || RESID) bl = lf(b[l]);
         float diag, off;
         if (m & 0x7eu) {
-            const LevelTypes ty{L.actf, L.tc};   // level 0 (N = 16): the couplings from the types
             int I, J, K;
             unlin(l, n0, n1, I, J, K);
-            coarserow_post<N, C, float>(t, m, fx, L.cf, P, I, J, K, diag, off, N == 16 ? &ty : nullptr);
+            coarserow_post<N, C, float>(t, m, fx, L.cf, L.actf, P, I, J, K, diag, off);   // (level 0: actf the cell types)
         } else {
             coarserow_flat(P, diag, off);
         }
@@ -1201,8 +1149,10 @@ __device__ inline Place place_of(uint32_t share) {
     const uint32_t c0 = __umulhi(g, share), c1 = (uint32_t)(((uint64_t)g * share + share) >> 32);
     return c1 > c0 ? Place{c0, true} : Place{g - c0, false};
 }
+// (Seven wavefronts a SIMD for level 0's prolonging sweep, which the registers allow: 40 us for
+// 4,200 slots in FP16, 44 with six.)
 template <int N, int MODE, class T, class C, int NQ, class X>
-__global__ __launch_bounds__(256) void k_rowcomp(T* __restrict__ outf, T* __restrict__ outc, const X* __restrict__ xf,
+__global__ __launch_bounds__(256, N == 16 && MODE == 8 ? 7 : 1) void k_rowcomp(T* __restrict__ outf, T* __restrict__ outc, const X* __restrict__ xf,
                                                  const X* __restrict__ xc, const T* __restrict__ bf,
                                                  const T* __restrict__ bc, CompT<C> L, STopo t, RowArgs<T> S, uint32_t share) {
     const Place at = place_of(share);
@@ -1315,9 +1265,9 @@ __global__ __launch_bounds__(256) void k_residrestrict(T* __restrict__ bc, const
     }
 }
 
-// Conversions between the Krylov vectors (FP32) and the reduced-precision hierarchy:
-// y = x * mult * scal[slot] (or * mult when slot < 0), over the fine and the coarse range,
-// four values a thread (both parts are multiples of 4 long).
+// The reduced-precision hierarchy's result as a Krylov vector (FP32): y = x scal[slot] (x
+// itself when slot < 0), over the fine and the coarse range, four values a thread (both parts
+// are multiples of 4 long).
 template <class Y, class X>
 __global__ void k_convert(Y* __restrict__ yf, const X* __restrict__ xf, size_t nf, Y* __restrict__ yc, const X* __restrict__ xc,
                           size_t nc, const double* __restrict__ scal, int slot) {
@@ -1604,7 +1554,7 @@ __global__ __launch_bounds__(256) void k_resid64fine(float* __restrict__ r, cons
     double res = 0.0;
     if (L.actf[n] == LIQUID) {
         double diag, off;
-        finerow<16, double, float, double>(t, nb, x, xc, L.cf, L.dDf, s, c & 15, (c >> 4) & 15, c >> 8, w, diag, off);
+        finerow64(t, nb, x, xc, L.cf, L.dDf, s, c & 15, (c >> 4) & 15, c >> 8, w, diag, off);
         res = (double)b[n] - (diag * x[n] - off);
     }
     r[n] = (float)res;
@@ -1612,17 +1562,17 @@ __global__ __launch_bounds__(256) void k_resid64fine(float* __restrict__ r, cons
 __global__ __launch_bounds__(256) void k_resid64coarse(float* __restrict__ r, const double* __restrict__ x,
                                                        const double* __restrict__ xf, const float* __restrict__ b,
                                                        CompT<float> L, STopo t) {
-    int n0 = t.g.nc(0), n1 = t.g.nc(1), n2 = t.g.nc(2);
-    size_t l = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (l >= (size_t)n0 * n1 * n2) return;
-    int I, J, K;
-    unlin(l, n0, n1, I, J, K);
+    const int n0 = t.g.nc(0), n1 = t.g.nc(1), n2 = t.g.nc(2);
+    const uint32_t l = blockIdx.x * blockDim.x + threadIdx.x;
+    if (l >= (uint32_t)n0 * (uint32_t)n1 * (uint32_t)n2) return;
     double res = 0.0;
-    unsigned msk = L.cmask[l];
-    if (L.actc[l] != 0 && !(msk & 1u)) {
+    const unsigned m = L.crow[l];
+    if (m & CROW) {
         double diag, off;
-        const LevelTypes ty{L.actf, L.tc};
-        coarserow<16, double, float, double>(t, msk, xf, L.cf, x, L.cc, L.dDc, I, J, K, diag, off, &ty);
+        int I, J, K;
+        unlin(l, n0, n1, I, J, K);
+        const CoarsePre<double> P = coarserow_pre<double>(t, m, l, [&](uint32_t i) { return x[i]; }, (double)L.dDc[l]);
+        coarserow_post<16, float, double>(t, m, [&](uint32_t i) { return xf[i]; }, L.cf, L.actf, P, I, J, K, diag, off);
         res = (double)b[l] - (diag * x[l] - off);
     }
     r[l] = (float)res;
@@ -1994,11 +1944,9 @@ struct SparseSolver {
             H.Dx.push_back(L.x.p); H.Db.push_back(L.b.p); H.Dt.push_back(L.t.p);
             H.D.push_back(DViewT<float>{i3(L.n), {L.c[0].p, L.c[1].p, L.c[2].p}, L.dD.p, L.act.p});
         }
-        H.L0 = CompT<float>{{{s.cf[0].p, s.cf[1].p, s.cf[2].p}}, s.dD.fine.p, s.types.fine.p,
-                            {{s.cc[0].p, s.cc[1].p, s.cc[2].p}}, s.dD.coarse.p, s.D[0].act.p, s.cmask.p, s.crow.p, s.types.coarse.p,
-                            nullptr, s.dgf.p};
-        H.L1 = CompT<float>{{{s.c1[0].p, s.c1[1].p, s.c1[2].p}}, s.dD1.p, s.act1.p,
-                            {{s.cc[0].p, s.cc[1].p, s.cc[2].p}}, s.dD.coarse.p, s.D[0].act.p, s.cmask.p, s.crow.p, s.types.coarse.p};
+        H.L0 = CompT<float>{{{s.cf[0].p, s.cf[1].p, s.cf[2].p}}, s.dD.fine.p, s.types.fine.p, s.dD.coarse.p, s.crow.p,
+                            s.types.coarse.p, nullptr, s.dgf.p};
+        H.L1 = CompT<float>{{{s.c1[0].p, s.c1[1].p, s.c1[2].p}}, s.dD1.p, s.act1.p, s.dD.coarse.p, s.crow.p, s.types.coarse.p};
         return H;
     }
     // The reduced-precision hierarchy (storage in s.mp): vectors and couplings, the dense
@@ -2018,11 +1966,10 @@ struct SparseSolver {
         }
         // level 0's rows take their couplings from the cell types, the coarse rows from their
         // masks: no copies of these couplings
-        H.L0 = CompT<T>{{{nullptr, nullptr, nullptr}}, (T*)m.dDf.p, s.types.fine.p,
-                        {{nullptr, nullptr, nullptr}}, (T*)m.dDc.p, s.D[0].act.p, s.cmask.p, s.crow.p, s.types.coarse.p,
+        H.L0 = CompT<T>{{{nullptr, nullptr, nullptr}}, (T*)m.dDf.p, s.types.fine.p, (T*)m.dDc.p, s.crow.p, s.types.coarse.p,
                         (T*)m.rwf.p};
-        H.L1 = CompT<T>{{{(T*)m.c1[0].p, (T*)m.c1[1].p, (T*)m.c1[2].p}}, (T*)m.dD1.p, s.act1.p,
-                        {{nullptr, nullptr, nullptr}}, (T*)m.dDc.p, s.D[0].act.p, s.cmask.p, s.crow.p, s.types.coarse.p};
+        H.L1 = CompT<T>{{{(T*)m.c1[0].p, (T*)m.c1[1].p, (T*)m.c1[2].p}}, (T*)m.dD1.p, s.act1.p, (T*)m.dDc.p, s.crow.p,
+                        s.types.coarse.p};
         H.rscale = 0.25f;
         return H;
     }

@@ -29,7 +29,7 @@ struct DenseNodes {
     }
     static constexpr int TAB = 1;   // no table
     struct Near {};
-    __device__ Near near(bool, const int*, const int*) const { return {}; }
+    __device__ Near near(const int*, const int*) const { return {}; }
     __device__ void stage(const Near&, int32_t*) const {}
     __device__ int64_t at(const Near&, const int32_t*, int a, int I, int J, int K) const { return index(a, I, J, K); }
 };
@@ -42,7 +42,7 @@ struct DenseCells {
     }
     static constexpr int TAB = 1;   // no table
     struct Near {};
-    __device__ Near near(bool, const int*, const int*) const { return {}; }
+    __device__ Near near(const int*, const int*) const { return {}; }
     __device__ void stage(const Near&, int32_t*) const {}
     __device__ int64_t at(const Near&, const int32_t*, int I, int J, int K) const { return index(I, J, K); }
 };
@@ -138,7 +138,7 @@ struct DenseClampNodes {
     }
     static constexpr int TAB = 1;   // no table
     struct Near {};
-    __device__ Near near(bool, const int*, const int*) const { return {}; }
+    __device__ Near near(const int*, const int*) const { return {}; }
     __device__ void stage(const Near&, int32_t*) const {}
     __device__ int64_t at(const Near&, const int32_t*, int a, int I, int J, int K) const { return index(a, I, J, K); }
 };

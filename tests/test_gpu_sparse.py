@@ -195,8 +195,8 @@ def test_p2g_parity(M):
 
 def _orders(n, seed=5):
     """Particle orders that drive the tiled transfers down each of their paths: cell order
-    (a box per workgroup), 128-particle runs from the two halves interleaved (every
-    workgroup straddles two regions, so a box per wavefront), and a random order (mostly
+    (mostly one box per workgroup), 128-particle runs from the two halves interleaved (every
+    workgroup straddles two regions, so several boxes in turn), and a random order (mostly
     the direct path)."""
     half = n // 2 // 128 * 128
     runs = []
@@ -248,7 +248,7 @@ def test_g2p_bitexact(M):
     o.g2p(dt, 9.81)
     for nm in PNAMES:
         np.testing.assert_array_equal(s.get(nm.upper()), o.array(nm)[:o.n], err_msg=nm)
-    for name in ("interleaved", "random"):   # the wavefront and direct paths of the tiled gather
+    for name in ("interleaved", "random"):   # several boxes in turn, and the direct path
         order = orders[name]
         s = _upload(M, o)
         for nm in PNAMES:
