@@ -344,7 +344,8 @@ __device__ inline int32_t nbslot(const STopo& t, int4 w, int d) {
 // Level 0's couplings follow from the cell types (k_finecoef, k_coarsecoef,
 // sflip.jl:1323-1353): for a LIQUID uncovered cell, 4 to an uncovered LIQUID coarse
 // neighbour and 0.4 to a LIQUID fine cell across a sub-face, else 0: the values that the FP32
-// arrays hold.
+// arrays hold, which a level-0 row need not read.
+struct LevelTypes { const uint8_t* tf; const uint8_t* tc; };   // fine, coarse
 // A level-0 fine cell of slot s: diag and the neighbours' sum, A x = diag x - off, in FP64
 // (iterative refinement's residual). Neighbours in the block index directly; across a face
 // they are the neighbour block's (slots in nb) or, without one, the coarse cell's. Every
@@ -443,11 +444,11 @@ template <class A> __device__ inline void coarserow_flat(const CoarsePre<A>& P, 
         off += P.cc[d] * P.xv[d];
     }
 }
-// With covered neighbours; level 0's couplings to their cells (N = 16) from the types tf,
-// level 1's from the arrays.
+// With covered neighbours; level 0's couplings to their cells from the types, level 1's (`ty`
+// null) from the arrays.
 template <int N, class C, class A, class FX>
-__device__ inline void coarserow_post(const STopo& t, unsigned mask, FX fx, const FineCoefT<C>& cf,
-                                      const uint8_t* __restrict__ tf, const CoarsePre<A>& P, int I, int J, int K, A& diag, A& off) {
+__device__ inline void coarserow_post(const STopo& t, unsigned mask, FX fx, const FineCoefT<C>& cf, const CoarsePre<A>& P,
+                                      int I, int J, int K, A& diag, A& off, const LevelTypes* ty) {
     constexpr int R = N / 4, V = N * N * N, m = N - 1;
     constexpr uint32_t per = (N + 1) * N * N;
     const A* cc = P.cc;
@@ -480,7 +481,7 @@ __device__ inline void coarserow_post(const STopo& t, unsigned mask, FX fx, cons
                 for (int p = 0; p < R; ++p) {
                     const uint32_t cidx = c0 + (uint32_t)p * sp + (uint32_t)q * sq;
                     A c;
-                    if constexpr (N == 16) c = (A)(tf[cidx] == LIQUID ? FINE_COARSE : 0.0f);
+                    if (ty) c = (A)(ty->tf[cidx] == LIQUID ? FINE_COARSE : 0.0f);
                     else c = (A)lf(cf.c[a][f0 + (uint32_t)p * fp + (uint32_t)q * fq]);
                     diag += c;
                     off += c * fx(cidx);
@@ -1105,9 +1106,10 @@ __device__ __forceinline__ void rowcoarse_wg(const uint32_t cb, const uint32_t p
         if constexpr ((JACOBI && MODE != 10) || RESID) bl = lf(b[l]);
         float diag, off;
         if (m & 0x7eu) {
+            const LevelTypes ty{L.actf, L.tc};   // (N = 16: actf holds the cell types)
             int I, J, K;
             unlin(l, n0, n1, I, J, K);
-            coarserow_post<N, C, float>(t, m, fx, L.cf, L.actf, P, I, J, K, diag, off);   // (level 0: actf the cell types)
+            coarserow_post<N, C, float>(t, m, fx, L.cf, P, I, J, K, diag, off, N == 16 ? &ty : nullptr);
         } else {
             coarserow_flat(P, diag, off);
         }
@@ -1149,10 +1151,8 @@ __device__ inline Place place_of(uint32_t share) {
     const uint32_t c0 = __umulhi(g, share), c1 = (uint32_t)(((uint64_t)g * share + share) >> 32);
     return c1 > c0 ? Place{c0, true} : Place{g - c0, false};
 }
-// (Seven wavefronts a SIMD for level 0's prolonging sweep, which the registers allow: 40 us for
-// 4,200 slots in FP16, 44 with six.)
 template <int N, int MODE, class T, class C, int NQ, class X>
-__global__ __launch_bounds__(256, N == 16 && MODE == 8 ? 7 : 1) void k_rowcomp(T* __restrict__ outf, T* __restrict__ outc, const X* __restrict__ xf,
+__global__ __launch_bounds__(256) void k_rowcomp(T* __restrict__ outf, T* __restrict__ outc, const X* __restrict__ xf,
                                                  const X* __restrict__ xc, const T* __restrict__ bf,
                                                  const T* __restrict__ bc, CompT<C> L, STopo t, RowArgs<T> S, uint32_t share) {
     const Place at = place_of(share);
@@ -1572,7 +1572,8 @@ __global__ __launch_bounds__(256) void k_resid64coarse(float* __restrict__ r, co
         int I, J, K;
         unlin(l, n0, n1, I, J, K);
         const CoarsePre<double> P = coarserow_pre<double>(t, m, l, [&](uint32_t i) { return x[i]; }, (double)L.dDc[l]);
-        coarserow_post<16, float, double>(t, m, [&](uint32_t i) { return xf[i]; }, L.cf, L.actf, P, I, J, K, diag, off);
+        const LevelTypes ty{L.actf, L.tc};
+        coarserow_post<16, float, double>(t, m, [&](uint32_t i) { return xf[i]; }, L.cf, P, I, J, K, diag, off, &ty);
         res = (double)b[l] - (diag * x[l] - off);
     }
     r[l] = (float)res;
