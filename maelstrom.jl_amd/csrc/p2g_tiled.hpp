@@ -237,7 +237,7 @@ constexpr int BOX_ROUNDS = 4;
 // straddles blocks, or a row that crosses the funnel's ring: 8 % of the workgroups at 5 cm,
 // 44 % on the dense grid) take up to BOX_ROUNDS boxes in turn; the global adds of those that
 // fitted neither the workgroup's box nor one per wavefront were half the kernel's time. 14.2 M
-// particles at 5 cm 3,200 -> 1,750 us (of which the arithmetic issues for 0.8 ms and the LDS
+// particles at 5 cm 3,200 -> 1,850 us (of which the arithmetic issues for 0.8 ms and the LDS
 // is busy for 0.7 ms), 1.6 M on 256 x 256 x 128 626 -> 199 us. Boxes of 1,024 and 1,536
 // nodes were 3-8 % slower at 5 cm (more rounds), 3,072 and 4,096 2-4 % slower on the dense grid
 // (fewer workgroups a CU), as were five workgroups a CU with 1,984.
